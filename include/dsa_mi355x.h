@@ -238,6 +238,19 @@ int dsa_sparse_mla_bwd(const void* q, const void* kv, const int32_t* indices, co
                        int64_t q_offset, void* stream);
 
 /*
+ * dsa_sparse_mla_fwd (sinks NULL) or dsa_sparse_mla_fwd_sink with a caller workspace of
+ * dsa_sparse_mla_fwd_workspace_size() bytes (16-byte aligned).  The size is 0 where the
+ * workspace has no use; with fewer bytes, or none, the call runs as the entry points without
+ * one do.  bf16 calls of at most 64 heads use it to let several consecutive tokens share a
+ * workgroup, which gathers the union of their keys once.
+ */
+int64_t dsa_sparse_mla_fwd_workspace_size(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
+                                          int64_t topk, int64_t q_offset);
+int dsa_sparse_mla_fwd_ws(const void* q, const void* kv, const int32_t* indices, const float* sinks, void* out,
+                          float* softmax_max, float* softmax_sum, int dtype, int64_t batch, int64_t s_q, int64_t s_kv,
+                          int64_t n_heads, int64_t d_qk, int64_t d_v, int64_t topk, float scale, int64_t q_offset,
+                          void* workspace, int64_t workspace_bytes, void* stream);
+/*
  * dsa_sparse_mla_fwd / dsa_sparse_mla_bwd with the DeepSeek-V4 per-head attention sink folded
  * in (reference: SparseAttention.forward's attn_sink, models/deepseek_v4/model.py:573-623,
  * passed as `sinks` to npu_sparse_attn_shared_kv{,_grad}, converters/kernels/npu_smla.py:351-400).
@@ -337,6 +350,10 @@ int dsa_indexer_kl_grad_ex(const void* q_idx, const void* k_idx, const float* w,
  * backward's dKV and the indexer loss's dK_index, which use the same indices, build it once.
  */
 int64_t dsa_pair_csr_size(int64_t batch, int64_t s_q, int64_t s_k, int64_t topk);
+/* 1 where dsa_sparse_mla_bwd{,_ex,_sink} with this workspace runs over packed tokens (bf16, at
+ * most 64 heads): it then reduces dKV by its own plan and takes no pair CSR */
+int dsa_sparse_mla_bwd_packed(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t d_qk, int64_t topk,
+                              int64_t q_offset, int64_t workspace_bytes);
 /* query rows per chunk that a workspace of workspace_bytes gives dsa_sparse_mla_bwd{,_ex}
  * (bf16 path) / dsa_indexer_kl_grad{,_ex} (H_I = 64, D_I = 128); s_q means one chunk, where a
  * prebuilt pair CSR is used; 0 = the workspace is too small */
@@ -545,8 +562,11 @@ int dsa_lightning_indexer_tnd(const void* q, const float* q_scale, const void* k
  * (0 <= v < len_k_i, v <= s - cu_seqlens_q[i] + max(0, len_k_i - len_q_i)), else -1.  The
  * fixed-length attention, mass and indexer KL entry points then take the whole batch as one
  * [1, t_q] problem with q_offset >= t_k (no causal test): dsa_sparse_mla_fwd(_varlen)
- * results are bit-identical per row; dKV and dk_I sum the same contributions in another
- * fp32 grouping. */
+ * results are bit-identical per row (without a forward workspace); dKV and dk_I sum the same
+ * contributions in another fp32 grouping.  dsa_tnd_global_indices_varlen: the same from host
+ * bounds (host int32 arrays), passed as kernel arguments. */
+int dsa_tnd_global_indices_varlen(const int32_t* indices, int32_t* out, const int32_t* cu_seqlens_q,
+                                  const int32_t* cu_seqlens_k, int64_t n_seq, int64_t topk, void* stream);
 int dsa_tnd_global_indices(const int32_t* indices, int32_t* out, const int32_t* cu_seqlens_q,
                            const int32_t* cu_seqlens_k, int64_t n_seq, int64_t t_q, int64_t t_k, int64_t topk,
                            void* stream);

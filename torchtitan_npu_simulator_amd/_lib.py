@@ -14,7 +14,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "libdsa_mi355x.so"
-ABI_VERSION = 17
+ABI_VERSION = 18
 
 DSA_F32, DSA_BF16, DSA_FP8_E4M3 = 0, 1, 2
 
@@ -49,6 +49,11 @@ _SIGNATURES = {
                                _i64, _vp, _i64, _vp], _i32),
     "dsa_sparse_mla_fwd": (
         [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _i64, _vp],
+        _i32,
+    ),
+    "dsa_sparse_mla_fwd_workspace_size": ([_i32, _i64, _i64, _i64, _i64, _i64, _i64], _i64),
+    "dsa_sparse_mla_fwd_ws": (
+        [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _i64, _vp, _i64, _vp],
         _i32,
     ),
     "dsa_sparse_mla_bwd_workspace_size": ([_i64, _i64, _i64, _i64, _i64, _i64], _i64),
@@ -87,6 +92,7 @@ _SIGNATURES = {
         _i32,
     ),
     "dsa_pair_csr_size": ([_i64, _i64, _i64, _i64], _i64),
+    "dsa_sparse_mla_bwd_packed": ([_i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64], _i32),
     "dsa_sparse_mla_bwd_chunk_rows": ([_i64, _i64, _i64, _i64, _i64, _i64], _i64),
     "dsa_indexer_kl_grad_chunk_rows": ([_i64, _i64, _i64, _i64, _i64], _i64),
     "dsa_pair_csr_build": ([_vp, _i64, _i64, _i64, _i64, _i64, _vp, _i64, _vp], _i32),
@@ -127,6 +133,7 @@ _SIGNATURES = {
          _vp, _i64, _vp],
         _i32,
     ),
+    "dsa_tnd_global_indices_varlen": ([_vp, _vp, _vp, _vp, _i64, _i64, _vp], _i32),
     "dsa_tnd_global_indices": ([_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp], _i32),
     "dsa_indexer_kl_grad_varlen_workspace_size": ([_vp, _vp, _i64, _i64, _i64, _i64], _i64),
     "dsa_indexer_kl_grad_varlen": (

@@ -24,6 +24,7 @@
 // workspace.
 #include <algorithm>
 
+#include "attn_pack.h"
 #include "dsa_common.h"
 #include "dsa_csr.h"
 #include "dsa_gather.h"
@@ -74,13 +75,17 @@ constexpr int kSdpWaves = 8;
 
 // kD: row width of Q and KV, 576 (latent + rope) or 512 (no rope).  kOwnDelta: delta =
 // rowsum(dO o O) of each head is formed here from O (read beside dO, in dO's lane layout,
-// then summed over the head's four lane groups) instead of read from dbuf
-template <int kD, bool kOwnDelta>
+// then summed over the head's four lane groups) instead of read from dbuf.  kPack: the
+// workgroup is a group of packed tokens (attn_pack.h): "heads" are its (token, head) rows,
+// 16 per wave and so of one token, whose mask words give the wave's validity bits (scalar
+// loads, one block ahead), and the mass is summed per token into pk.mass by slot.
+template <int kD, bool kOwnDelta, bool kPack>
 __global__ void __launch_bounds__(64 * kSdpWaves, 1)
 bwd_sdp_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, const int32_t* __restrict__ idx,
                 const uint16_t* __restrict__ dout, const uint16_t* __restrict__ out, const float* __restrict__ smax,
                 const float* __restrict__ ssum, const float* __restrict__ dbuf, uint16_t* __restrict__ gbuf,
-                float* __restrict__ mass, int S, int s_kv, int H, int K, float scale, int64_t q_offset, int row0) {
+                float* __restrict__ mass, int S, int s_kv, int H, int K, float scale, int64_t q_offset, int row0,
+                PackView pk) {
   constexpr int kW = kSdpWaves;
   using Gather = RowGather<kW, kD, true>;
   using Geo = GatherGeomT<kD>;
@@ -96,21 +101,35 @@ bwd_sdp_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, 
   __shared__ int sidx[GatherGeom::kRing][Gather::kRingInts];
   __shared__ int sh_last;
 
-  const int lr = blockIdx.x, tok = row0 + lr, b = blockIdx.z, tid = threadIdx.x;
+  // local row of the chunk: a token, or (packed, the longest unions first) a group of tokens
+  const int lr = kPack ? launch_row() : (int)blockIdx.x, b = blockIdx.z, tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int c = lane & 15, g = lane >> 4;  // MFMA column (head) and k group; A row c
-  const int hl = wave * 16 + c;            // head (the workgroup holds all heads)
-  const bool hok = hl < H;
+  const int hl = wave * 16 + c;            // row (the workgroup holds all heads)
+  int tok = row0 + lr, head = hl;
+  bool hok = hl < H;
+  if constexpr (kPack) {
+    int t;
+    pack_row(pk, hl, t, head);
+    tok = (row0 + lr) * pk.tt + t;
+    hok = t < pk.tt && tok < S && head < H;
+    if (!hok) tok = (row0 + lr) * pk.tt;  // (a token that exists)
+  }
   const int64_t row_id = (int64_t)b * S + tok;
-  const int64_t hrow = row_id * H + (hok ? hl : 0);
-  const int32_t* ridx = idx + row_id * K;
-  const int64_t limit = tok + q_offset;
+  const int64_t hrow = row_id * H + (hok ? head : 0);
+  const int64_t pgrp = (int64_t)b * pk.groups + row0 + lr;
+  const int32_t* ridx = kPack ? pk.idx + pgrp * pk.cap : idx + row_id * K;
+  if constexpr (kPack) K = pk.cap;
+  const int64_t limit = kPack ? (int64_t)s_kv : tok + q_offset;  // (packed: the plan applied the causal rule)
   const uint16_t* kvb = kv + (int64_t)b * s_kv * kD;
   uint16_t* grow = gbuf + ((int64_t)b * gridDim.x + lr) * (int64_t)g_slots(K) * kGW;
-  float* mrow = mass ? mass + row_id * K : nullptr;
+  // mass row of the token; packed: of the group's first token, by union slot
+  float* mrow = kPack ? (pk.mass ? pk.mass + ((int64_t)b * gridDim.x + lr) * pk.tt * pk.cap : nullptr)
+                      : (mass ? mass + row_id * K : nullptr);
+  const pack_word* mwords = kPack ? pack_mask_row(pk, pgrp, 16 * wave) : nullptr;
 
   int vidx[kIdxU];
-  load_row_indices(ridx, K, vidx);
+  if constexpr (!kPack) load_row_indices(ridx, K, vidx);
   if (wave == 0) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) Gather::issue_idx(ridx, K, i, sidx[i], lane);
@@ -136,9 +155,16 @@ bwd_sdp_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, 
   }
   const float mx = smax[hrow], sm = ssum[hrow];
   float dlt;
-  if constexpr (!kOwnDelta) dlt = dbuf[((int64_t)b * gridDim.x + lr) * H + (hok ? hl : 0)];
-  const int nblk = count_row_blocks(ridx, K, s_kv, limit, vidx, &sh_last);
-  if (mrow)  // slots past the last usable block carry no mass
+  if constexpr (!kOwnDelta) {
+    if constexpr (kPack) {  // (delta rows of the chunk's tokens, from the chunk's first)
+      const int t0 = row0 * pk.tt, nt = min((int)gridDim.x * pk.tt, S - t0);
+      dlt = dbuf[((int64_t)b * nt + (tok - t0)) * H + (hok ? head : 0)];
+    } else {
+      dlt = dbuf[((int64_t)b * gridDim.x + lr) * H + (hok ? hl : 0)];
+    }
+  }
+  const int nblk = kPack ? (pk.count[pgrp] + kBN - 1) / kBN : count_row_blocks(ridx, K, s_kv, limit, vidx, &sh_last);
+  if (!kPack && mrow)  // slots past the last usable block carry no mass
     for (int j = nblk * kBN + tid; j < K; j += 64 * kW) mrow[j] = 0.f;
   if (nblk == 0) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the ring DMA has landed before the LDS is released
@@ -202,6 +228,20 @@ bwd_sdp_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, 
   auto flush_part = [&](int fb, int part) {
     const int sb = fb & 1;
     if (part == 2) {
+      if constexpr (kPack) {  // per token: the waves of its rows, paired as below
+        const int t = tid / kBN, key = tid % kBN;
+        if (mrow && t < pk.tt) {
+          const int nw = pk.hp >> 4, w0 = t * nw;
+          float sum = 0.f;
+          for (int w = w0; w < w0 + nw; w += 4) {
+            const float a = pst[sb][w][key] + (w + 1 < w0 + nw ? pst[sb][w + 1][key] : 0.f);
+            const float e = (w + 2 < w0 + nw ? pst[sb][w + 2][key] : 0.f) + (w + 3 < w0 + nw ? pst[sb][w + 3][key] : 0.f);
+            sum = w == w0 ? a + e : sum + (a + e);
+          }
+          mrow[(int64_t)t * pk.cap + fb * kBN + key] = sum;
+        }
+        return;
+      }
       if (mrow && tid < kBN && fb * kBN + tid < K)
         mrow[fb * kBN + tid] = ((pst[sb][0][tid] + pst[sb][1][tid]) + (pst[sb][2][tid] + pst[sb][3][tid])) +
                                ((pst[sb][4][tid] + pst[sb][5][tid]) + (pst[sb][6][tid] + pst[sb][7][tid]));
@@ -226,7 +266,9 @@ bwd_sdp_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, 
   const lds_char* qpe_b = lds_bytes(&qpe[0][0]);
   if (wave == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // ring entries 0..2 landed
   __syncthreads();                                                  // publishes them and qpe
-  uint32_t vm_cur = Gather::ring_valid(sidx[0], lane, lim, K);
+  uint32_t vm_cur;
+  if constexpr (kPack) vm_cur = mwords[0];
+  else vm_cur = Gather::ring_valid(sidx[0], lane, lim, K);
 #pragma unroll
   for (int i = 0; i < kPer; ++i)
     Gather::issue_slot(kvb, &tile[0][0], i, wave, Gather::ring_slot(sidx[0], i, gl), gl, lim, K);
@@ -321,7 +363,9 @@ bwd_sdp_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, 
     u32x4* dst_tile = &tile[(blk + 1) & 1][0];
     const int* ring = sidx[(blk + 1) & (GatherGeom::kRing - 1)];
     const int rows_left = K - (blk + 1) * kBN;
-    const uint32_t vm_next = Gather::ring_valid(ring, lane, lim, rows_left);
+    uint32_t vm_next;
+    if constexpr (kPack) vm_next = mwords[min(blk + 1, nblk - 1)];
+    else vm_next = Gather::ring_valid(ring, lane, lim, rows_left);
     uint32_t raw_next = Gather::ring_slot(ring, 0, gl);
 #pragma unroll
     for (int x = 0; x < 2; ++x) sacc[x] = pacc[x] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -438,10 +482,10 @@ struct DqkShape {
   static constexpr int kOwn = (kDT + kPh - 1) / kPh;  // d tiles per wave: 3 | 4
 };
 
-template <int kD>  // row width of KV and dQ: 576 or 512
+template <int kD, bool kPack>  // row width of KV and dQ: 576 or 512; packed tokens (attn_pack.h)
 __global__ void __launch_bounds__(DqkShape<kD>::kWaves * 64, 1)
 bwd_dqk_kernel(const uint16_t* __restrict__ kv, const int32_t* __restrict__ idx, const uint16_t* __restrict__ gbuf,
-               uint16_t* __restrict__ dq, int S, int s_kv, int H, int K, int64_t q_offset, int row0) {
+               uint16_t* __restrict__ dq, int S, int s_kv, int H, int K, int64_t q_offset, int row0, PackView pk) {
   using Shape = DqkShape<kD>;
   constexpr int kWaves = Shape::kWaves, kPh = Shape::kPh;
   using Gather = RowGather<kWaves, kD>;
@@ -457,26 +501,29 @@ bwd_dqk_kernel(const uint16_t* __restrict__ kv, const int32_t* __restrict__ idx,
   __shared__ int sidx[GatherGeom::kRing][Gather::kRingInts];
   __shared__ int sh_last;
 
-  const int lr = blockIdx.x, tok = row0 + lr, b = blockIdx.z, tid = threadIdx.x;
+  const int lr = kPack ? launch_row() : (int)blockIdx.x, tok = row0 + lr, b = blockIdx.z, tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int wt = wave % kPh, hh2 = wave / kPh;  // d-tile owner, head half (groups 2 hh2, 2 hh2 + 1)
   const int n = lane & 31, h = lane >> 5;
-  const int64_t row_id = (int64_t)b * S + tok;
-  const int32_t* ridx = idx + row_id * K;
-  const int64_t limit = tok + q_offset;
+  const int64_t row_id = kPack ? (int64_t)b * S + (int64_t)tok * pk.tt : (int64_t)b * S + tok;  // (first) token's row
+  const int64_t pgrp = (int64_t)b * pk.groups + tok;
+  const int32_t* ridx = kPack ? pk.idx + pgrp * pk.cap : idx + row_id * K;
+  if constexpr (kPack) K = pk.cap;
+  const int64_t limit = kPack ? (int64_t)s_kv : tok + q_offset;
   const uint16_t* kvb = kv + (int64_t)b * s_kv * kD;
   const uint16_t* grow = gbuf + ((int64_t)b * gridDim.x + lr) * (int64_t)g_slots(K) * kGW;
 
   int vidx[kIdxU];
-  load_row_indices(ridx, K, vidx);
+  if constexpr (!kPack) load_row_indices(ridx, K, vidx);
   if (wave == 0) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) Gather::issue_idx(ridx, K, i, sidx[i], lane);
   }
-  const int nblk = count_row_blocks(ridx, K, s_kv, limit, vidx, &sh_last);
+  const int nblk = kPack ? (pk.count[pgrp] + kBN - 1) / kBN : count_row_blocks(ridx, K, s_kv, limit, vidx, &sh_last);
   if (nblk == 0) {  // no usable key: dQ = 0
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    for (int i = tid; i < H * (kD / 2); i += kWaves * 64)
+    const int nt = kPack ? min(pk.tt, S - tok * pk.tt) : 1;  // (the tokens' rows are consecutive)
+    for (int i = tid; i < nt * H * (kD / 2); i += kWaves * 64)
       reinterpret_cast<uint32_t*>(dq + row_id * H * kD)[i] = 0u;
     return;
   }
@@ -603,8 +650,15 @@ bwd_dqk_kernel(const uint16_t* __restrict__ kv, const int32_t* __restrict__ idx,
     if (dt >= kDT) break;
 #pragma unroll
     for (int gg = 0; gg < 2; ++gg) {
-      const int hd = 32 * (2 * hh2 + gg) + n;
-      if (hd >= H) continue;
+      int hd = 32 * (2 * hh2 + gg) + n;
+      if constexpr (kPack) {  // (token, head) of the row, as an offset of whole heads from the group's first
+        int t;
+        pack_row(pk, hd, t, hd);
+        if (t >= pk.tt || tok * pk.tt + t >= S || hd >= H) continue;
+        hd += t * H;
+      } else {
+        if (hd >= H) continue;
+      }
       uint2* drow = reinterpret_cast<uint2*>(dq + (row_id * H + hd) * kD);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -653,11 +707,11 @@ struct ContribGeom {
 // C stage layout: row r (slot), 16-byte chunk c stored at c ^ ((r >> 1) & 7)
 __device__ __forceinline__ int stage_swz(int r) { return (r >> 1) & 7; }
 
-template <int kHGroups, int kD>
+template <int kHGroups, int kD, bool kPack>
 __global__ void __launch_bounds__(kCThreads, 1)
 bwd_contrib_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ dout,
                    const int32_t* __restrict__ idx, const uint16_t* __restrict__ gbuf, uint16_t* __restrict__ cbuf,
-                   int S, int s_kv, int H, int K, int64_t q_offset, int row0, int rows) {
+                   int S, int s_kv, int H, int K, int64_t q_offset, int row0, int rows, PackView pk) {
   using CG = ContribGeom<kD>;
   constexpr int kRC = CG::kRC, kStChunks = CG::kStChunks, kXChunks = CG::kXChunks;
   constexpr int kKSteps = 4 * kHGroups;                // 32-row k steps of X (128 rows per head group)
@@ -668,11 +722,18 @@ bwd_contrib_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ 
   const int tok = row0 + lr, b = blockIdx.y;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int col = lane & 15, g = lane >> 4;
-  const int64_t row_id = (int64_t)b * S + tok;
-  const int32_t* ridx = idx + row_id * K;
-  int vidx[kIdxU];
-  load_row_indices(ridx, K, vidx);
-  const int nblk = count_row_blocks(ridx, K, s_kv, tok + q_offset, vidx, &sh_last);
+  const int64_t row_id = kPack ? (int64_t)b * S + (int64_t)tok * pk.tt : (int64_t)b * S + tok;  // (first) token's row
+  const int64_t pgrp = (int64_t)b * pk.groups + tok;
+  const int32_t* ridx = kPack ? pk.idx + pgrp * pk.cap : idx + row_id * K;
+  if constexpr (kPack) K = pk.cap;
+  int nblk;
+  if constexpr (kPack) {
+    nblk = (pk.count[pgrp] + kBN - 1) / kBN;
+  } else {
+    int vidx[kIdxU];
+    load_row_indices(ridx, K, vidx);
+    nblk = count_row_blocks(ridx, K, s_kv, tok + q_offset, vidx, &sh_last);
+  }
   if (nblk == 0) return;
   const int nslots = min(K, nblk * kBN);
   const uint16_t* grow = gbuf + ((int64_t)b * rows + lr) * (int64_t)g_slots(K) * kGW;
@@ -729,11 +790,20 @@ bwd_contrib_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ 
       const int i = tid + kCThreads * m;
       const int ic = min(i, kXChunks - 1);
       const int row = ic / kRC, c = ic - row * kRC;
-      const int head = hgk * kHG + row;
-      const int64_t hrow = row_id * H + min(head, H - 1);
+      int head = hgk * kHG + row;
+      bool hok = head < H;
+      if constexpr (kPack) {  // (token, head) of the row, as an offset of whole heads from the group's first
+        int t;
+        pack_row(pk, head, t, head);
+        hok = t < pk.tt && tok * pk.tt + t < S && head < H;
+        head = hok ? t * H + head : 0;
+      } else {
+        head = min(head, H - 1);
+      }
+      const int64_t hrow = row_id * H + head;
       const u32x4 v = type == 0 ? *reinterpret_cast<const u32x4*>(q + hrow * kD + c * 8)
                                 : *reinterpret_cast<const u32x4*>(dout + hrow * kDv + min(c, kDv / 8 - 1) * 8);
-      const bool ok = i < kXChunks && head < H && (type == 0 || c < kDv / 8);
+      const bool ok = i < kXChunks && hok && (type == 0 || c < kDv / 8);
       xraw[kc][m] = ok ? v : (u32x4){0u, 0u, 0u, 0u};
     }
   }
@@ -1021,18 +1091,140 @@ BwdPlan plan_bwd(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int64_t
 
 constexpr int64_t kDefaultBudget = 32LL << 30;  // scratch for the G / C chunks (C3 in one chunk)
 
+// Scratch of the packed-token backward: the plan, then per chunk of `rows` groups G, C, delta
+// (twice: delta and the sink part) and the per-token mass.  total = 0: unpacked.
+struct PackBwdPlan {
+  int tt;
+  int64_t rows, plan_bytes, g_bytes, c_bytes, delta_bytes, mass_bytes, total;
+};
+PackBwdPlan plan_pack_bwd(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t topk, int64_t q_offset,
+                          int64_t budget, int64_t width) {
+  PackBwdPlan p{};
+  p.tt = pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset);
+  if (p.tt <= 1) return p;
+  const int64_t cap = pack_cap(topk, p.tt), groups = pack_groups(s_q, p.tt);
+  auto al = [](int64_t x) { return (x + 255) / 256 * 256; };
+  p.plan_bytes = pack_plan_bytes(batch, s_q, s_kv, topk, p.tt, true);
+  const int64_t per_row = batch * (cap * (kGW * 2 + width * 2 + p.tt * 4) + 2 * kHeadsMax * 4);
+  p.rows = std::min<int64_t>(groups, (budget - p.plan_bytes - 5 * 256) / per_row);
+  if (p.rows < 1) return p;
+  p.g_bytes = al(batch * p.rows * cap * kGW * 2);
+  p.c_bytes = al(batch * p.rows * cap * width * 2);
+  p.delta_bytes = al(batch * p.rows * kHeadsMax * 4);
+  p.mass_bytes = al(batch * p.rows * p.tt * cap * 4);
+  p.total = p.plan_bytes + p.rows * per_row + 5 * 256;  // (at least the parts; the same rows for this budget)
+  return p;
+}
+
 }  // namespace
 }  // namespace dsa
 
 extern "C" int64_t dsa_sparse_mla_bwd_workspace_size(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
                                                      int64_t d_qk, int64_t topk) {
-  (void)n_heads;
   if (batch <= 0 || s_q <= 0 || s_kv <= 0 || topk <= 0) return 0;
   const int64_t width = d_qk == dsa::kDv ? dsa::kDv : dsa::kDqk;  // C row width of the bf16 path
-  return dsa::plan_bwd(batch, s_q, s_kv, topk, dsa::kDefaultBudget, width).total;
+  const dsa::PackBwdPlan pp = dsa::plan_pack_bwd(batch, s_q, s_kv, n_heads, topk, 0, dsa::kDefaultBudget, width);
+  const bool either = pp.total && !dsa::plan_pack_bwd(batch, s_q, s_kv, n_heads, topk, s_kv, dsa::kDefaultBudget,
+                                                      width).total;  // (packed or not by the call's q_offset)
+  if (pp.total && !either) return pp.total;
+  return std::max(pp.total, dsa::plan_bwd(batch, s_q, s_kv, topk, dsa::kDefaultBudget, width).total);
 }
 
 namespace dsa {
+// delta and d sink of the tokens [t0, t0 + nt) of every batch element
+static int launch_sink_delta(const void* out, const void* dout, const float* smax, const float* ssum,
+                             const float* sinks, float* dsink, float* dbuf, float* pdbuf, int64_t batch, int64_t s_q,
+                             int64_t n_heads, int t0, int nt, hipStream_t st) {
+  {
+    const int64_t groups = batch * nt * n_heads;
+    const TimedLaunch tl("bwd_delta_kernel", st);
+    bwd_delta_kernel<<<(unsigned)((groups * 16 + 255) / 256), 256, 0, st>>>(
+        (const uint16_t*)out, (const uint16_t*)dout, dbuf, groups, (int)s_q, (int)n_heads, t0, nt, sinks, smax, ssum,
+        pdbuf);
+    if (int rc = check_launch("dsa_sparse_mla_bwd(delta)")) return rc;
+  }
+  const TimedLaunch tl("sink_colsum_kernel", st);
+  sink_colsum_kernel<<<(unsigned)n_heads, 256, 0, st>>>(pdbuf, batch * nt, (int)n_heads, dsink);
+  return check_launch("dsa_sparse_mla_bwd(sink)");
+}
+
+// alpha-1, alpha-2 and beta over the chunk's rows (tokens, or groups of packed tokens)
+template <bool kPack>
+static int launch_pair_kernels(dim3 ga, int hgroups, const void* q, const void* kv, const int32_t* indices,
+                               const void* out, const void* dout, const float* softmax_max, const float* softmax_sum,
+                               const float* dbuf, uint16_t* gbuf, uint16_t* cbuf, void* dq, float* mass, int64_t s_q,
+                               int64_t s_kv, int64_t n_heads, bool rope, int64_t topk, float scale, int64_t q_offset,
+                               int r0, int rows, const float* sinks, const PackView& pk, hipStream_t st) {
+  {
+    static const char* const names[2][2] = {{"bwd_sdp_kernel<512>", "bwd_sdp_kernel<512, packed>"},
+                                            {"bwd_sdp_kernel", "bwd_sdp_kernel<packed>"}};
+    const TimedLaunch tl(names[rope][kPack], st);
+    // with no sink, delta is formed inside (the sink's gradient needs the delta pass)
+    auto* kern = sinks ? (rope ? bwd_sdp_kernel<kDqk, false, kPack> : bwd_sdp_kernel<kDv, false, kPack>)
+                       : (rope ? bwd_sdp_kernel<kDqk, true, kPack> : bwd_sdp_kernel<kDv, true, kPack>);
+    kern<<<ga, 64 * kSdpWaves, 0, st>>>((const uint16_t*)q, (const uint16_t*)kv, indices, (const uint16_t*)dout,
+                                        (const uint16_t*)out, softmax_max, softmax_sum, dbuf, gbuf, mass, (int)s_q,
+                                        (int)s_kv, (int)n_heads, (int)topk, scale, q_offset, r0, pk);
+  }
+  if (int rc = check_launch("dsa_sparse_mla_bwd(sdp)")) return rc;
+  {
+    static const char* const names[2][2] = {{"bwd_dqk_kernel<512>", "bwd_dqk_kernel<512, packed>"},
+                                            {"bwd_dqk_kernel", "bwd_dqk_kernel<packed>"}};
+    const TimedLaunch tl(names[rope][kPack], st);
+    auto* kern = rope ? bwd_dqk_kernel<kDqk, kPack> : bwd_dqk_kernel<kDv, kPack>;
+    const int threads = 64 * (rope ? DqkShape<kDqk>::kWaves : DqkShape<kDv>::kWaves);
+    kern<<<ga, threads, 0, st>>>((const uint16_t*)kv, indices, gbuf, (uint16_t*)dq, (int)s_q, (int)s_kv, (int)n_heads,
+                                 (int)topk, q_offset, r0, pk);
+  }
+  if (int rc = check_launch("dsa_sparse_mla_bwd(dq)")) return rc;
+  dim3 gb(ga.x, ga.z);
+  static const char* const names[2][2][2] = {
+      {{"bwd_contrib_kernel<1,512>", "bwd_contrib_kernel<1,512, packed>"},
+       {"bwd_contrib_kernel<2,512>", "bwd_contrib_kernel<2,512, packed>"}},
+      {{"bwd_contrib_kernel<1>", "bwd_contrib_kernel<1, packed>"},
+       {"bwd_contrib_kernel<2>", "bwd_contrib_kernel<2, packed>"}}};
+  const TimedLaunch tl(names[rope][hgroups == 1 ? 0 : 1][kPack], st);
+  auto* kern = rope ? (hgroups == 1 ? bwd_contrib_kernel<1, kDqk, kPack> : bwd_contrib_kernel<2, kDqk, kPack>)
+                    : (hgroups == 1 ? bwd_contrib_kernel<1, kDv, kPack> : bwd_contrib_kernel<2, kDv, kPack>);
+  kern<<<gb, kCThreads, 0, st>>>((const uint16_t*)q, (const uint16_t*)dout, indices, gbuf, cbuf, (int)s_q, (int)s_kv,
+                                 (int)n_heads, (int)topk, q_offset, r0, rows, pk);
+  return check_launch("dsa_sparse_mla_bwd(contrib)");
+}
+
+// The backward over groups of packed tokens (attn_pack.h).
+static int sparse_mla_bwd_packed(const void* q, const void* kv, const int32_t* indices, const void* out,
+                                 const void* dout, const float* softmax_max, const float* softmax_sum, void* dq,
+                                 float* dkv_accum, float* mass, char* ws, const PackBwdPlan& plan, int64_t batch,
+                                 int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t d_qk, int64_t topk, float scale,
+                                 int64_t q_offset, const float* sinks, float* dsink, hipStream_t st) {
+  PackView pk;
+  if (int rc = pack_plan_build(indices, batch, s_q, s_kv, n_heads, topk, q_offset, plan.tt, true, ws, st, &pk))
+    return rc;
+  char* p = ws + plan.plan_bytes;
+  uint16_t* gbuf = (uint16_t*)p;
+  uint16_t* cbuf = (uint16_t*)(p + plan.g_bytes);
+  float* dbuf = (float*)(p + plan.g_bytes + plan.c_bytes);
+  float* pdbuf = (float*)(p + plan.g_bytes + plan.c_bytes + plan.delta_bytes);
+  if (mass) pk.mass = (float*)(p + plan.g_bytes + plan.c_bytes + 2 * plan.delta_bytes);
+  const int hgroups = plan.tt * pk.hp <= kHG ? 1 : 2;  // 64-row halves of the workgroup in use
+  for (int64_t g0 = 0; g0 < pk.groups; g0 += plan.rows) {
+    const int n = (int)std::min<int64_t>(plan.rows, pk.groups - g0);
+    const int t0 = (int)(g0 * plan.tt), nt = (int)std::min<int64_t>((int64_t)n * plan.tt, s_q - t0);
+    if (sinks)
+      if (int rc = launch_sink_delta(out, dout, softmax_max, softmax_sum, sinks, dsink, dbuf, pdbuf, batch, s_q,
+                                     n_heads, t0, nt, st))
+        return rc;
+    if (int rc = launch_pair_kernels<true>(dim3((unsigned)n, 1, (unsigned)batch), hgroups, q, kv, indices, out, dout,
+                                           softmax_max, softmax_sum, dbuf, gbuf, cbuf, dq, nullptr, s_q, s_kv, n_heads,
+                                           d_qk == kDqk, topk, scale, q_offset, (int)g0, n, sinks, pk, st))
+      return rc;
+    if (mass)
+      if (int rc = pack_mass_gather(pk, mass, batch, s_q, topk, g0, n, st)) return rc;
+    if (int rc = pack_dkv_reduce(pk, cbuf, dkv_accum, batch, s_kv, d_qk, g0, n, st)) return rc;
+  }
+  return DSA_OK;
+}
+
 static int sparse_mla_bwd_impl(const void* q, const void* kv, const int32_t* indices, const void* out,
                                const void* dout, const float* softmax_max, const float* softmax_sum, void* dq,
                                float* dkv_accum, float* mass, void* workspace, int64_t workspace_bytes, int dtype,
@@ -1070,6 +1262,12 @@ static int sparse_mla_bwd_impl(const void* q, const void* kv, const int32_t* ind
   const int64_t max_rows = rope ? GatherGeom::kMaxRows : GatherGeomT<kDv>::kMaxRows;
   if (s_kv > max_rows) return set_error(DSA_ERR_UNSUPPORTED, "dsa_sparse_mla_bwd: S_kv > %lld", (long long)max_rows);
   if (!workspace) return set_error(DSA_ERR_INVALID_ARG, "dsa_sparse_mla_bwd: workspace required");
+  const unsigned hgroups = ceil_div(n_heads, kHG);
+  const PackBwdPlan pp = plan_pack_bwd(batch, s_q, s_kv, n_heads, topk, q_offset, workspace_bytes, d_qk);
+  if (pp.total && (uintptr_t)workspace % 16 == 0)
+    return sparse_mla_bwd_packed(q, kv, indices, out, dout, softmax_max, softmax_sum, dq, dkv_accum, mass,
+                                 (char*)workspace, pp, batch, s_q, s_kv, n_heads, d_qk, topk, scale, q_offset, sinks,
+                                 dsink, st);
   // choose the largest chunk whose scratch fits the given workspace
   BwdPlan plan = plan_bwd(batch, s_q, s_kv, topk, workspace_bytes, d_qk);
   while (plan.total > workspace_bytes && plan.rows > 1) plan = plan_bwd(batch, plan.rows - 1, s_kv, topk, 0, d_qk);
@@ -1084,53 +1282,18 @@ static int sparse_mla_bwd_impl(const void* q, const void* kv, const int32_t* ind
   int* counts = (int*)(ws + al(plan.g_bytes) + al(plan.c_bytes) + al(plan.pairs_bytes));
   float* dbuf = (float*)(ws + al(plan.g_bytes) + al(plan.c_bytes) + al(plan.pairs_bytes) + al(plan.csr_bytes));
   float* pdbuf = (float*)((char*)dbuf + al(plan.delta_bytes));  // the sink's per-(row, head) gradient parts
-  const unsigned hgroups = ceil_div(n_heads, kHG);
 
   for (int64_t r0 = 0; r0 < s_q; r0 += plan.rows) {
     const int rows = (int)std::min<int64_t>(plan.rows, s_q - r0);
-    if (sinks) {
-      const int64_t groups = batch * rows * n_heads;
-      const TimedLaunch tl("bwd_delta_kernel", st);
-      bwd_delta_kernel<<<(unsigned)((groups * 16 + 255) / 256), 256, 0, st>>>(
-          (const uint16_t*)out, (const uint16_t*)dout, dbuf, groups, (int)s_q, (int)n_heads, (int)r0, rows, sinks,
-          softmax_max, softmax_sum, pdbuf);
-      if (int rc = check_launch("dsa_sparse_mla_bwd(delta)")) return rc;
-    }
-    if (sinks) {
-      const TimedLaunch tl("sink_colsum_kernel", st);
-      sink_colsum_kernel<<<(unsigned)n_heads, 256, 0, st>>>(pdbuf, batch * rows, (int)n_heads, dsink);
-      if (int rc = check_launch("dsa_sparse_mla_bwd(sink)")) return rc;
-    }
+    if (sinks)
+      if (int rc = launch_sink_delta(out, dout, softmax_max, softmax_sum, sinks, dsink, dbuf, pdbuf, batch, s_q,
+                                     n_heads, (int)r0, rows, st))
+        return rc;
     dim3 ga((unsigned)rows, 1, (unsigned)batch);
-    {
-      const TimedLaunch tl(rope ? "bwd_sdp_kernel" : "bwd_sdp_kernel<512>", st);
-      // with no sink, delta is formed inside (the sink's gradient needs the delta pass)
-      auto* kern = sinks ? (rope ? bwd_sdp_kernel<kDqk, false> : bwd_sdp_kernel<kDv, false>)
-                         : (rope ? bwd_sdp_kernel<kDqk, true> : bwd_sdp_kernel<kDv, true>);
-      kern<<<ga, 64 * kSdpWaves, 0, st>>>((const uint16_t*)q, (const uint16_t*)kv, indices, (const uint16_t*)dout,
-                                          (const uint16_t*)out, softmax_max, softmax_sum, dbuf, gbuf, mass, (int)s_q,
-                                          (int)s_kv, (int)n_heads, (int)topk, scale, q_offset, (int)r0);
-    }
-    if (int rc = check_launch("dsa_sparse_mla_bwd(sdp)")) return rc;
-    {
-      const TimedLaunch tl(rope ? "bwd_dqk_kernel" : "bwd_dqk_kernel<512>", st);
-      auto* kern = rope ? bwd_dqk_kernel<kDqk> : bwd_dqk_kernel<kDv>;
-      const int threads = 64 * (rope ? DqkShape<kDqk>::kWaves : DqkShape<kDv>::kWaves);
-      kern<<<ga, threads, 0, st>>>((const uint16_t*)kv, indices, gbuf, (uint16_t*)dq, (int)s_q, (int)s_kv,
-                                   (int)n_heads, (int)topk, q_offset, (int)r0);
-    }
-    if (int rc = check_launch("dsa_sparse_mla_bwd(dq)")) return rc;
-    dim3 gb((unsigned)rows, (unsigned)batch);
-    {
-      static const char* const names[2][2] = {{"bwd_contrib_kernel<1,512>", "bwd_contrib_kernel<2,512>"},
-                                              {"bwd_contrib_kernel<1>", "bwd_contrib_kernel<2>"}};
-      const TimedLaunch tl(names[rope][hgroups == 1 ? 0 : 1], st);
-      auto* kern = rope ? (hgroups == 1 ? bwd_contrib_kernel<1, kDqk> : bwd_contrib_kernel<2, kDqk>)
-                        : (hgroups == 1 ? bwd_contrib_kernel<1, kDv> : bwd_contrib_kernel<2, kDv>);
-      kern<<<gb, kCThreads, 0, st>>>((const uint16_t*)q, (const uint16_t*)dout, indices, gbuf, cbuf, (int)s_q,
-                                     (int)s_kv, (int)n_heads, (int)topk, q_offset, (int)r0, rows);
-    }
-    if (int rc = check_launch("dsa_sparse_mla_bwd(contrib)")) return rc;
+    if (int rc = launch_pair_kernels<false>(ga, (int)hgroups, q, kv, indices, out, dout, softmax_max, softmax_sum, dbuf,
+                                            gbuf, cbuf, dq, mass, s_q, s_kv, n_heads, rope, topk, scale, q_offset,
+                                            (int)r0, rows, sinks, PackView(), st))
+      return rc;
     // a prebuilt CSR of every row serves a one-chunk plan; otherwise each chunk builds its own
     const bool prebuilt = csr && rows == s_q;
     for (int b = 0; b < (int)batch; ++b) {
@@ -1157,6 +1320,13 @@ static int check_pair_csr(const void* csr, int64_t csr_bytes, int64_t batch, int
   return DSA_OK;
 }
 }  // namespace dsa
+
+extern "C" int dsa_sparse_mla_bwd_packed(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t d_qk,
+                                         int64_t topk, int64_t q_offset, int64_t workspace_bytes) {
+  using namespace dsa;
+  if (batch <= 0 || s_q <= 0 || s_kv <= 0 || topk <= 0 || workspace_bytes <= 0) return 0;
+  return plan_pack_bwd(batch, s_q, s_kv, n_heads, topk, q_offset, workspace_bytes, d_qk).total ? 1 : 0;
+}
 
 extern "C" int64_t dsa_sparse_mla_bwd_chunk_rows(int64_t batch, int64_t s_q, int64_t s_kv, int64_t d_qk,
                                                  int64_t topk, int64_t workspace_bytes) {

@@ -19,6 +19,7 @@
 //     accumulation registers.
 // LDS traffic per token and block is 4 waves x (QK + PV) tile reads; one barrier per
 // block, for the tile hand-off.
+#include "attn_pack.h"
 #include "dsa_common.h"
 #include "dsa_gather.h"
 
@@ -37,12 +38,16 @@ constexpr int kLatSteps = kDv / 16;            // 32 latent k-steps (Q in regist
 
 
 
-template <int kD>  // row width of Q and KV: 576 (latent + rope) or 512 (no rope)
+// kD: row width of Q and KV, 576 (latent + rope) or 512 (no rope).  kPack: the workgroup is a
+// group of packed tokens (attn_pack.h): its rows are (token, head) pairs, its slots the
+// union of the tokens' keys, and a row's validity bits its own token's mask words (scalar
+// loads, one block ahead; at most two tokens per 32-row wave, split at row 16).
+template <int kD, bool kPack>
 __global__ void __launch_bounds__(kFwdThreads, 1)
 sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv,
                            const int32_t* __restrict__ idx, uint16_t* __restrict__ out, float* __restrict__ smax,
                            float* __restrict__ ssum, int S, int s_kv, int H, int K, float scale_log2,
-                           int64_t q_offset, const float* __restrict__ sinks) {
+                           int64_t q_offset, const float* __restrict__ sinks, PackView pk) {
   using Gather = RowGather<kFwdWaves, kD>;
   using Geo = GatherGeomT<kD>;
   constexpr int kPer = Gather::kMaxPerWave;
@@ -54,22 +59,37 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
   __shared__ int sidx[GatherGeom::kRing][Gather::kRingInts];
   __shared__ int sh_last;
 
-  const int tok = blockIdx.x, b = blockIdx.z, tid = threadIdx.x;
+  const int b = blockIdx.z, tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int n = lane & 31, h = lane >> 5;  // MFMA column (head / key row) and k half
-  const int hl = wave * 32 + n;           // head within the workgroup
-  const int head = blockIdx.y * kFwdHeads + hl;
-  const bool hok = head < H;
+  const int hl = wave * 32 + n;           // row within the workgroup
+  const int grp = kPack ? launch_row() : 0;
+  int tok = blockIdx.x, head = blockIdx.y * kFwdHeads + hl;
+  bool hok = head < H;
+  if constexpr (kPack) {
+    int t;
+    pack_row(pk, hl, t, head);
+    tok = grp * pk.tt + t;
+    hok = t < pk.tt && tok < S && head < H;
+    if (!hok) tok = grp * pk.tt;  // (a token that exists)
+  }
   const int64_t row_id = (int64_t)b * S + tok;
-  const int64_t orow = row_id * H + (hok ? head : 0);
-  const int32_t* ridx = idx + row_id * K;
-  const int64_t limit = tok + q_offset;
+  int64_t orow = row_id * H + (hok ? head : 0);
+  const int64_t pgrp = (int64_t)b * pk.groups + grp;
+  const int32_t* ridx = kPack ? pk.idx + pgrp * pk.cap : idx + row_id * K;
+  if constexpr (kPack) K = pk.cap;
+  const int64_t limit = kPack ? (int64_t)s_kv : tok + q_offset;  // (packed: the plan applied the causal rule)
   const uint16_t* kvb = kv + (int64_t)b * s_kv * kD;
+  // packed: mask words of the tokens of rows 0..15 and 16..31 of the wave
+  const pack_word* mrow[2] = {nullptr, nullptr};
+  if constexpr (kPack)
+#pragma unroll
+    for (int x = 0; x < 2; ++x) mrow[x] = pack_mask_row(pk, pgrp, 32 * wave + 16 * x);
 
   // the row's slot indices (block count), the index ring entries of blocks 0..2 (wave 0,
   // DMA) and the row's Q are requested together; the block count waits only for the indices
   int vidx[kIdxU];
-  load_row_indices(ridx, K, vidx);
+  if constexpr (!kPack) load_row_indices(ridx, K, vidx);
   if (wave == 0) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) Gather::issue_idx(ridx, K, i, sidx[i], lane);  // clamped to slot K-1
@@ -87,7 +107,7 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
 #pragma unroll
     for (int j = 0; j < 4; ++j) qr[j] = kRope ? qh[64 + 4 * h + j] : (u32x4){0u, 0u, 0u, 0u};  // rope chunks 64 + 4h ..
   }
-  const int nblk = count_row_blocks(ridx, K, s_kv, limit, vidx, &sh_last);
+  const int nblk = kPack ? (pk.count[pgrp] + kBN - 1) / kBN : count_row_blocks(ridx, K, s_kv, limit, vidx, &sh_last);
   if (nblk == 0) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the ring DMA has landed before the LDS is released
     if (hok) {
@@ -163,7 +183,12 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
   if (wave == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // ring entries 0..2 landed
   __syncthreads();                                                  // publishes them and qpe
   for (int i = tid; i < kTC; i += kFwdThreads) tile[2][i] = (u32x4){0u, 0u, 0u, 0u};
-  uint32_t vm_cur = Gather::ring_valid(sidx[0], lane, lim, K);
+  uint32_t vm_cur = 0u;
+  if constexpr (!kPack) vm_cur = Gather::ring_valid(sidx[0], lane, lim, K);
+  uint32_t mw[2] = {0u, 0u};  // (packed) mask words of the block
+  if constexpr (kPack)
+#pragma unroll
+    for (int x = 0; x < 2; ++x) mw[x] = mrow[x][0];
 #pragma unroll
   for (int i = 0; i < kPer; ++i) Gather::issue_slot(kvb, &tile[0][0], i, wave, Gather::ring_slot(sidx[0], i, gl), gl, lim, K);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -184,7 +209,8 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
   // the rows land in a buffer nobody reads: every offset stays inside the KV tensor (a slot
   // is used only if it is <= lim, else row 0 is read).
   auto qk = [&](const lds_char* tb, u32x4* dst_tile, const int* ring, int rows_left, f32x16& sacc) {
-    const uint32_t vm_n = Gather::ring_valid(ring, lane, lim, rows_left);
+    uint32_t vm_n = 0u;
+    if constexpr (!kPack) vm_n = Gather::ring_valid(ring, lane, lim, rows_left);
     uint32_t raw_next = Gather::ring_slot(ring, 0, gl);
     sacc = (f32x16){0.f};
     u32x4 a[2][kQBatch];
@@ -305,6 +331,12 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
   for (int blk = 0; blk < nblk; ++blk) {
     if (wave == 0 && blk + 3 < nblk)
       Gather::issue_idx(ridx, K, blk + 3, sidx[(blk + 3) & (GatherGeom::kRing - 1)], lane);
+    uint32_t mw_next[2] = {0u, 0u};
+    if constexpr (kPack) {
+      vm_cur = n < 16 ? mw[0] : mw[1];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) mw_next[x] = mrow[x][min(blk + 1, nblk - 1)];
+    }
     f32x16 sacc;
     // ring entry blk+1 landed during iteration blk-2 (or before the loop)
     const uint32_t vm_next = qk(lds_bytes(&tile[blk % 3][0]), &tile[(blk + 1) % 3][0],
@@ -314,6 +346,10 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // block blk+1 and ring entry blk+3 landed
     __syncthreads();
     vm_cur = vm_next;
+    if constexpr (kPack) {
+      mw[0] = mw_next[0];
+      mw[1] = mw_next[1];
+    }
     bp_prev[0] = bp_new[0];
     bp_prev[1] = bp_new[1];
   }
@@ -321,6 +357,14 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
 
   // ---- epilogue: lane holds dv = 32 dt + 8 j + 4 h + i of its head ----
   const float ls = xor32_sum(lsum);
+  if constexpr (kPack) {  // (the row is found again instead of holding it in registers over the loop)
+    int r = hl, t;
+    asm volatile("" : "+v"(r));
+    pack_row(pk, r, t, head);
+    const int tk = grp * pk.tt + t;
+    hok = t < pk.tt && tk < S && head < H;
+    orow = ((int64_t)b * S + tk) * H + head;
+  }
   if (!hok) return;
   // a per-head sink (a logit with no value, natural-log units of the scaled score) joins
   // the row's denominator: O = acc / (ls + 2^(sink2 - m_ref)), and the row statistics
@@ -714,10 +758,18 @@ extern "C" int dsa_attn_mass(const void* q, const void* kv, const int32_t* indic
 }
 
 namespace dsa {
+// Workspace of the packed-token forward (0: the problem runs unpacked).
+static int64_t fwd_workspace_bytes(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
+                                   int64_t topk, int64_t q_offset) {
+  if (dtype != DSA_BF16 || topk <= 0) return 0;
+  const int tt = pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset);
+  return tt > 1 ? pack_plan_bytes(batch, s_q, s_kv, topk, tt, false) : 0;
+}
+
 static int sparse_mla_fwd_impl(const void* q, const void* kv, const int32_t* indices, const float* sinks, void* out,
                                float* softmax_max, float* softmax_sum, int dtype, int64_t batch, int64_t s_q,
                                int64_t s_kv, int64_t n_heads, int64_t d_qk, int64_t d_v, int64_t topk, float scale,
-                               int64_t q_offset, void* stream) {
+                               int64_t q_offset, void* workspace, int64_t workspace_bytes, void* stream) {
   if (!q || !kv || !indices || !out || !softmax_max || !softmax_sum)
     return set_error(DSA_ERR_INVALID_ARG, "dsa_sparse_mla_fwd: null pointer");
   if (batch <= 0 || s_q <= 0 || s_kv <= 0 || n_heads <= 0 || topk <= 0 || d_v <= 0 || d_qk < d_v)
@@ -736,17 +788,25 @@ static int sparse_mla_fwd_impl(const void* q, const void* kv, const int32_t* ind
     const bool rope = d_qk == kDqk;
     const int64_t max_rows = rope ? GatherGeom::kMaxRows : GatherGeomT<kDv>::kMaxRows;
     if (s_kv > max_rows) return set_error(DSA_ERR_UNSUPPORTED, "dsa_sparse_mla_fwd: S_kv > %lld", (long long)max_rows);
-    dim3 grid((unsigned)s_q, ceil_div(n_heads, kFwdHeads), (unsigned)batch);
+    PackView pk;
+    const int64_t need = workspace ? fwd_workspace_bytes(dtype, batch, s_q, s_kv, n_heads, topk, q_offset) : 0;
+    const bool pack = need > 0 && workspace_bytes >= need && (uintptr_t)workspace % 16 == 0;
+    if (pack) {
+      if (int rc = pack_plan_build(indices, batch, s_q, s_kv, n_heads, topk, q_offset,
+                                   pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset), false, workspace, st, &pk))
+        return rc;
+    }
+    dim3 grid((unsigned)(pack ? pk.groups : s_q), pack ? 1 : ceil_div(n_heads, kFwdHeads), (unsigned)batch);
     {
-      const TimedLaunch tl(rope ? "sparse_mla_fwd_bf16_kernel" : "sparse_mla_fwd_bf16_kernel<512>", st);
-      if (rope)
-        sparse_mla_fwd_bf16_kernel<kDqk><<<grid, kFwdThreads, 0, st>>>(
-            (const uint16_t*)q, (const uint16_t*)kv, indices, (uint16_t*)out, softmax_max, softmax_sum, (int)s_q,
-            (int)s_kv, (int)n_heads, (int)topk, scale * kLog2e, q_offset, sinks);
-      else
-        sparse_mla_fwd_bf16_kernel<kDv><<<grid, kFwdThreads, 0, st>>>(
-            (const uint16_t*)q, (const uint16_t*)kv, indices, (uint16_t*)out, softmax_max, softmax_sum, (int)s_q,
-            (int)s_kv, (int)n_heads, (int)topk, scale * kLog2e, q_offset, sinks);
+      static const char* const names[2][2] = {
+          {"sparse_mla_fwd_bf16_kernel<512>", "sparse_mla_fwd_bf16_kernel<512, packed>"},
+          {"sparse_mla_fwd_bf16_kernel", "sparse_mla_fwd_bf16_kernel<packed>"}};
+      const TimedLaunch tl(names[rope][pack], st);
+      auto* kern = pack ? (rope ? sparse_mla_fwd_bf16_kernel<kDqk, true> : sparse_mla_fwd_bf16_kernel<kDv, true>)
+                        : (rope ? sparse_mla_fwd_bf16_kernel<kDqk, false> : sparse_mla_fwd_bf16_kernel<kDv, false>);
+      kern<<<grid, kFwdThreads, 0, st>>>((const uint16_t*)q, (const uint16_t*)kv, indices, (uint16_t*)out, softmax_max,
+                                         softmax_sum, (int)s_q, (int)s_kv, (int)n_heads, (int)topk, scale * kLog2e,
+                                         q_offset, sinks, pk);
     }
     if (int rc = check_launch("dsa_sparse_mla_fwd(bf16)")) return rc;
     dim3 fgrid((unsigned)s_q, 1, (unsigned)batch);
@@ -773,7 +833,22 @@ extern "C" int dsa_sparse_mla_fwd(const void* q, const void* kv, const int32_t* 
                                   int64_t n_heads, int64_t d_qk, int64_t d_v, int64_t topk, float scale,
                                   int64_t q_offset, void* stream) {
   return dsa::sparse_mla_fwd_impl(q, kv, indices, nullptr, out, softmax_max, softmax_sum, dtype, batch, s_q, s_kv,
-                                  n_heads, d_qk, d_v, topk, scale, q_offset, stream);
+                                  n_heads, d_qk, d_v, topk, scale, q_offset, nullptr, 0, stream);
+}
+
+extern "C" int64_t dsa_sparse_mla_fwd_workspace_size(int dtype, int64_t batch, int64_t s_q, int64_t s_kv,
+                                                     int64_t n_heads, int64_t topk, int64_t q_offset) {
+  if (batch <= 0 || s_q <= 0 || s_kv <= 0) return 0;
+  return dsa::fwd_workspace_bytes(dtype, batch, s_q, s_kv, n_heads, topk, q_offset);
+}
+
+extern "C" int dsa_sparse_mla_fwd_ws(const void* q, const void* kv, const int32_t* indices, const float* sinks,
+                                     void* out, float* softmax_max, float* softmax_sum, int dtype, int64_t batch,
+                                     int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t d_qk, int64_t d_v,
+                                     int64_t topk, float scale, int64_t q_offset, void* workspace,
+                                     int64_t workspace_bytes, void* stream) {
+  return dsa::sparse_mla_fwd_impl(q, kv, indices, sinks, out, softmax_max, softmax_sum, dtype, batch, s_q, s_kv,
+                                  n_heads, d_qk, d_v, topk, scale, q_offset, workspace, workspace_bytes, stream);
 }
 
 extern "C" int dsa_sparse_mla_fwd_sink(const void* q, const void* kv, const int32_t* indices, const float* sinks,
@@ -782,5 +857,5 @@ extern "C" int dsa_sparse_mla_fwd_sink(const void* q, const void* kv, const int3
                                        int64_t topk, float scale, int64_t q_offset, void* stream) {
   if (!sinks) return dsa::set_error(DSA_ERR_INVALID_ARG, "dsa_sparse_mla_fwd_sink: null sinks");
   return dsa::sparse_mla_fwd_impl(q, kv, indices, sinks, out, softmax_max, softmax_sum, dtype, batch, s_q, s_kv,
-                                  n_heads, d_qk, d_v, topk, scale, q_offset, stream);
+                                  n_heads, d_qk, d_v, topk, scale, q_offset, nullptr, 0, stream);
 }

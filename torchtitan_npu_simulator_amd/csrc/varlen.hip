@@ -269,6 +269,57 @@ tnd_global_indices_kernel(const int32_t* __restrict__ idx, int32_t* __restrict__
 }  // namespace
 }  // namespace dsa
 
+// The same with the bounds of up to kHostSeqs sequences as kernel arguments (host bounds: no
+// copy to the device, so the call can be captured).  Workgroup y = sequence of the launch.
+namespace dsa {
+namespace {
+constexpr int kHostSeqs = 64;
+struct HostSeqs {
+  int q0[kHostSeqs + 1], k0[kHostSeqs + 1];
+};
+__global__ void __launch_bounds__(256)
+tnd_global_indices_host_kernel(const int32_t* __restrict__ idx, int32_t* __restrict__ out, HostSeqs seqs, int topk) {
+  const int i = blockIdx.y, lane = threadIdx.x & 63;
+  const int q0 = seqs.q0[i], lq = seqs.q0[i + 1] - q0, k0 = seqs.k0[i], lk = seqs.k0[i + 1] - k0;
+  const int off = max(0, lk - lq);
+  for (int r = blockIdx.x * 4 + (threadIdx.x >> 6); r < lq; r += gridDim.x * 4) {
+    const int n = min(r + off + 1, lk);
+    const int32_t* src = idx + (int64_t)(q0 + r) * topk;
+    int32_t* dst = out + (int64_t)(q0 + r) * topk;
+    for (int j = lane; j < topk; j += 64) {
+      const int v = src[j];
+      dst[j] = (v >= 0 && v < n) ? k0 + v : -1;
+    }
+  }
+}
+}  // namespace
+}  // namespace dsa
+
+extern "C" int dsa_tnd_global_indices_varlen(const int32_t* indices, int32_t* out, const int32_t* cu_seqlens_q,
+                                             const int32_t* cu_seqlens_k, int64_t n_seq, int64_t topk, void* stream) {
+  using namespace dsa;
+  const char* what = "dsa_tnd_global_indices_varlen";
+  if (!indices || !out) return set_error(DSA_ERR_INVALID_ARG, "%s: null pointer", what);
+  if (topk <= 0 || topk > 2147483647LL) return set_error(DSA_ERR_INVALID_ARG, "%s: bad sizes", what);
+  if (int rc = check_seqs(cu_seqlens_q, cu_seqlens_k, n_seq, what)) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  for (int64_t i0 = 0; i0 < n_seq; i0 += kHostSeqs) {
+    const int n = (int)std::min<int64_t>(kHostSeqs, n_seq - i0);
+    HostSeqs seqs{};
+    int most = 0;
+    for (int i = 0; i <= n; ++i) {
+      seqs.q0[i] = cu_seqlens_q[i0 + i];
+      seqs.k0[i] = cu_seqlens_k[i0 + i];
+      if (i > 0) most = std::max(most, seqs.q0[i] - seqs.q0[i - 1]);
+    }
+    if (most == 0) continue;
+    const TimedLaunch tl("tnd_global_indices_host_kernel", st);
+    tnd_global_indices_host_kernel<<<dim3(std::min(ceil_div(most, 4), 2048u), (unsigned)n), 256, 0, st>>>(indices, out,
+                                                                                                        seqs, (int)topk);
+  }
+  return check_launch(what);
+}
+
 extern "C" int dsa_tnd_global_indices(const int32_t* indices, int32_t* out, const int32_t* cu_seqlens_q,
                                       const int32_t* cu_seqlens_k, int64_t n_seq, int64_t t_q, int64_t t_k,
                                       int64_t topk, void* stream) {

@@ -560,10 +560,21 @@ def tnd_global_indices(indices, cu_seqlens_q, cu_seqlens_k, t_k):
     return out
 
 
-def _varlen_global(indices, cu_seqlens_q, cu_seqlens_kv, T, T_kv, device):
-    """Global indices [T,K] when the sequence bounds are on the device, else None."""
+def _varlen_global(indices, cu_seqlens_q, cu_seqlens_kv, T, T_kv, device, packed=False):
+    """Global indices [T,K] when the sequence bounds are on the device, or when the batch runs
+    over ``packed`` tokens (which may belong to neighbouring sequences); else None."""
     if not (_on_device(cu_seqlens_q) or _on_device(cu_seqlens_kv)):
-        return None
+        if not packed:
+            return None
+        cu_q, cu_k, n_seq = _varlen_seqs(cu_seqlens_q, cu_seqlens_kv, T, T_kv)
+        if any(q1 > q0 and k1 == k0 for q0, q1, k0, k1 in zip(cu_q, cu_q[1:], cu_k, cu_k[1:])):
+            return None  # (queries without keys: the per-sequence schedule refuses them)
+        indices = indices.reshape(T, -1).to(torch.int32).contiguous()
+        out = torch.empty_like(indices)
+        check(load_library().dsa_tnd_global_indices_varlen(ptr(indices), ptr(out), host_i32(cu_q), host_i32(cu_k),
+                                                           n_seq, indices.shape[1], stream_of(device)),
+              "dsa_tnd_global_indices_varlen")
+        return out
     cu_q, cu_k = _device_bounds(cu_seqlens_q, cu_seqlens_kv, device=device)
     if cu_q.numel() != cu_k.numel() or cu_q.numel() < 2:
         raise ValueError("cu_seqlens_q and cu_seqlens_kv describe different numbers of sequences")
@@ -574,11 +585,11 @@ def _varlen_global(indices, cu_seqlens_q, cu_seqlens_kv, T, T_kv, device):
 # gathered sparse MLA attention
 # ---------------------------------------------------------------------------
 def sparse_mla_fwd(q, kv, indices, scale, *, d_v=512, q_offset=0, sinks=None):
-    """(out [B,S,H,d_v], softmax_max [B,S,H], softmax_sum [B,S,H]) from dsa_sparse_mla_fwd.
+    """(out [B,S,H,d_v], softmax_max [B,S,H], softmax_sum [B,S,H]) from dsa_sparse_mla_fwd_ws.
 
     q [B,S,H,D_qk] bf16/fp32, kv [B,S_kv,D_qk] (v = kv[..., :d_v]), indices [B,S,K] int32.
-    ``sinks`` [H] (DeepSeek-V4's per-head attention sink) selects dsa_sparse_mla_fwd_sink: the
-    sink joins every row's softmax with no value, and the statistics returned include it.
+    ``sinks`` [H]: DeepSeek-V4's per-head attention sink; it joins every
+    row's softmax with no value, and the statistics returned include it.
     """
     global _attn_mass_entry
     _attn_mass_entry = None  # a mass kept by the last backward (take_attn_mass) is not for this call
@@ -593,18 +604,15 @@ def sparse_mla_fwd(q, kv, indices, scale, *, d_v=512, q_offset=0, sinks=None):
     out = torch.empty(B, S, H, d_v, dtype=q.dtype, device=q.device)
     smax = torch.empty(B, S, H, dtype=torch.float32, device=q.device)
     ssum = torch.empty(B, S, H, dtype=torch.float32, device=q.device)
-    if sinks is not None:
-        sk = _sink_vector(sinks, H, q.device)
-        check(
-            lib.dsa_sparse_mla_fwd_sink(ptr(q), ptr(kv), ptr(indices), ptr(sk), ptr(out), ptr(smax), ptr(ssum),
-                                        _lib.dtype_code(q.dtype), B, S, s_kv, H, D, d_v, K, float(scale),
-                                        int(q_offset), stream_of(q.device)),
-            "dsa_sparse_mla_fwd_sink",
-        )
-        return out, smax, ssum
+    sk = None if sinks is None else _sink_vector(sinks, H, q.device)
+    dt = _lib.dtype_code(q.dtype)
+    # scratch of the packed-token forward (fewer heads than a workgroup's rows)
+    ws_bytes = int(lib.dsa_sparse_mla_fwd_workspace_size(dt, B, S, s_kv, H, K, int(q_offset)))
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
     check(
-        lib.dsa_sparse_mla_fwd(ptr(q), ptr(kv), ptr(indices), ptr(out), ptr(smax), ptr(ssum), _lib.dtype_code(q.dtype),
-                               B, S, s_kv, H, D, d_v, K, float(scale), int(q_offset), stream_of(q.device)),
+        lib.dsa_sparse_mla_fwd_ws(ptr(q), ptr(kv), ptr(indices), ptr(sk), ptr(out), ptr(smax), ptr(ssum), dt, B, S,
+                                  s_kv, H, D, d_v, K, float(scale), int(q_offset), ptr(ws), ws_bytes,
+                                  stream_of(q.device)),
         "dsa_sparse_mla_fwd",
     )
     return out, smax, ssum
@@ -711,9 +719,12 @@ def sparse_mla_bwd(q, kv, indices, out, dout, smax, ssum, scale, *, q_offset=0, 
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=q.device)
     res = (dq, dkv, mass) if return_mass else (dq, dkv)
     # one chunk of rows: the dKV reduction takes the shared pair CSR (also the indexer loss's)
+    # (packed tokens reduce dKV by their own plan: there it is built for the loss alone, which
+    # a caller that asks for the mass runs next on the same indices)
     csr = None
     if _share_pair_csr and q.dtype == torch.bfloat16 and \
-            int(lib.dsa_sparse_mla_bwd_chunk_rows(B, S, s_kv, D, K, ws_bytes)) >= S:
+            (return_mass if lib.dsa_sparse_mla_bwd_packed(B, S, s_kv, H, D, K, int(q_offset), ws_bytes) else
+             int(lib.dsa_sparse_mla_bwd_chunk_rows(B, S, s_kv, D, K, ws_bytes)) >= S):
         csr = pair_csr(indices, s_kv, q_offset)
     sk = dsink = None
     if sinks is not None:
@@ -762,13 +773,16 @@ def sparse_mla_fwd_varlen(q, kv, indices, scale, cu_seqlens_q, cu_seqlens_kv, *,
     """Packed varlen forward (dsa_sparse_mla_fwd_varlen): q [T,H,D_qk], kv [T_kv,D_qk],
     indices [T,K] sequence-local; returns (out [T,H,d_v], softmax_max [T,H], softmax_sum [T,H]).
     With GPU-tensor bounds the batch runs as one launch on global key rows
-    (tnd_global_indices), with no host read; with host bounds, one launch per sequence."""
+    (tnd_global_indices), with no host read; with host bounds, one launch per sequence, or,
+    with few enough heads for several tokens to share a workgroup, the same one launch."""
     lib = load_library()
     require_gpu_tensor(q, "q")
     T, H, D = q.shape
     kv = kv.reshape(kv.shape[0], kv.shape[-1]).contiguous()
-    g = _varlen_global(indices, cu_seqlens_q, cu_seqlens_kv, T, kv.shape[0], q.device)
-    if g is not None:  # device bounds: one launch over the batch
+    packed = q.dtype == torch.bfloat16 and T > 0 and lib.dsa_sparse_mla_fwd_workspace_size(
+        _lib.DSA_BF16, 1, T, kv.shape[0], H, indices.shape[-1], _NO_MASK_OFFSET) > 0
+    g = _varlen_global(indices, cu_seqlens_q, cu_seqlens_kv, T, kv.shape[0], q.device, packed)
+    if g is not None:  # device bounds, packed tokens: one launch over the batch
         out, smax, ssum = sparse_mla_fwd(q.unsqueeze(0), kv.unsqueeze(0), g.unsqueeze(0), scale, d_v=d_v,
                                          q_offset=_NO_MASK_OFFSET)
         return out[0], smax[0], ssum[0]
@@ -797,8 +811,12 @@ def sparse_mla_bwd_varlen(q, kv, indices, out, dout, smax, ssum, scale, cu_seqle
     T, H, D = q.shape
     kv = kv.reshape(kv.shape[0], kv.shape[-1]).contiguous()
     T_kv = kv.shape[0]
-    g = _varlen_global(indices, cu_seqlens_q, cu_seqlens_kv, T, T_kv, q.device)
-    if g is not None:  # device bounds: one launch over the batch
+    K = indices.shape[-1]
+    packed = q.dtype == torch.bfloat16 and T > 0 and lib.dsa_sparse_mla_bwd_packed(
+        1, T, T_kv, H, D, K, _NO_MASK_OFFSET, lib.dsa_sparse_mla_bwd_workspace_size(1, T, T_kv, H, D, K)
+        if workspace_bytes is None else int(workspace_bytes)) == 1
+    g = _varlen_global(indices, cu_seqlens_q, cu_seqlens_kv, T, T_kv, q.device, packed)
+    if g is not None:  # device bounds, packed tokens: one launch over the batch
         res = sparse_mla_bwd(q.unsqueeze(0), kv.unsqueeze(0), g.unsqueeze(0), out.unsqueeze(0), dout.unsqueeze(0),
                              smax.unsqueeze(0), ssum.unsqueeze(0), scale, q_offset=_NO_MASK_OFFSET,
                              workspace_bytes=workspace_bytes, return_mass=return_mass)
