@@ -242,7 +242,8 @@ int dsa_sparse_mla_bwd(const void* q, const void* kv, const int32_t* indices, co
  * dsa_sparse_mla_fwd_workspace_size() bytes (16-byte aligned).  The size is 0 where the
  * workspace has no use; with fewer bytes, or none, the call runs as the entry points without
  * one do.  bf16 calls of at most 64 heads use it to let several consecutive tokens share a
- * workgroup, which gathers the union of their keys once.
+ * workgroup, which gathers the union of their keys once; bf16 calls of few tokens (generation)
+ * to split a token's keys over several workgroups.
  */
 int64_t dsa_sparse_mla_fwd_workspace_size(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
                                           int64_t topk, int64_t q_offset);

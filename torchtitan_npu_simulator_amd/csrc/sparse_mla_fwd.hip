@@ -19,6 +19,8 @@
 //     accumulation registers.
 // LDS traffic per token and block is 4 waves x (QK + PV) tile reads; one barrier per
 // block, for the tile hand-off.
+#include <algorithm>
+
 #include "attn_pack.h"
 #include "dsa_common.h"
 #include "dsa_gather.h"
@@ -42,12 +44,23 @@ constexpr int kLatSteps = kDv / 16;            // 32 latent k-steps (Q in regist
 // group of packed tokens (attn_pack.h): its rows are (token, head) pairs, its slots the
 // union of the tokens' keys, and a row's validity bits its own token's mask words (scalar
 // loads, one block ahead; at most two tokens per 32-row wave, split at row 16).
-template <int kD, bool kPack>
+// kSplit (at most 128 heads): blockIdx.y is a key split: the workgroup runs its share of the token's
+// blocks and leaves the unnormalised O and the row statistics in `part` (fp32), which
+// fwd_combine_kernel merges.
+enum class FwdMode { kPlain, kPack, kSplit };
+
+// partial results of one row and split: O [512], then the reference max, the true max (base 2,
+// -inf: no key), the sum at the reference and whether a logit outgrew the headroom
+constexpr int kPartFloats = kDv + 4;
+
+template <int kD, FwdMode kMode>
 __global__ void __launch_bounds__(kFwdThreads, 1)
 sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv,
                            const int32_t* __restrict__ idx, uint16_t* __restrict__ out, float* __restrict__ smax,
                            float* __restrict__ ssum, int S, int s_kv, int H, int K, float scale_log2,
-                           int64_t q_offset, const float* __restrict__ sinks, PackView pk) {
+                           int64_t q_offset, const float* __restrict__ sinks, PackView pk,
+                           float* __restrict__ part, int n_split) {
+  constexpr bool kPack = kMode == FwdMode::kPack, kSplit = kMode == FwdMode::kSplit;
   using Gather = RowGather<kFwdWaves, kD>;
   using Geo = GatherGeomT<kD>;
   constexpr int kPer = Gather::kMaxPerWave;
@@ -64,7 +77,8 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
   const int n = lane & 31, h = lane >> 5;  // MFMA column (head / key row) and k half
   const int hl = wave * 32 + n;           // row within the workgroup
   const int grp = kPack ? launch_row() : 0;
-  int tok = blockIdx.x, head = blockIdx.y * kFwdHeads + hl;
+  int tok = blockIdx.x, head = kSplit ? hl : (int)blockIdx.y * kFwdHeads + hl;
+  const int split = kSplit ? (int)blockIdx.y : 0;
   bool hok = head < H;
   if constexpr (kPack) {
     int t;
@@ -90,10 +104,14 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
   // DMA) and the row's Q are requested together; the block count waits only for the indices
   int vidx[kIdxU];
   if constexpr (!kPack) load_row_indices(ridx, K, vidx);
-  if (wave == 0) {
+  int bofs = 0;  // the row's block that is this workgroup's first
+  auto start_ring = [&]() {
+    if (wave == 0) {
 #pragma unroll
-    for (int i = 0; i < 3; ++i) Gather::issue_idx(ridx, K, i, sidx[i], lane);  // clamped to slot K-1
-  }
+      for (int i = 0; i < 3; ++i) Gather::issue_idx(ridx, K, bofs + i, sidx[i], lane);  // clamped to slot K-1
+    }
+  };
+  if constexpr (!kSplit) start_ring();
   // ---- Q: latent qb[s] = q[16s + 8h .. +8] of head `head` (B operand of S^T = K Q^T for
   // k-step s) in VGPRs; the rope columns go to LDS below ----
   // (unconditional loads, orow points at head 0 for absent heads: a load under a branch
@@ -107,7 +125,19 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
 #pragma unroll
     for (int j = 0; j < 4; ++j) qr[j] = kRope ? qh[64 + 4 * h + j] : (u32x4){0u, 0u, 0u, 0u};  // rope chunks 64 + 4h ..
   }
-  const int nblk = kPack ? (pk.count[pgrp] + kBN - 1) / kBN : count_row_blocks(ridx, K, s_kv, limit, vidx, &sh_last);
+  int nblk = kPack ? (pk.count[pgrp] + kBN - 1) / kBN : count_row_blocks(ridx, K, s_kv, limit, vidx, &sh_last);
+  if constexpr (kSplit) {  // the split's blocks of the row
+    const int b0 = __builtin_amdgcn_readfirstlane(nblk * split / n_split);  // (at most 512 blocks, 64 splits)
+    const int b1 = __builtin_amdgcn_readfirstlane(nblk * (split + 1) / n_split);
+    part += ((row_id * H + (hok ? head : 0)) * n_split + split) * kPartFloats;
+    if (b1 == b0) {
+      if (hok && h == 0) *reinterpret_cast<float4*>(part + kDv) = make_float4(-INFINITY, -INFINITY, 0.f, 0.f);
+      return;
+    }
+    bofs = b0;
+    nblk = b1 - b0;
+    start_ring();
+  }
   if (nblk == 0) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the ring DMA has landed before the LDS is released
     if (hok) {
@@ -184,13 +214,13 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
   __syncthreads();                                                  // publishes them and qpe
   for (int i = tid; i < kTC; i += kFwdThreads) tile[2][i] = (u32x4){0u, 0u, 0u, 0u};
   uint32_t vm_cur = 0u;
-  if constexpr (!kPack) vm_cur = Gather::ring_valid(sidx[0], lane, lim, K);
+  if constexpr (!kPack) vm_cur = Gather::ring_valid(sidx[0], lane, lim, K - bofs * kBN);
   uint32_t mw[2] = {0u, 0u};  // (packed) mask words of the block
   if constexpr (kPack)
 #pragma unroll
     for (int x = 0; x < 2; ++x) mw[x] = mrow[x][0];
 #pragma unroll
-  for (int i = 0; i < kPer; ++i) Gather::issue_slot(kvb, &tile[0][0], i, wave, Gather::ring_slot(sidx[0], i, gl), gl, lim, K);
+  for (int i = 0; i < kPer; ++i) Gather::issue_slot(kvb, &tile[0][0], i, wave, Gather::ring_slot(sidx[0], i, gl), gl, lim, K - bofs * kBN);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
 
@@ -330,7 +360,7 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
 
   for (int blk = 0; blk < nblk; ++blk) {
     if (wave == 0 && blk + 3 < nblk)
-      Gather::issue_idx(ridx, K, blk + 3, sidx[(blk + 3) & (GatherGeom::kRing - 1)], lane);
+      Gather::issue_idx(ridx, K, bofs + blk + 3, sidx[(blk + 3) & (GatherGeom::kRing - 1)], lane);
     uint32_t mw_next[2] = {0u, 0u};
     if constexpr (kPack) {
       vm_cur = n < 16 ? mw[0] : mw[1];
@@ -340,7 +370,7 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
     f32x16 sacc;
     // ring entry blk+1 landed during iteration blk-2 (or before the loop)
     const uint32_t vm_next = qk(lds_bytes(&tile[blk % 3][0]), &tile[(blk + 1) % 3][0],
-                                sidx[(blk + 1) & (GatherGeom::kRing - 1)], K - (blk + 1) * kBN, sacc);
+                                sidx[(blk + 1) & (GatherGeom::kRing - 1)], K - (bofs + blk + 1) * kBN, sacc);
     u32x4 bp_new[2];
     softmax_pv(lds_bytes(&tile[(blk + 2) % 3][0]), sacc, vm_cur, bp_new);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // block blk+1 and ring entry blk+3 landed
@@ -366,6 +396,16 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
     orow = ((int64_t)b * S + tk) * H + head;
   }
   if (!hok) return;
+  if constexpr (kSplit) {
+#pragma unroll
+    for (int dt = 0; dt < kDv / 32; ++dt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<float4*>(part + 32 * dt + 8 * j + 4 * h) =
+            make_float4(o[dt][4 * j], o[dt][4 * j + 1], o[dt][4 * j + 2], o[dt][4 * j + 3]);
+    if (h == 0) *reinterpret_cast<float4*>(part + kDv) = make_float4(m_ref, m_true, ls, clamped ? 1.f : 0.f);
+    return;
+  }
   // a per-head sink (a logit with no value, natural-log units of the scaled score) joins
   // the row's denominator: O = acc / (ls + 2^(sink2 - m_ref)), and the row statistics
   // become (m2, s2) = (max(m, sink), sum e^(x - m2) + e^(sink - m2)); with no valid key
@@ -394,6 +434,73 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
     // a negative sum marks a row whose logits outgrew the headroom; the fixup pass redoes it
     ssum[orow] = clamped ? -1.f : l_out;
   }
+}
+
+// Merges the splits of a row (one wave per row, lane l = columns 8 l .. +7):
+//   O = sum_s 2^(m_s - M) O_s / (sum_s 2^(m_s - M) l_s + 2^(sink - M)),  M = max m_s,
+// in fp32, with the statistics as the one-pass epilogue writes them.
+__global__ void __launch_bounds__(256)
+fwd_combine_kernel(const float* __restrict__ part, uint16_t* __restrict__ out, float* __restrict__ smax,
+                   float* __restrict__ ssum, int64_t rows, int H, int n_split, const float* __restrict__ sinks) {
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (row >= rows) return;
+  const float* p = part + row * n_split * kPartFloats;
+  // lane s holds split s's statistics (at most 64 splits)
+  float4 st = make_float4(-INFINITY, -INFINITY, 0.f, 0.f);
+  if (lane < n_split) st = *reinterpret_cast<const float4*>(p + (int64_t)lane * kPartFloats + kDv);
+  const float M = wave_max(st.x), mt = wave_max(st.y);
+  const float sk2 = sinks ? sinks[row % H] * kLog2e : -INFINITY;
+  const float w = st.x == -INFINITY ? 0.f : exp2f(st.x - M);
+  const float ls = wave_sum(w * st.z);
+  const bool clamped = __ballot(st.w != 0.f) != 0;
+  // (no key: M = -inf, every weight and O are 0, and a sink makes the denominator infinite)
+  const float den = sinks ? ls + exp2f(sk2 - M) : ls;
+  const float inv = den > 0.f ? 1.f / den : 0.f;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  constexpr int kU = 8;  // splits in flight
+  for (int s0 = 0; s0 < n_split; s0 += kU) {
+    f32x4 x[kU][2];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const f32x4* o4 = reinterpret_cast<const f32x4*>(p + (int64_t)min(s0 + u, n_split - 1) * kPartFloats + 8 * lane);
+      x[u][0] = o4[0];
+      x[u][1] = o4[1];
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const float ws = s0 + u < n_split ? __shfl(w, s0 + u, 64) : 0.f;
+      if (ws == 0.f) continue;  // (wave-uniform: a split without keys left no O)
+#pragma unroll
+      for (int r = 0; r < 8; ++r) acc[r] = fmaf(ws, x[u][r >> 2][r & 3], acc[r]);
+    }
+  }
+  u32x4 v;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v[r] = pack_bf16x2(acc[2 * r] * inv, acc[2 * r + 1] * inv);
+  *reinterpret_cast<u32x4*>(out + row * kDv + 8 * lane) = v;
+  if (lane == 0) {
+    const float l_true = ls > 0.f ? ls * exp2f(M - mt) : 0.f;
+    float m_out = mt, l_out = l_true;
+    if (sinks) {
+      m_out = fmaxf(mt, sk2);
+      l_out = (l_true > 0.f ? l_true * exp2f(mt - m_out) : 0.f) + exp2f(sk2 - m_out);
+    }
+    smax[row] = m_out * kLn2;
+    ssum[row] = clamped ? -1.f : l_out;  // (as the one-pass epilogue: the fixup pass redoes the row)
+  }
+}
+
+// Key splits per token (1: none).  A workgroup per (token, 128 heads) leaves CUs idle below 256
+// of them, as in generation: the row's blocks are then shared out so that the workgroups
+// about fill the chip, four blocks or more each.  Four rows of 128 heads over 2048 selected
+// keys: 133 us on 4 workgroups, 30 us on 64 and 6 us for the merge (two blocks each: 29 and
+// 9 us, the workgroup's start, about 20 us of cold code, Q and first gather, being the rest).
+int fwd_splits(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t topk) {
+  const int64_t wgs = batch * s_q;
+  const int64_t blocks = (std::min(topk, s_kv) + kBN - 1) / kBN;
+  if (wgs > 128 || n_heads > kFwdHeads) return 1;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / wgs, blocks / 4), 64));
 }
 
 // Head-summed softmax mass at the selected slots (target of the indexer KL loss):
@@ -758,12 +865,14 @@ extern "C" int dsa_attn_mass(const void* q, const void* kv, const int32_t* indic
 }
 
 namespace dsa {
-// Workspace of the packed-token forward (0: the problem runs unpacked).
+// Workspace of the packed-token or key-split forward (0: the problem runs as it is).
 static int64_t fwd_workspace_bytes(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
                                    int64_t topk, int64_t q_offset) {
   if (dtype != DSA_BF16 || topk <= 0) return 0;
   const int tt = pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset);
-  return tt > 1 ? pack_plan_bytes(batch, s_q, s_kv, topk, tt, false) : 0;
+  if (tt > 1) return pack_plan_bytes(batch, s_q, s_kv, topk, tt, false);
+  const int n_split = fwd_splits(batch, s_q, s_kv, n_heads, topk);
+  return n_split > 1 ? batch * s_q * n_heads * n_split * kPartFloats * 4 : 0;
 }
 
 static int sparse_mla_fwd_impl(const void* q, const void* kv, const int32_t* indices, const float* sinks, void* out,
@@ -790,23 +899,37 @@ static int sparse_mla_fwd_impl(const void* q, const void* kv, const int32_t* ind
     if (s_kv > max_rows) return set_error(DSA_ERR_UNSUPPORTED, "dsa_sparse_mla_fwd: S_kv > %lld", (long long)max_rows);
     PackView pk;
     const int64_t need = workspace ? fwd_workspace_bytes(dtype, batch, s_q, s_kv, n_heads, topk, q_offset) : 0;
-    const bool pack = need > 0 && workspace_bytes >= need && (uintptr_t)workspace % 16 == 0;
+    const bool use_ws = need > 0 && workspace_bytes >= need && (uintptr_t)workspace % 16 == 0;
+    const bool pack = use_ws && pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset) > 1;
+    const int n_split = use_ws && !pack ? fwd_splits(batch, s_q, s_kv, n_heads, topk) : 1;
     if (pack) {
       if (int rc = pack_plan_build(indices, batch, s_q, s_kv, n_heads, topk, q_offset,
                                    pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset), false, workspace, st, &pk))
         return rc;
     }
-    dim3 grid((unsigned)(pack ? pk.groups : s_q), pack ? 1 : ceil_div(n_heads, kFwdHeads), (unsigned)batch);
+    dim3 grid((unsigned)(pack ? pk.groups : s_q), pack ? 1 : n_split > 1 ? n_split : ceil_div(n_heads, kFwdHeads),
+              (unsigned)batch);
     {
-      static const char* const names[2][2] = {
-          {"sparse_mla_fwd_bf16_kernel<512>", "sparse_mla_fwd_bf16_kernel<512, packed>"},
-          {"sparse_mla_fwd_bf16_kernel", "sparse_mla_fwd_bf16_kernel<packed>"}};
-      const TimedLaunch tl(names[rope][pack], st);
-      auto* kern = pack ? (rope ? sparse_mla_fwd_bf16_kernel<kDqk, true> : sparse_mla_fwd_bf16_kernel<kDv, true>)
-                        : (rope ? sparse_mla_fwd_bf16_kernel<kDqk, false> : sparse_mla_fwd_bf16_kernel<kDv, false>);
+      static const char* const names[2][3] = {
+          {"sparse_mla_fwd_bf16_kernel<512>", "sparse_mla_fwd_bf16_kernel<512, packed>",
+           "sparse_mla_fwd_bf16_kernel<512, split>"},
+          {"sparse_mla_fwd_bf16_kernel", "sparse_mla_fwd_bf16_kernel<packed>", "sparse_mla_fwd_bf16_kernel<split>"}};
+      const int mode = pack ? 1 : n_split > 1 ? 2 : 0;
+      const TimedLaunch tl(names[rope][mode], st);
+      using M = FwdMode;
+      auto* kern = mode == 1   ? (rope ? sparse_mla_fwd_bf16_kernel<kDqk, M::kPack> : sparse_mla_fwd_bf16_kernel<kDv, M::kPack>)
+                   : mode == 2 ? (rope ? sparse_mla_fwd_bf16_kernel<kDqk, M::kSplit> : sparse_mla_fwd_bf16_kernel<kDv, M::kSplit>)
+                               : (rope ? sparse_mla_fwd_bf16_kernel<kDqk, M::kPlain> : sparse_mla_fwd_bf16_kernel<kDv, M::kPlain>);
       kern<<<grid, kFwdThreads, 0, st>>>((const uint16_t*)q, (const uint16_t*)kv, indices, (uint16_t*)out, softmax_max,
                                          softmax_sum, (int)s_q, (int)s_kv, (int)n_heads, (int)topk, scale * kLog2e,
-                                         q_offset, sinks, pk);
+                                         q_offset, sinks, pk, (float*)workspace, n_split);
+    }
+    if (n_split > 1) {
+      if (int rc = check_launch("dsa_sparse_mla_fwd(bf16, split)")) return rc;
+      const int64_t rows = batch * s_q * n_heads;
+      const TimedLaunch tl("fwd_combine_kernel", st);
+      fwd_combine_kernel<<<ceil_div(rows, 4), 256, 0, st>>>((const float*)workspace, (uint16_t*)out, softmax_max,
+                                                           softmax_sum, rows, (int)n_heads, n_split, sinks);
     }
     if (int rc = check_launch("dsa_sparse_mla_fwd(bf16)")) return rc;
     dim3 fgrid((unsigned)s_q, 1, (unsigned)batch);
