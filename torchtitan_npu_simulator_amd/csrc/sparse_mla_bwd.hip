@@ -24,6 +24,7 @@
 // workspace.
 #include <algorithm>
 
+#include "attn_f32.h"
 #include "attn_pack.h"
 #include "dsa_common.h"
 #include "dsa_csr.h"
@@ -1244,6 +1245,10 @@ static int sparse_mla_bwd_impl(const void* q, const void* kv, const int32_t* ind
     if (topk * 4 > 64 * 1024) return set_error(DSA_ERR_UNSUPPORTED, "dsa_sparse_mla_bwd: fp32 topk <= 16384");
     if (s_q > 2147483647LL || n_heads > 65535)
       return set_error(DSA_ERR_INVALID_ARG, "dsa_sparse_mla_bwd: sizes out of range");
+    if (attn_f32_fits(d_qk, d_v, n_heads) && attn_f32_aligned(q, kv, out, dout))
+      return attn_f32_bwd((const float*)q, (const float*)kv, indices, (const float*)out, (const float*)dout,
+                          softmax_max, softmax_sum, (float*)dq, dkv_accum, batch, s_q, s_kv, n_heads, d_qk, d_v, topk,
+                          scale, q_offset, sinks, dsink, st);
     dim3 grid((unsigned)s_q, (unsigned)n_heads, (unsigned)batch);
     {
       const TimedLaunch tl("bwd_exact_f32_kernel", st);

@@ -21,6 +21,7 @@
 // block, for the tile hand-off.
 #include <algorithm>
 
+#include "attn_f32.h"
 #include "attn_pack.h"
 #include "dsa_common.h"
 #include "dsa_gather.h"
@@ -940,6 +941,9 @@ static int sparse_mla_fwd_impl(const void* q, const void* kv, const int32_t* ind
     return check_launch("dsa_sparse_mla_fwd(bf16 fixup)");
   }
   if (dtype == DSA_F32) {
+    if (attn_f32_fits(d_qk, d_v, n_heads) && attn_f32_aligned(q, kv))
+      return attn_f32_fwd((const float*)q, (const float*)kv, indices, (float*)out, softmax_max, softmax_sum, batch, s_q,
+                          s_kv, n_heads, d_qk, d_v, topk, scale, q_offset, sinks, st);
     dim3 grid((unsigned)s_q, (unsigned)n_heads, (unsigned)batch);
     const TimedLaunch tl("sparse_mla_fwd_exact_kernel<float>", st);
     sparse_mla_fwd_exact_kernel<float><<<grid, 256, sc_bytes, st>>>(
