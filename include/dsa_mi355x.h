@@ -444,6 +444,17 @@ int dsa_compressor_fwd_tnd(const float* kv, const float* score, const float* ape
                            const float* rope_cs, int64_t n_pos, int64_t rope_dim, void* stream);
 
 /*
+ * Weight gradient of the absorb products, per head: g[i, j] = sum_t a[t, h, i] b[t, h, j] over
+ * bf16 rows a [tokens, heads, lda] (128 used) and b [tokens, heads, ldb] (512 used), fp32 sums.
+ * out (bf16 or fp32) is [heads, 128, 512], or [heads, 512, 128] (the transpose) with wide_rows.
+ * The workspace (dsa_mla_absorb_wgrad_workspace_size() bytes, 16-byte aligned) lets few heads
+ * split the tokens over workgroups; NULL or fewer bytes runs without.
+ */
+int64_t dsa_mla_absorb_wgrad_workspace_size(int64_t tokens, int64_t heads);
+int dsa_mla_absorb_wgrad(const void* a, int64_t lda, const void* b, int64_t ldb, void* out, int out_dtype,
+                         int wide_rows, int64_t tokens, int64_t heads, void* workspace, int64_t workspace_bytes,
+                         void* stream);
+/*
  * MLA weight absorption (reference: models/deepseek_v32/model.py:520-535, the einsum
  * q_nope . w_uk before the attention, and :574-575, the output . w_uv_t after it):
  *   c[t, h, 0:n] = sum_k a[t, h, k] * wt[h, :, k]   (bf16 in, fp32 accumulation, bf16 out)

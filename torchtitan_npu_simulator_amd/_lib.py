@@ -105,6 +105,8 @@ _SIGNATURES = {
     "dsa_indexer_prep": ([_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i32, _i32, _vp],
                          _i32),
     "dsa_mla_absorb": ([_vp, _i64, _vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp], _i32),
+    "dsa_mla_absorb_wgrad_workspace_size": ([_i64, _i64], _i64),
+    "dsa_mla_absorb_wgrad": ([_vp, _i64, _vp, _i64, _vp, _i32, _i32, _i64, _i64, _vp, _i64, _vp], _i32),
     "dsa_tnd_metadata": ([_vp, _i32, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp], _i32),
     # packed varlen: cu_seqlens / cmp_residual_k are host int32 arrays (ctypes arrays or None)
     "dsa_lightning_indexer_varlen": (

@@ -19,6 +19,8 @@
 //          32 k-steps stream the A rows from global memory three steps ahead.
 // Each workgroup stages its weight once and then walks token chunks; the waves share no
 // state after the staging barrier.
+#include <algorithm>
+
 #include "dsa_common.h"
 
 namespace dsa {
@@ -203,8 +205,190 @@ mla_absorb_o_kernel(const uint16_t* __restrict__ a, int64_t lda, const uint16_t*
   }
 }
 
+// Weight gradient of either product, per head h:
+//   G[i, j] = sum_t A[t, h, i] . B[t, h, j]   (A rows 128 wide, B rows 512 wide, fp32 sums)
+// written as [128, 512] (the query projection's w_uk) or transposed, [512, 128] (w_uv).
+//
+// Bound by one read of A and B (each row element is used in 512 or 128 products of its own
+// token only).  Workgroup = head x 256 of B's columns, 8 waves of 64 x 64 outputs on
+// v_mfma_f32_32x32x16_bf16; the tokens are the k dimension, so both operands are read
+// transposed (ds_read_b64_tr_b16) out of 32-token tiles that are DMA'd into three LDS buffers
+// two tiles ahead (16-byte chunk c of row r at c ^ 4 (r & 3): the four rows of a transposed read
+// take distinct banks).  The two workgroups of a head run on one XCD (head = blockIdx.x), so
+// A's second read comes from its L2.  Few heads: the tokens are split over workgroups too
+// (about 256 in all), whose fp32 partial sums wgrad_sum_kernel adds in order.
+// 4096 tokens, 128 heads: permuting copies, fp32 conversions and an fp32 library product
+// 1.73 ms -> 0.128 ms (w_uk; 5.2 TB/s of operand bytes) and 0.166 ms (w_uv, transposed stores).
+constexpr int kGTok = 32;             // tokens per tile
+constexpr int kGThreads = 512;
+constexpr int kNar = 128, kWide = 512, kGCols = 256;
+constexpr int64_t kGElems = (int64_t)kNar * kWide;
+
+template <bool kWideRows>
+__global__ void __launch_bounds__(kGThreads, 2)
+mla_absorb_wgrad_kernel(const uint16_t* __restrict__ a, int64_t lda, const uint16_t* __restrict__ b, int64_t ldb,
+                        void* __restrict__ out, int out_bf16, float* __restrict__ part, int64_t tokens, int heads,
+                        int64_t per_split) {
+  __shared__ u32x4 ta[3][kGTok * kNar / 8];
+  __shared__ u32x4 tb[3][kGTok * kGCols / 8];
+  const int h = blockIdx.x, cpart = blockIdx.y, sp = blockIdx.z;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave & 1, wn = wave >> 1;  // 64 columns of A, of B
+  const int64_t t_beg = sp * per_split, t_end = min(tokens, t_beg + per_split);
+  const int n_tiles = t_end > t_beg ? (int)((t_end - t_beg + kGTok - 1) / kGTok) : 0;
+  const uint32_t sa = (uint32_t)(heads * lda * 2), sb = (uint32_t)(heads * ldb * 2);  // bytes per token
+  auto issue = [&](int tl, int buf) {  // three instructions per wave: 4 rows of A, 2 x 2 rows of B
+    const int64_t t0 = t_beg + (int64_t)tl * kGTok;
+    const int last = (int)min<int64_t>(kGTok - 1, t_end - 1 - t0);
+    const uint16_t* ab = a + (t0 * heads + h) * lda;
+    const uint16_t* bb = b + (t0 * heads + h) * ldb + cpart * kGCols;
+    {
+      const int r = 4 * wave + (lane >> 4), c = (lane & 15) ^ (4 * (r & 3));
+      dma16_to_lds(ab, (uint32_t)min(r, last) * sa + 16u * c, (uint32_t)(uintptr_t)&ta[buf][64 * wave]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int J = wave + 8 * i, r = 2 * J + (lane >> 5), c = (lane & 31) ^ (4 * (r & 3));
+      dma16_to_lds(bb, (uint32_t)min(r, last) * sb + 16u * c, (uint32_t)(uintptr_t)&tb[buf][64 * J]);
+    }
+  };
+  // transposed operand reads (the lane pattern of the attention forward's V reads): lane group
+  // G = lane / 16 covers columns 16 (G & 1) .. +15 and token half G >> 1; source lane c
+  // supplies token 8x + 4 (G >> 1) + c / 4 and columns 4 (c % 4) .. +3
+  const int c16 = lane & 15, G = lane >> 4, n = lane & 31, half = lane >> 5;
+  uint32_t oa[2][2], ob[2][2];  // [32-column tile][x], bytes
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y) {
+      const int r = 8 * x + 4 * half + (c16 >> 2);
+      const int ca = 8 * wm + 4 * y + 2 * (G & 1) + ((c16 & 3) >> 1), cb = 8 * wn + 4 * y + 2 * (G & 1) + ((c16 & 3) >> 1);
+      oa[y][x] = r * (kNar * 2) + 16 * (ca ^ (4 * (r & 3))) + 8 * (c16 & 1);
+      ob[y][x] = r * (kGCols * 2) + 16 * (cb ^ (4 * (r & 3))) + 8 * (c16 & 1);
+    }
+  f32x16 acc[2][2];  // [A tile][B tile]
+#pragma unroll
+  for (int y = 0; y < 2; ++y)
+#pragma unroll
+    for (int z = 0; z < 2; ++z) acc[y][z] = (f32x16){0.f};
+  if (n_tiles > 0) issue(0, 0);
+  if (n_tiles > 1) issue(1, 1);
+  int buf = 0;
+  for (int tl = 0; tl < n_tiles; ++tl) {
+    if (tl + 1 < n_tiles) {
+      asm volatile("s_waitcnt vmcnt(3)" ::: "memory");  // (the next tile's three may be in flight)
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    __syncthreads();  // every wave's part landed; the buffer of the tile before is free
+    if (tl + 2 < n_tiles) issue(tl + 2, buf == 0 ? 2 : buf - 1);
+    const int valid = (int)min<int64_t>(kGTok, t_end - t_beg - (int64_t)tl * kGTok);
+    if (valid < kGTok) {  // (workgroup-uniform, the last tile) rows past the last token add nothing
+      for (int i = tid; i < (kGTok - valid) * (kNar / 8); i += kGThreads) ta[buf][valid * (kNar / 8) + i] = (u32x4){0u, 0u, 0u, 0u};
+      for (int i = tid; i < (kGTok - valid) * (kGCols / 8); i += kGThreads) tb[buf][valid * (kGCols / 8) + i] = (u32x4){0u, 0u, 0u, 0u};
+      __syncthreads();
+    }
+    const lds_char* pa = lds_bytes(&ta[buf][0]);
+    const lds_char* pb = lds_bytes(&tb[buf][0]);
+#pragma unroll
+    for (int ks = 0; ks < kGTok / 16; ++ks) {
+      u32x4 va[2], vb[2];
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        va[y] = lds_read_tr_pair(pa + oa[y][0] + ks * 16 * kNar * 2, pa + oa[y][1] + ks * 16 * kNar * 2);
+        vb[y] = lds_read_tr_pair(pb + ob[y][0] + ks * 16 * kGCols * 2, pb + ob[y][1] + ks * 16 * kGCols * 2);
+      }
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int z = 0; z < 2; ++z)
+          acc[y][z] = kWideRows ? mfma32x32x16(as_bf16x8(vb[z]), as_bf16x8(va[y]), acc[y][z])
+                                : mfma32x32x16(as_bf16x8(va[y]), as_bf16x8(vb[z]), acc[y][z]);
+    }
+    buf = buf == 2 ? 0 : buf + 1;
+  }
+  // lane holds rows 8j + 4 half + i of the first operand's tile, column n of the second's
+  float* po = part ? part + ((int64_t)sp * heads + h) * kGElems : nullptr;
+#pragma unroll
+  for (int y = 0; y < 2; ++y)
+#pragma unroll
+    for (int z = 0; z < 2; ++z)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int r = 8 * (v >> 2) + 4 * half + (v & 3);
+        const int ia = 64 * wm + 32 * y, ib = cpart * kGCols + 64 * wn + 32 * z;
+        const int64_t e = kWideRows ? (int64_t)(ib + r) * kNar + ia + n : (int64_t)(ia + r) * kWide + ib + n;
+        if (po) po[e] = acc[y][z][v];
+        else if (out_bf16) reinterpret_cast<uint16_t*>(out)[h * kGElems + e] = f_to_bf16(acc[y][z][v]);
+        else reinterpret_cast<float*>(out)[h * kGElems + e] = acc[y][z][v];
+      }
+}
+
+// out = sum of the token splits' partial sums, in order; four elements per thread
+__global__ void __launch_bounds__(256)
+wgrad_sum_kernel(const float* __restrict__ part, void* __restrict__ out, int out_bf16, int64_t n4, int splits) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  f32x4 s = reinterpret_cast<const f32x4*>(part)[i];
+  for (int k = 1; k < splits; ++k) s += reinterpret_cast<const f32x4*>(part)[k * n4 + i];
+  if (out_bf16) reinterpret_cast<uint2*>(out)[i] = make_uint2(pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]));
+  else reinterpret_cast<f32x4*>(out)[i] = s;
+}
+
+// token splits: about 256 workgroups, 256 tokens or more each (a split costs a write and a
+// read of the fp32 gradient)
+int wgrad_splits(int64_t tokens, int64_t heads) {
+  const int64_t wgs = heads * (kWide / kGCols);
+  return (int)std::max<int64_t>(1, std::min<int64_t>(256 / wgs, tokens / 256));
+}
+
 }  // namespace
 }  // namespace dsa
+
+extern "C" int64_t dsa_mla_absorb_wgrad_workspace_size(int64_t tokens, int64_t heads) {
+  if (tokens <= 0 || heads <= 0) return 0;
+  const int s = dsa::wgrad_splits(tokens, heads);
+  return s > 1 ? s * heads * dsa::kGElems * 4 : 0;
+}
+
+extern "C" int dsa_mla_absorb_wgrad(const void* a, int64_t lda, const void* b, int64_t ldb, void* out, int out_dtype,
+                                    int wide_rows, int64_t tokens, int64_t heads, void* workspace,
+                                    int64_t workspace_bytes, void* stream) {
+  using namespace dsa;
+  const char* what = "dsa_mla_absorb_wgrad";
+  if (!a || !b || !out) return set_error(DSA_ERR_INVALID_ARG, "%s: null pointer", what);
+  if (tokens < 0 || heads <= 0 || heads > 65535) return set_error(DSA_ERR_INVALID_ARG, "%s: bad sizes", what);
+  if (out_dtype != DSA_BF16 && out_dtype != DSA_F32)
+    return set_error(DSA_ERR_UNSUPPORTED, "%s: out dtype %d", what, out_dtype);
+  if (lda < kNar || ldb < kWide || lda % 8 || ldb % 8)
+    return set_error(DSA_ERR_INVALID_ARG, "%s: leading dimensions (lda %lld, ldb %lld; multiples of 8 elements)", what,
+                     (long long)lda, (long long)ldb);
+  if (heads * std::max(lda, ldb) * 2 * kGTok > (int64_t)UINT32_MAX)
+    return set_error(DSA_ERR_UNSUPPORTED, "%s: a tile of %d tokens exceeds 4 GiB", what, kGTok);
+  if (((uintptr_t)a | (uintptr_t)b | (uintptr_t)out) % 16)
+    return set_error(DSA_ERR_INVALID_ARG, "%s: operands must be 16-byte aligned", what);
+  int splits = wgrad_splits(tokens, heads);
+  if (splits > 1 && (!workspace || workspace_bytes < splits * heads * kGElems * 4 || (uintptr_t)workspace % 16)) splits = 1;
+  int64_t per = (tokens + splits - 1) / splits;
+  per = std::max<int64_t>(kGTok, (per + kGTok - 1) / kGTok * kGTok);
+  hipStream_t st = (hipStream_t)stream;
+  float* part = splits > 1 ? (float*)workspace : nullptr;
+  {
+    const TimedLaunch tl("mla_absorb_wgrad_kernel", st);
+    auto* kern = wide_rows ? mla_absorb_wgrad_kernel<true> : mla_absorb_wgrad_kernel<false>;
+    kern<<<dim3((unsigned)heads, kWide / kGCols, (unsigned)splits), kGThreads, 0, st>>>(
+        (const uint16_t*)a, lda, (const uint16_t*)b, ldb, out, out_dtype == DSA_BF16, part, tokens, (int)heads, per);
+  }
+  if (int rc = check_launch(what)) return rc;
+  if (splits > 1) {
+    const int64_t n4 = heads * kGElems / 4;
+    const TimedLaunch tl("wgrad_sum_kernel", st);
+    wgrad_sum_kernel<<<ceil_div(n4, 256), 256, 0, st>>>(part, out, out_dtype == DSA_BF16, n4, splits);
+    return check_launch(what);
+  }
+  return DSA_OK;
+}
 
 extern "C" int dsa_mla_absorb(const void* a, int64_t lda, const void* wt, void* c, int64_t ldc, const void* append,
                               int64_t ld_append, int64_t append_width, int64_t tokens, int64_t heads, int64_t k,

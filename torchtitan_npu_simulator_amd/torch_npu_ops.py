@@ -2085,6 +2085,24 @@ def mla_absorb(a, wt, *, append=None):
     return out
 
 
+def _absorb_wgrad(a, b, dtype, *, wide_rows):
+    """Per head sum_t a[t, h]^T b[t, h] (dsa_mla_absorb_wgrad): a [..., H, 128], b [..., H, 512]
+    bf16 (rows may be strided views) -> [H, 128, 512], or [H, 512, 128] with ``wide_rows``, in
+    ``dtype`` from fp32 sums."""
+    lib = load_library()
+    a, lda = _rows_view(a)
+    b, ldb = _rows_view(b)
+    H = a.shape[-2]
+    tokens = math.prod(a.shape[:-2])
+    od = torch.bfloat16 if dtype == torch.bfloat16 else torch.float32
+    d_w = torch.empty((H, 512, 128) if wide_rows else (H, 128, 512), dtype=od, device=a.device)
+    ws_bytes = int(lib.dsa_mla_absorb_wgrad_workspace_size(tokens, H))
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
+    check(lib.dsa_mla_absorb_wgrad(ptr(a), lda, ptr(b), ldb, ptr(d_w), _lib.dtype_code(od), int(wide_rows), tokens, H,
+                                   ptr(ws), ws_bytes, stream_of(a.device)), "dsa_mla_absorb_wgrad")
+    return d_w.to(dtype)
+
+
 class _AbsorbQ(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q_nope, q_pe, w_uk):
@@ -2100,7 +2118,10 @@ class _AbsorbQ(torch.autograd.Function):
         R = w_uk.shape[-1]
         dq = dq.to(torch.bfloat16)
         d_nope = mla_absorb(dq[..., :R], w_uk.to(torch.bfloat16).contiguous())  # [.., H, 128]
-        # d w_uk[h] = sum_t q_nope[t, h]^T dq[t, h, :R]: a plain batched GEMM (hipBLASLt)
+        # d w_uk[h] = sum_t q_nope[t, h]^T dq[t, h, :R]
+        if q_nope.dtype == torch.bfloat16:
+            d_w = _absorb_wgrad(q_nope, dq[..., :R], w_uk.dtype, wide_rows=False)
+            return d_nope, dq[..., R:], d_w
         H = q_nope.shape[-2]
         qn = q_nope.reshape(-1, H, q_nope.shape[-1]).permute(1, 2, 0).contiguous().float()
         dqa = dq[..., :R].reshape(-1, H, R).transpose(0, 1).contiguous().float()
@@ -2121,6 +2142,8 @@ class _AbsorbOut(torch.autograd.Function):
         out, w_uv_t = ctx.saved_tensors
         dy = dy.to(torch.bfloat16)
         d_out = mla_absorb(dy, w_uv_t.to(torch.bfloat16).contiguous())  # [.., H, 512]
+        if out.dtype == torch.bfloat16:
+            return d_out, _absorb_wgrad(dy, out, w_uv_t.dtype, wide_rows=True)
         H = out.shape[-2]
         o = out.reshape(-1, H, out.shape[-1]).permute(1, 2, 0).contiguous().float()
         g = dy.reshape(-1, H, dy.shape[-1]).transpose(0, 1).contiguous().float()
@@ -2132,7 +2155,7 @@ def mla_absorb_q(q_nope, q_pe, w_uk):
     """The absorbed query of MLA (reference PreAttention, models/deepseek_v32/model.py:520-535):
     ``cat([einsum("bshq,hqr->bshr", q_nope, w_uk), q_pe], -1)`` in one kernel.
     q_nope [B,S,H,128], q_pe [B,S,H,64], w_uk [H,128,512] bf16 -> q [B,S,H,576];
-    differentiable in all three (the weight gradient is a batched GEMM)."""
+    differentiable in all three."""
     return _AbsorbQ.apply(q_nope, q_pe, w_uk)
 
 
