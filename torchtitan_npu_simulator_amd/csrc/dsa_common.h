@@ -164,6 +164,40 @@ __device__ __forceinline__ uint32_t e4m3fn_rne(float f) {
   return sgn | (enc > 0x7eu ? 0x7fu : enc);
 }
 
+// The bytes e4m3fn_rne(v / s) of a row whose scale s is finite (so |v / s| <= 448 up to the
+// rounding of the scale, far below the 464 that rounds to NaN), from r = 1 / s rounded to
+// nearest: v / s is corrected once from its residual, which gives the correctly rounded
+// quotient (Markstein's theorem) wherever the residual does not underflow; it can only below
+// 2^-11, where the byte is a signed zero either way.  The sign is v's (a residual step turns
+// -0 into +0).  The hardware conversion rounds to nearest even as e4m3fn_rne does.  Against a
+// divide and the conversion in integer code this is a quarter of the instructions.
+__device__ __forceinline__ float row_quotient(float v, float s, float r) {
+  const float q = v * r;
+  return copysignf(fmaf(fmaf(-q, s, v), r, q), v);
+}
+__device__ __forceinline__ uint32_t e4m3_pack4(float a, float b, float c, float d) {
+  int w = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
+  w = __builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true);
+  return (uint32_t)w;
+}
+__device__ __forceinline__ void e4m3_row8(const float (&v)[8], float s, uint32_t (&w)[2]) {
+  if (s <= 3.4028235e38f) {
+    const float r = 1.0f / s;
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = row_quotient(v[e], s, r);
+    w[0] = e4m3_pack4(x[0], x[1], x[2], x[3]);
+    w[1] = e4m3_pack4(x[4], x[5], x[6], x[7]);
+  } else {  // a row with an infinity or a NaN
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      w[h] = 0u;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[h] |= e4m3fn_rne(v[4 * h + e] / s) << (8 * e);
+    }
+  }
+}
+
 // relu as one integer max on the bit pattern (negative floats, -0 included, have the sign
 // bit set and compare below 0): a float max would add a canonicalising max per operand in
 // IEEE mode.  +NaN passes through like torch.relu.

@@ -77,16 +77,14 @@ quantize_fp8_kernel(const T* __restrict__ x, uint8_t* __restrict__ q, float* __r
   for (int c = 0; c < kMaxChunks; ++c) {
     const int i0 = 8 * (l + c * G);
     if (i0 >= D) continue;
-    uint32_t b[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) b[e] = e4m3fn_rne(v[c][e] / s);
+    uint32_t w[2];
+    e4m3_row8(v[c], s, w);
     if (kVec) {
-      const uint2 w = {b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24), b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24)};
-      *reinterpret_cast<uint2*>(qr + i0) = w;
+      *reinterpret_cast<uint2*>(qr + i0) = make_uint2(w[0], w[1]);
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        if (i0 + e < D) qr[i0 + e] = (uint8_t)b[e];
+        if (i0 + e < D) qr[i0 + e] = (uint8_t)(w[e >> 2] >> (8 * (e & 3)));
     }
   }
 }
@@ -128,11 +126,9 @@ quantize_fp8_rows_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ q
     s = s < 1e-12f ? 1e-12f : s;  // (keeps NaN)
     if (row >= rows) continue;  // (uniform over the lane group)
     if (l == 0) scale[row] = s;
-    uint32_t b[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) b[e] = e4m3fn_rne(v[e] / s);
-    const uint2 o = {b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24), b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24)};
-    *reinterpret_cast<uint2*>(q + row * D + 8 * l) = o;
+    uint32_t o[2];
+    e4m3_row8(v, s, o);
+    *reinterpret_cast<uint2*>(q + row * D + 8 * l) = make_uint2(o[0], o[1]);
   }
 }
 
