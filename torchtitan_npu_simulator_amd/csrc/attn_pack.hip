@@ -144,7 +144,7 @@ pack_plan_kernel(const int32_t* __restrict__ indices, int S, int s_kv, int K, in
     const int t = i / used, w = i - t * used;
     mo[t * pk.words + w] = mk[t * pk.words + w];
   }
-  for (int j = n + tid; j < pk.cap; j += kPlanThreads) io[j] = -1;
+  for (int j = n + tid; j < 32 * used; j += kPlanThreads) io[j] = -1;
   if (tid == 0) count_out[(int64_t)b * pk.groups + grp] = n;
 }
 
@@ -161,10 +161,12 @@ pack_mass_gather_kernel(PackView pk, float* __restrict__ mass, int S, int K, int
   }
 }
 
-// One wave per key: the groups are looked at 64 at a time (one sel entry per lane), and the
-// contribution rows of those that hold the key are summed in fp32, eight rows in flight.  A
-// row is read once, non-temporally; the key has one owner, so no atomics are issued and the
-// order of the sum is fixed.  (A token-major pair list as dsa_csr.h builds it would be read
+// One workgroup per key, its four waves on a quarter of the groups each: the groups are looked
+// at 64 at a time (one sel entry per lane), and the contribution rows of those that hold the
+// key are summed in fp32, eight rows in flight; the waves' sums meet in LDS.  A row is read
+// once, non-temporally; the key has one owner, so no atomics are issued and the order of the
+// sum is fixed.  (One wave per key left the chip idle with few keys: 700 tokens, 64 heads,
+// top-1000 90 -> 44 us.)  (A token-major pair list as dsa_csr.h builds it would be read
 // and sorted at the lists' capacity, several times the union.)
 template <int kChunks>
 __global__ void __launch_bounds__(256)
@@ -172,9 +174,14 @@ pack_dkv_reduce_kernel(PackView pk, const uint16_t* __restrict__ cbuf, float* __
                        int n) {
   constexpr int kWidth = kChunks * 8;
   constexpr int kRows = 8;
-  const int k = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), b = blockIdx.y;
-  const int lane = threadIdx.x & 63;
-  if (k >= s_kv) return;
+  __shared__ float sums[3][kWidth];  // waves 1..3
+  __shared__ int held;
+  const int k = blockIdx.x, b = blockIdx.y;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (threadIdx.x == 0) held = 0;
+  __syncthreads();
+  // (whole steps of 64 groups per wave)
+  const int per = ((n + 3) / 4 + 63) / 64 * 64, n0 = min(n, wave * per), n1 = min(n, n0 + per);
   const uint2* sel = pk.sel + ((int64_t)b * pk.key_words + (k >> 5)) * pk.groups + g0;
   const uint32_t bit = 1u << (k & 31);
   const uint16_t* cb = cbuf + (int64_t)b * n * pk.cap * kWidth;
@@ -188,8 +195,8 @@ pack_dkv_reduce_kernel(PackView pk, const uint16_t* __restrict__ cbuf, float* __
     }
   };
   bool any = false;
-  for (int gb = 0; gb < n; gb += 64) {
-    const uint2 e = gb + lane < n ? sel[gb + lane] : make_uint2(0u, 0u);
+  for (int gb = n0; gb < n1; gb += 64) {
+    const uint2 e = gb + lane < n1 ? sel[gb + lane] : make_uint2(0u, 0u);
     const int slot = (int)(e.y & ~kRepeats) + __popc(e.x & (bit - 1u));
     uint64_t m = __ballot((e.x & bit) != 0u);
     any |= m != 0;
@@ -228,7 +235,24 @@ pack_dkv_reduce_kernel(PackView pk, const uint16_t* __restrict__ cbuf, float* __
         }
     }
   }
-  if (!any) return;
+  if (any && lane == 0) held = 1;
+  if (wave > 0) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) sums[wave - 1][8 * lane + r] = acc[r];
+    if constexpr (kChunks == 72)
+      if (lane < 8)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) sums[wave - 1][512 + 8 * lane + r] = acc2[r];
+  }
+  __syncthreads();
+  if (wave > 0 || !held) return;
+#pragma unroll
+  for (int u = 0; u < 3; ++u)
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      acc[r] += sums[u][8 * lane + r];
+      if constexpr (kChunks == 72) acc2[r] += sums[u][512 + 8 * (lane & 7) + r];
+    }
   float* d = acc_out + ((int64_t)b * s_kv + k) * kWidth;
   auto put = [](float* p, const float (&a)[8]) {
     float4* d4 = reinterpret_cast<float4*>(p);
@@ -312,7 +336,7 @@ int pack_plan_build(const int32_t* indices, int64_t batch, int64_t s_q, int64_t 
 
 int pack_dkv_reduce(const PackView& view, const uint16_t* cbuf, float* acc, int64_t batch, int64_t s_kv, int64_t width,
                     int64_t g0, int64_t n, hipStream_t st) {
-  const dim3 grid(ceil_div(s_kv, 4), (unsigned)batch);
+  const dim3 grid((unsigned)s_kv, (unsigned)batch);
   const TimedLaunch tl(width == 576 ? "pack_dkv_reduce_kernel<72>" : "pack_dkv_reduce_kernel<64>", st);
   if (width == 576)
     pack_dkv_reduce_kernel<72><<<grid, 256, 0, st>>>(view, cbuf, acc, (int)s_kv, (int)g0, (int)n);

@@ -23,16 +23,31 @@
 namespace dsa {
 namespace {
 
-constexpr int kCsrRowsMin = 16;   // query rows per counting workgroup: at least
+constexpr int kCsrRowsMin = 16;   // query rows per counting workgroup: at least (many rows)
+constexpr int kCsrRowsLow = 4;    // (few rows)
 constexpr int kCsrRowsMax = 512;  // and at most
 constexpr int kCsrRowBatch = 8;   // index rows loaded together
 constexpr int kLdsKeys = 16384;  // keys privatised in LDS
 constexpr int kColChunk = 32;    // row blocks per chunk of the count table's column scan
 
-// query rows per counting workgroup: about four pairs per key of a range
-inline int csr_rows_per_wg(int64_t s_kv, int64_t K) {
-  const int64_t want = 4 * s_kv / (K > 0 ? K : 1);
-  return (int)(want < kCsrRowsMin ? kCsrRowsMin : want > kCsrRowsMax ? kCsrRowsMax : want);
+// query rows per counting workgroup: about four pairs per key of a range; fewer (down to one
+// pair per key, so that the table stays within four times the pair list) where the rows
+// would not fill the chip with workgroups
+inline int csr_rows_per_wg(int64_t s_kv, int64_t K, int64_t rows) {
+  const int64_t k = K > 0 ? K : 1;
+  int64_t want = 4 * s_kv / k;
+  want = want < kCsrRowsMin ? kCsrRowsMin : want > kCsrRowsMax ? kCsrRowsMax : want;
+  int64_t low = s_kv / k;
+  low = low < kCsrRowsLow ? kCsrRowsLow : low;
+  const int64_t fill = (rows + 255) / 256;
+  const int64_t r = fill > low ? fill : low;
+  return (int)(r < want ? r : want);
+}
+// the most row blocks of any chunk of at most `rows` rows (a last chunk may be cut finer)
+inline int64_t csr_row_blocks_max(int64_t s_kv, int64_t K, int64_t rows) {
+  const int64_t per = csr_rows_per_wg(s_kv, K, rows), one = csr_rows_per_wg(s_kv, K, 1);
+  const int64_t n = (rows + per - 1) / per, few = (rows + one - 1) / one;
+  return n > 256 ? n : few < 256 ? (few > n ? few : n) : 256;
 }
 
 __device__ __forceinline__ bool csr_slot_ok(int v, int s_kv, int64_t limit) {
@@ -159,6 +174,11 @@ constexpr int kFillKeys = 3584;
 constexpr int kFillRangesMax = 4;
 constexpr int kFillRB = 4;          // count-pass row blocks per fill workgroup
 constexpr int kFillThreads = 512;
+// A fill workgroup walks its rows one after another (two barriers per row): the staged fill is
+// taken where it has a workgroup for every CU.  Staged against unstaged: 300 rows of top-256
+// 100 and 6.4 us, 1000 rows of top-512 120 and 9 us, 4096 rows of 1152 slots over 5120 keys
+// 111 and 38 us; 8192 rows of top-2048 222 and 208 us at a fifth of the bytes written.
+constexpr int kFillStagedMin = 256;
 
 template <bool kVec>
 __global__ void __launch_bounds__(kFillThreads)
@@ -386,9 +406,9 @@ __global__ void __launch_bounds__(1024) csr_scan_kernel(const int* __restrict__ 
 }
 
 // acc[key] += sum over the key's pairs of bf16 contribution rows of kChunks 16-byte chunks.
-// The key-sorted pair list is cut into segments of kSegPairs pairs, one wave each, so a
+// The key-sorted pair list is cut into segments of 32 to 256 pairs, one wave each, so a
 // key selected by thousands of rows (the causal prefix) is summed by many waves instead of
-// one; seg_key[s] names the key holding pair s * kSegPairs.  A wave walks its segment in
+// one; seg_key[s] names the key holding pair s << seg_shift.  A wave walks its segment in
 // groups of 8 pairs (indices through scalar loads, all 8 rows loaded before any is summed)
 // and flushes its partial sum whenever the key changes: with a plain read-add-write if the
 // key lies wholly inside the segment (sole owner), else into the segment's partial-sum slot
@@ -401,7 +421,22 @@ __global__ void __launch_bounds__(1024) csr_scan_kernel(const int* __restrict__ 
 // chunks): lane l owns chunk l.  128-wide rows
 // (16 chunks): lanes 16s .. 16s+15 own the row of pair 4g + s of each group of 4 (four
 // streams), combined with two lane exchanges at the flush.
-constexpr int kSegPairs = 256;
+// pairs per wave: 256, fewer where those would not fill the chip (a segment costs two partial
+// rows).  150 rows of top-256: the reduction of 576-wide rows 57 us on 150 segments of 256
+// pairs, 12 us on 1200 of 32; 1500 rows of top-1024, 128-wide: 67 us of 256, 56 us of 64.
+inline int csr_seg_shift(int64_t rows, int64_t K) {
+  const int64_t pairs = rows * K;
+  return pairs >= (1 << 22) ? 8 : pairs >= (1 << 21) ? 7 : pairs >= (1 << 20) ? 6 : 5;
+}
+inline int64_t csr_segments(int64_t rows, int64_t K) {
+  const int sh = csr_seg_shift(rows, K);
+  return (rows * K + (1 << sh) - 1) >> sh;
+}
+// the most segments of any chunk of at most `rows` rows
+inline int64_t csr_segments_max(int64_t rows, int64_t K) {
+  const int64_t n = csr_segments(rows, K), few = (rows * K + 31) / 32;
+  return n > 32768 ? n : few < 32768 ? few : 32768;
+}
 
 __device__ __forceinline__ void add_bf16x8(float (&acc)[8], const u32x4& v) {
 #pragma unroll
@@ -425,12 +460,13 @@ __device__ __forceinline__ void flush8(float* d, float (&acc)[8], bool sole) {
   for (int r = 0; r < 8; ++r) acc[r] = 0.f;
 }
 
-// seg_key[s] = the key k with row_ptr[k] <= s * kSegPairs < row_ptr[k + 1]
+// seg_key[s] = the key k with row_ptr[k] <= s << seg_shift < row_ptr[k + 1]
 __global__ void __launch_bounds__(256)
-csr_seg_key_kernel(const int* __restrict__ row_ptr, int* __restrict__ seg_key, int s_kv) {
+csr_seg_key_kernel(const int* __restrict__ row_ptr, int* __restrict__ seg_key, int s_kv, int seg_shift) {
   const int k = blockIdx.x * 256 + threadIdx.x;
   if (k >= s_kv) return;
-  const int s0 = (row_ptr[k] + kSegPairs - 1) / kSegPairs, s1 = (row_ptr[k + 1] + kSegPairs - 1) / kSegPairs;
+  const int up = (1 << seg_shift) - 1;
+  const int s0 = (row_ptr[k] + up) >> seg_shift, s1 = (row_ptr[k + 1] + up) >> seg_shift;
   for (int s = s0; s < s1; ++s) seg_key[s] = k;
 }
 
@@ -438,16 +474,16 @@ template <int kChunks>
 __global__ void __launch_bounds__(256)
 dkv_reduce_kernel(const uint16_t* __restrict__ cbuf, const int* __restrict__ row_ptr, const int* __restrict__ pairs,
                   const int* __restrict__ seg_key, float* __restrict__ acc_out, float* __restrict__ part, int s_kv,
-                  int rows, int K, int b) {
+                  int rows, int K, int b, int seg_shift) {
   static_assert(kChunks == 72 || kChunks == 64 || kChunks == 16, "row widths of the attention and indexer reductions");
   constexpr int kWidth = kChunks * 8;
   constexpr int kGroup = kChunks == 16 ? 16 : 8;  // pairs per load group (16-chunk rows: four per load)
   const int seg = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int n_pairs = row_ptr[s_kv];
-  const int seg0 = seg * kSegPairs;
+  const int seg0 = seg << seg_shift;
   if (seg0 >= n_pairs) return;
-  const int seg1 = min(seg0 + kSegPairs, n_pairs);
+  const int seg1 = min(seg0 + (1 << seg_shift), n_pairs);
   const uint16_t* cb = cbuf + (int64_t)b * rows * K * kWidth;
   float* dbase = acc_out + (int64_t)b * s_kv * kWidth;
   int k = seg_key[seg];
@@ -523,13 +559,14 @@ dkv_reduce_kernel(const uint16_t* __restrict__ cbuf, const int* __restrict__ row
 template <int kWidth>
 __global__ void __launch_bounds__(256)
 csr_partial_fixup_kernel(const int* __restrict__ row_ptr, const int* __restrict__ seg_key,
-                         const float* __restrict__ part, float* __restrict__ acc_out, int s_kv, int b) {
+                         const float* __restrict__ part, float* __restrict__ acc_out, int s_kv, int b,
+                         int seg_shift) {
   const int k = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (k >= s_kv) return;
   const int kbeg = row_ptr[k], kend = row_ptr[k + 1];
   if (kend <= kbeg) return;
-  const int s0 = kbeg / kSegPairs, s1 = (kend - 1) / kSegPairs;
+  const int s0 = kbeg >> seg_shift, s1 = (kend - 1) >> seg_shift;
   if (s0 == s1) return;  // inside one segment: its owner added it
   constexpr int kPer = kWidth / 64;
   float acc[kPer];
@@ -546,17 +583,17 @@ csr_partial_fixup_kernel(const int* __restrict__ row_ptr, const int* __restrict_
 }
 
 // Bytes of the CSR workspace csr_reduce needs for contribution rows of `width` floats:
-// counts and row_ptr (s_kv + 1 ints each), the segment table (one int per kSegPairs pairs
+// counts and row_ptr (s_kv + 1 ints each), the segment table (one int per segment
 // of the chunk), the [row block][key] count table, the [column chunk][key] chunk offsets
 // and two partial-sum rows per segment (at a 16-byte boundary).
 inline int64_t csr_ws_ints(int64_t s_kv, int64_t rows, int64_t K) {
-  const int64_t n_rb = (rows + csr_rows_per_wg(s_kv, K) - 1) / csr_rows_per_wg(s_kv, K);
+  const int64_t n_rb = csr_row_blocks_max(s_kv, K, rows);
   const int64_t n_chunks = (n_rb + kColChunk - 1) / kColChunk;
-  const int64_t n_seg = (rows * K + kSegPairs - 1) / kSegPairs;
+  const int64_t n_seg = csr_segments_max(rows, K);
   return (2 * (s_kv + 1) + n_seg + (n_rb + n_chunks) * s_kv + 3) / 4 * 4 + 4;  // (+4: the fill's dup flag last)
 }
 inline int64_t csr_part_bytes(int64_t rows, int64_t K, int64_t width) {
-  return (rows * K + kSegPairs - 1) / kSegPairs * 2 * width * 4;
+  return csr_segments_max(rows, K) * 2 * width * 4;
 }
 inline int64_t csr_ws_bytes(int64_t s_kv, int64_t rows, int64_t K, int64_t width) {
   return csr_ws_ints(s_kv, rows, K) * 4 + csr_part_bytes(rows, K, width);
@@ -573,13 +610,13 @@ struct CsrView {
 // rows * K ints, csr_ws csr_ws_ints(s_kv, rows, K) ints.
 inline int csr_build(const int32_t* idx, int* pairs, int* csr_ws, int S, int s_kv, int K, int64_t q_offset, int row0,
                      int rows, int b, hipStream_t st, CsrView* view) {
-  const int rows_per_wg = csr_rows_per_wg(s_kv, K);
+  const int rows_per_wg = csr_rows_per_wg(s_kv, K, rows);
   const int64_t n_rb = ceil_div(rows, rows_per_wg);
   const int64_t n_chunks = ceil_div(n_rb, kColChunk);
   int* counts = csr_ws;
   int* row_ptr = counts + (s_kv + 1);
   int* seg_key = row_ptr + (s_kv + 1);
-  const int64_t n_seg = ceil_div((int64_t)rows * K, kSegPairs);
+  const int64_t n_seg = csr_segments(rows, K);
   int* table = seg_key + n_seg;
   int* chunk_off = table + n_rb * s_kv;
   const int n_ranges = (int)ceil_div(s_kv, kLdsKeys);
@@ -590,7 +627,7 @@ inline int csr_build(const int32_t* idx, int* pairs, int* csr_ws, int S, int s_k
   const int64_t row_base = (int64_t)b * S + row0;  // int4 loads need 16-byte aligned index rows
   const bool vec = K % 4 == 0 && ((uintptr_t)(idx + row_base * K) % 16) == 0;
   const int n_franges = (int)ceil_div(s_kv, kFillKeys);
-  const bool staged = n_franges <= kFillRangesMax;
+  const bool staged = n_franges <= kFillRangesMax && n_franges * ceil_div(n_rb, kFillRB) >= kFillStagedMin;
   int* dup_flag = staged ? csr_ws + csr_ws_ints(s_kv, rows, K) - 1 : nullptr;
   launch_csr_count<false>(vec, (unsigned)cgrid, hist_bytes, st, idx, table, nullptr, nullptr, pairs, S, s_kv, K,
                           q_offset, row0, rows, b, n_ranges, rows_per_wg, dup_flag);
@@ -629,7 +666,7 @@ inline int csr_build(const int32_t* idx, int* pairs, int* csr_ws, int S, int s_k
   }
   {
     const TimedLaunch tl("csr_seg_key_kernel", st);
-    csr_seg_key_kernel<<<ceil_div(s_kv, 256), 256, 0, st>>>(row_ptr, seg_key, s_kv);
+    csr_seg_key_kernel<<<ceil_div(s_kv, 256), 256, 0, st>>>(row_ptr, seg_key, s_kv, csr_seg_shift(rows, K));
   }
   view->pairs = pairs;
   view->row_ptr = row_ptr;
@@ -641,17 +678,18 @@ inline int csr_build(const int32_t* idx, int* pairs, int* csr_ws, int S, int s_k
 // covers into acc_out[b][key][...]; `part` holds csr_part_bytes(rows, K, 8 * row_chunks).
 inline int csr_reduce_built(const CsrView& v, const uint16_t* cbuf, float* acc_out, float* part, int s_kv, int rows,
                             int K, int b, int row_chunks, hipStream_t st) {
-  const unsigned rgrid = ceil_div(ceil_div((int64_t)rows * K, kSegPairs), 4);
+  const int sh = csr_seg_shift(rows, K);
+  const unsigned rgrid = ceil_div(csr_segments(rows, K), 4);
   const TimedLaunch tl(row_chunks == 72   ? "dkv_reduce_kernel<72>"
                        : row_chunks == 64 ? "dkv_reduce_kernel<64>"
                                           : "dkv_reduce_kernel<16>",
                        st);
   if (row_chunks == 72)
-    dkv_reduce_kernel<72><<<rgrid, 256, 0, st>>>(cbuf, v.row_ptr, v.pairs, v.seg_key, acc_out, part, s_kv, rows, K, b);
+    dkv_reduce_kernel<72><<<rgrid, 256, 0, st>>>(cbuf, v.row_ptr, v.pairs, v.seg_key, acc_out, part, s_kv, rows, K, b, sh);
   else if (row_chunks == 64)
-    dkv_reduce_kernel<64><<<rgrid, 256, 0, st>>>(cbuf, v.row_ptr, v.pairs, v.seg_key, acc_out, part, s_kv, rows, K, b);
+    dkv_reduce_kernel<64><<<rgrid, 256, 0, st>>>(cbuf, v.row_ptr, v.pairs, v.seg_key, acc_out, part, s_kv, rows, K, b, sh);
   else if (row_chunks == 16)
-    dkv_reduce_kernel<16><<<rgrid, 256, 0, st>>>(cbuf, v.row_ptr, v.pairs, v.seg_key, acc_out, part, s_kv, rows, K, b);
+    dkv_reduce_kernel<16><<<rgrid, 256, 0, st>>>(cbuf, v.row_ptr, v.pairs, v.seg_key, acc_out, part, s_kv, rows, K, b, sh);
   else
     return set_error(DSA_ERR_UNSUPPORTED, "csr_reduce: row width %d chunks", row_chunks);
   if (int rc = check_launch("csr_reduce")) return rc;
@@ -659,11 +697,11 @@ inline int csr_reduce_built(const CsrView& v, const uint16_t* cbuf, float* acc_o
     const TimedLaunch tl2("csr_partial_fixup_kernel", st);
     const unsigned fgrid = (unsigned)ceil_div(s_kv, 4);
     if (row_chunks == 72)
-      csr_partial_fixup_kernel<576><<<fgrid, 256, 0, st>>>(v.row_ptr, v.seg_key, part, acc_out, s_kv, b);
+      csr_partial_fixup_kernel<576><<<fgrid, 256, 0, st>>>(v.row_ptr, v.seg_key, part, acc_out, s_kv, b, sh);
     else if (row_chunks == 64)
-      csr_partial_fixup_kernel<512><<<fgrid, 256, 0, st>>>(v.row_ptr, v.seg_key, part, acc_out, s_kv, b);
+      csr_partial_fixup_kernel<512><<<fgrid, 256, 0, st>>>(v.row_ptr, v.seg_key, part, acc_out, s_kv, b, sh);
     else
-      csr_partial_fixup_kernel<128><<<fgrid, 256, 0, st>>>(v.row_ptr, v.seg_key, part, acc_out, s_kv, b);
+      csr_partial_fixup_kernel<128><<<fgrid, 256, 0, st>>>(v.row_ptr, v.seg_key, part, acc_out, s_kv, b, sh);
   }
   return check_launch("csr_reduce(fix-up)");
 }
