@@ -414,6 +414,14 @@ int dsa_quantize_fp8_rows(const void* x, int in_dtype, uint8_t* q, float* scale,
                           void* stream);
 
 /*
+ * Slot indices [batch, s, window + n_sel] of the V4 shared-KV attention over the rows of
+ * cat(ori_kv [s], cmp_kv): tokens row - win_left .. row - win_left + window - 1 inside [0, s),
+ * then cmp_indices [batch, s, n_sel] as given or, with NULL, compressed row c at s + c for
+ * c < (row + 1) / cmp_ratio; -1 = empty (models/deepseek_v4/model.py:467-488).
+ */
+int dsa_v4_indices(const int32_t* cmp_indices, int32_t* out, int64_t batch, int64_t s, int64_t win_left,
+                   int64_t window, int64_t cmp_ratio, int64_t n_sel, void* stream);
+/*
  * Attention sink (DeepSeek-V4): a per-head logit with no value in every row's softmax.
  * dsa_attn_sink_fold, after dsa_sparse_mla_fwd over the row's keys: with m, l the row's
  * softmax_max / softmax_sum, m2 = max(m, sink[h]), a = l e^(m - m2), s2 = a + e^(sink - m2);

@@ -39,6 +39,7 @@ _SIGNATURES = {
     "dsa_indexer_fwd_noalloc": ([_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                  _vp], _i32),
     "dsa_quantize_fp8_rows": ([_vp, _i32, _vp, _vp, _i64, _i64, _vp], _i32),
+    "dsa_v4_indices": ([_vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp], _i32),
     "dsa_attn_sink_fold": ([_vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64, _vp], _i32),
     "dsa_attn_sink_grad": ([_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64, _vp], _i32),
     "dsa_topk": ([_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp], _i32),

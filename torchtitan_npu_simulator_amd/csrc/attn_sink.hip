@@ -150,3 +150,45 @@ extern "C" int dsa_attn_sink_grad(const void* out, const void* dout, const float
                                                        softmax_sum, sinks, dsink, rows, (int)n_heads, (int)d_v);
   return check_launch("dsa_attn_sink_grad");
 }
+
+// Slot indices of DeepSeek-V4's shared-KV attention over the rows of cat(ori_kv [S],
+// cmp_kv [n_cmp]) (SparseAttention.forward, models/deepseek_v4/model.py:467-488): the window
+// tokens s - win_left .. s + win_right, then the selected compressed rows as given or, with
+// none given, every causal one (c < (s + 1) / ratio, at row S + c); -1 = empty.  One
+// workgroup per token.  (A dozen elementwise launches on int64 tensors made them before:
+// 60 us of a 0.45 ms step at 1024 tokens.)
+namespace dsa {
+namespace {
+__global__ void __launch_bounds__(256)
+v4_indices_kernel(const int32_t* __restrict__ cmp, int32_t* __restrict__ out, int S, int win_left, int W, int ratio,
+                  int n_sel) {
+  const int s = blockIdx.x, b = blockIdx.y;
+  const int64_t row = (int64_t)b * S + s;
+  int32_t* o = out + row * (W + n_sel);
+  for (int j = threadIdx.x; j < W + n_sel; j += 256) {
+    int v;
+    if (j < W) {
+      const int64_t t = (int64_t)s - win_left + j;
+      v = t >= 0 && t < S ? (int)t : -1;
+    } else {
+      const int c = j - W;
+      v = cmp ? cmp[row * n_sel + c] : (c < (s + 1) / ratio ? c + S : -1);
+    }
+    o[j] = v;
+  }
+}
+}  // namespace
+}  // namespace dsa
+
+extern "C" int dsa_v4_indices(const int32_t* cmp_indices, int32_t* out, int64_t batch, int64_t s, int64_t win_left,
+                              int64_t window, int64_t cmp_ratio, int64_t n_sel, void* stream) {
+  using namespace dsa;
+  if (!out) return set_error(DSA_ERR_INVALID_ARG, "dsa_v4_indices: null pointer");
+  if (batch <= 0 || s <= 0 || window < 0 || n_sel < 0 || window + n_sel <= 0 || cmp_ratio <= 0 || batch > 65535 ||
+      s > INT32_MAX || window + n_sel > INT32_MAX || cmp_ratio > INT32_MAX || win_left > INT32_MAX || win_left < INT32_MIN)
+    return set_error(DSA_ERR_INVALID_ARG, "dsa_v4_indices: bad sizes");
+  const TimedLaunch tl("v4_indices_kernel", (hipStream_t)stream);
+  v4_indices_kernel<<<dim3((unsigned)s, (unsigned)batch), 256, 0, (hipStream_t)stream>>>(
+      cmp_indices, out, (int)s, (int)win_left, (int)window, (int)cmp_ratio, (int)n_sel);
+  return check_launch("dsa_v4_indices");
+}

@@ -4,9 +4,9 @@
 // per clock), far too slow for the dKV scatter-add (576 fp32 per (token, key) pair), so
 // the backward reduces dKV through a key-major pass instead:
 //
-//   (delta) delta = rowsum(dO o O) per (token, head): formed by bwd_sdp_kernel from the O
-//           rows it reads beside dO, or, with a per-head sink (whose gradient needs it for
-//           every row), by bwd_delta_kernel in one streaming pass; the same fp32 sum either way.
+//   (delta) delta = rowsum(dO o O) per (token, head) is formed by bwd_sdp_kernel from the O
+//           rows it reads beside dO; with a per-head sink it also leaves each row's part of
+//           the sink's gradient, -p_sink delta, which sink_colsum_kernel sums per head.
 //   (alpha) bwd_sdp_kernel, workgroup = token x 128 heads, 8 waves x 16 heads (the
 //           forward's gather pipeline): S^T = K Q^T and dP^T = V dO^T on
 //           v_mfma_f32_16x16x32_bf16 chains sharing every K operand read, P = exp2(S*scale*
@@ -74,17 +74,19 @@ __device__ __forceinline__ int g2_swz(int r) { return (r >> 1) & 7; }
 
 constexpr int kSdpWaves = 8;
 
-// kD: row width of Q and KV, 576 (latent + rope) or 512 (no rope).  kOwnDelta: delta =
-// rowsum(dO o O) of each head is formed here from O (read beside dO, in dO's lane layout,
-// then summed over the head's four lane groups) instead of read from dbuf.  kPack: the
+// kD: row width of Q and KV, 576 (latent + rope) or 512 (no rope).  delta = rowsum(dO o O) of
+// each head is formed here from O (read beside dO, in dO's lane layout, then summed over the
+// head's four lane groups); with sinks, pd[row][head] = -e^(sink - m2) / s2 delta from the row
+// statistics, which include the sink.  (A separate streaming pass over O and dO for the sink's
+// gradient cost 0.197 ms of a 4.32 ms step at S = 4096, 128 heads x 512.)  kPack: the
 // workgroup is a group of packed tokens (attn_pack.h): "heads" are its (token, head) rows,
 // 16 per wave and so of one token, whose mask words give the wave's validity bits (scalar
 // loads, one block ahead), and the mass is summed per token into pk.mass by slot.
-template <int kD, bool kOwnDelta, bool kPack>
+template <int kD, bool kPack>
 __global__ void __launch_bounds__(64 * kSdpWaves, 1)
 bwd_sdp_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, const int32_t* __restrict__ idx,
                 const uint16_t* __restrict__ dout, const uint16_t* __restrict__ out, const float* __restrict__ smax,
-                const float* __restrict__ ssum, const float* __restrict__ dbuf, uint16_t* __restrict__ gbuf,
+                const float* __restrict__ ssum, const float* __restrict__ sinks, float* __restrict__ pd, uint16_t* __restrict__ gbuf,
                 float* __restrict__ mass, int S, int s_kv, int H, int K, float scale, int64_t q_offset, int row0,
                 PackView pk) {
   constexpr int kW = kSdpWaves;
@@ -138,7 +140,7 @@ bwd_sdp_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, 
   // latent Q and dO of head hl: k-step s holds columns 32s + 8g .. +8; lane group g also
   // loads rope chunks 2g, 2g + 1 for the LDS copy (step kLat + j reads chunk 4j + g)
   u32x4 qb[kLat], db[kLat], qr[2];
-  u32x4 ob[kOwnDelta ? kLat : 1];  // O in dO's layout (kOwnDelta)
+  u32x4 ob[kLat];  // O in dO's layout
   {
     const u32x4* qh = reinterpret_cast<const u32x4*>(q + hrow * kD);
     const u32x4* dh = reinterpret_cast<const u32x4*>(dout + hrow * kDv);
@@ -148,26 +150,21 @@ bwd_sdp_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, 
     for (int st = 0; st < kLat; ++st) db[st] = dh[4 * st + g];
 #pragma unroll
     for (int j = 0; j < 2; ++j) qr[j] = kRope ? qh[64 + 2 * g + j] : (u32x4){0u, 0u, 0u, 0u};
-    if constexpr (kOwnDelta) {
-      const u32x4* oh = reinterpret_cast<const u32x4*>(out + hrow * kDv);
+    const u32x4* oh = reinterpret_cast<const u32x4*>(out + hrow * kDv);
 #pragma unroll
-      for (int st = 0; st < kLat; ++st) ob[st] = oh[4 * st + g];
-    }
+    for (int st = 0; st < kLat; ++st) ob[st] = oh[4 * st + g];
   }
   const float mx = smax[hrow], sm = ssum[hrow];
-  float dlt;
-  if constexpr (!kOwnDelta) {
-    if constexpr (kPack) {  // (delta rows of the chunk's tokens, from the chunk's first)
-      const int t0 = row0 * pk.tt, nt = min((int)gridDim.x * pk.tt, S - t0);
-      dlt = dbuf[((int64_t)b * nt + (tok - t0)) * H + (hok ? head : 0)];
-    } else {
-      dlt = dbuf[((int64_t)b * gridDim.x + lr) * H + (hok ? hl : 0)];
-    }
-  }
+  // the row's place among the chunk's tokens, for the sink's gradient
+  auto pd_row = [&]() -> float* {
+    const int t0 = kPack ? row0 * pk.tt : row0, nt = kPack ? min((int)gridDim.x * pk.tt, S - t0) : (int)gridDim.x;
+    return pd + ((int64_t)b * nt + (tok - t0)) * H + head;
+  };
   const int nblk = kPack ? (pk.count[pgrp] + kBN - 1) / kBN : count_row_blocks(ridx, K, s_kv, limit, vidx, &sh_last);
   if (!kPack && mrow)  // slots past the last usable block carry no mass
     for (int j = nblk * kBN + tid; j < K; j += 64 * kW) mrow[j] = 0.f;
   if (nblk == 0) {
+    if (sinks && hok && g == 0) *pd_row() = 0.f;  // (O = 0)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the ring DMA has landed before the LDS is released
     return;
   }
@@ -186,12 +183,10 @@ bwd_sdp_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, 
     }
   }
   const float lse2 = (hok && sm > 0.f) ? (mx + logf(sm)) * kLog2e : INFINITY;  // +inf -> P = 0
-  if constexpr (kOwnDelta) {
-    // The same fp32 sum as bwd_delta_kernel, bit for bit (so results do not depend on which
-    // of the two formed delta): its lane l of a head sums 16-byte chunks l + 16 j (j = 0..3,
-    // in order), which this lane group g holds for l = 4a + g as chunks 4 (a + 4j) + g; its
-    // xor tree over l (8, 4, 2, 1) is a's two bits here, then g's across the lanes 32 and 16
-    // apart (each step adds a value and its partner's, which commutes)
+  // four partial sums (chunks 4 (a + 4j) + g of O and dO, j = 0..3 in order), then the tree over a
+  // and the lane groups
+  float dlt;
+  {
     static_assert(kLat == 16, "four chunks per lane of the delta pass");
     float sa[4];
 #pragma unroll
@@ -208,6 +203,7 @@ bwd_sdp_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, 
     dlt = xor16_sum(xor32_sum((sa[0] + sa[2]) + (sa[1] + sa[3])));
   }
   const float delta = hok ? dlt : 0.f;
+  if (sinks && hok && g == 0) *pd_row() = -(expf(sinks[head] - mx) / sm) * delta;
   const float scale_log2 = scale * kLog2e;
   // landed before any DMA; held in AGPRs, which the MFMAs read directly as B operands
 #pragma unroll
@@ -1012,44 +1008,6 @@ bwd_exact_f32_kernel(const float* __restrict__ q, const float* __restrict__ kv, 
   }
 }
 
-// delta[b][lr][h] = sum_d dO[row, h, d] * O[row, h, d] (fp32) for the chunk's rows: one
-// 16-lane group per (row, head), 32 columns per lane (four 16-byte loads of each tensor).
-// With a per-head sink it also writes pd[b][lr][h] = -p_sink delta, p_sink = e^(sink - m2) /
-// s2 from the row statistics (which include the sink): the sink's gradient summed over rows.
-__global__ void __launch_bounds__(256)
-bwd_delta_kernel(const uint16_t* __restrict__ out, const uint16_t* __restrict__ dout, float* __restrict__ delta,
-                 int64_t n, int S, int H, int row0, int rows, const float* __restrict__ sinks,
-                 const float* __restrict__ smax, const float* __restrict__ ssum, float* __restrict__ pd) {
-  const int64_t grp = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 4;  // (b, lr, h) flattened, n of them
-  const int l = threadIdx.x & 15;
-  const int64_t g = grp < n ? grp : n - 1;
-  const int64_t b = g / ((int64_t)rows * H), rem = g - b * rows * H;
-  const int64_t hr = (b * S + row0 + rem / H) * H + rem % H;
-  const u32x4* o4 = reinterpret_cast<const u32x4*>(out + hr * kDv);
-  const u32x4* d4 = reinterpret_cast<const u32x4*>(dout + hr * kDv);
-  u32x4 ov[4], dv[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    ov[c] = o4[l + 16 * c];
-    dv[c] = d4[l + 16 * c];
-  }
-  float part = 0.f;
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      part += bf16_lo(dv[c][r]) * bf16_lo(ov[c][r]) + bf16_hi(dv[c][r]) * bf16_hi(ov[c][r]);
-#pragma unroll
-  for (int m = 8; m >= 1; m >>= 1) part += __shfl_xor(part, m, 64);
-  if (l == 0 && grp < n) {
-    delta[g] = part;
-    if (sinks) {
-      const float ps = expf(sinks[rem % H] - smax[hr]) / ssum[hr];
-      pd[g] = -ps * part;
-    }
-  }
-}
-
 // dsink[h] += sum over the chunk's rows of pd[row][h]: one workgroup per head
 __global__ void __launch_bounds__(256)
 sink_colsum_kernel(const float* __restrict__ pd, int64_t nrows, int H, float* __restrict__ dsink) {
@@ -1068,15 +1026,15 @@ sink_colsum_kernel(const float* __restrict__ pd, int64_t nrows, int H, float* __
 
 struct BwdPlan {
   int64_t rows;  // query rows per chunk
-  int64_t g_bytes, c_bytes, pairs_bytes, csr_bytes, delta_bytes, total;  // (delta twice: delta and the sink part)
+  int64_t g_bytes, c_bytes, pairs_bytes, csr_bytes, delta_bytes, total;  // delta_bytes: the sink's parts
 };
 
 // Scratch per chunk: G and C (bf16, C rows `width` columns), the CSR pair list and
-// offsets, and delta (fp32 per row and head).
+// offsets, and the sink's gradient parts (fp32 per row and head).
 BwdPlan plan_bwd(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int64_t budget, int64_t width) {
   BwdPlan p{};
   const int64_t per_row = batch * g_slots(topk) * kGW * 2 + batch * topk * (int64_t)(width * 2 + 4) +
-                          2 * batch * kHeadsMax * 4 + topk * width / 32;  // (last: CSR segment partials)
+                          batch * kHeadsMax * 4 + topk * width / 32;  // (last: CSR segment partials)
   int64_t rows = s_q;
   if (budget > 0) rows = std::max<int64_t>(1, std::min<int64_t>(s_q, budget / per_row));
   p.rows = rows;
@@ -1086,14 +1044,14 @@ BwdPlan plan_bwd(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int64_t
   p.csr_bytes = csr_ws_bytes(s_kv, rows, topk, width);
   p.delta_bytes = batch * rows * kHeadsMax * 4;
   auto al = [](int64_t x) { return (x + 255) / 256 * 256; };
-  p.total = al(p.g_bytes) + al(p.c_bytes) + al(p.pairs_bytes) + al(p.csr_bytes) + 2 * al(p.delta_bytes);
+  p.total = al(p.g_bytes) + al(p.c_bytes) + al(p.pairs_bytes) + al(p.csr_bytes) + al(p.delta_bytes);
   return p;
 }
 
 constexpr int64_t kDefaultBudget = 32LL << 30;  // scratch for the G / C chunks (C3 in one chunk)
 
-// Scratch of the packed-token backward: the plan, then per chunk of `rows` groups G, C, delta
-// (twice: delta and the sink part) and the per-token mass.  total = 0: unpacked.
+// Scratch of the packed-token backward: the plan, then per chunk of `rows` groups G, C, the
+// sink's gradient parts and the per-token mass.  total = 0: unpacked.
 struct PackBwdPlan {
   int tt;
   int64_t rows, plan_bytes, g_bytes, c_bytes, delta_bytes, mass_bytes, total;
@@ -1106,14 +1064,14 @@ PackBwdPlan plan_pack_bwd(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_he
   const int64_t cap = pack_cap(topk, p.tt), groups = pack_groups(s_q, p.tt);
   auto al = [](int64_t x) { return (x + 255) / 256 * 256; };
   p.plan_bytes = pack_plan_bytes(batch, s_q, s_kv, topk, p.tt, true);
-  const int64_t per_row = batch * (cap * (kGW * 2 + width * 2 + p.tt * 4) + 2 * kHeadsMax * 4);
-  p.rows = std::min<int64_t>(groups, (budget - p.plan_bytes - 5 * 256) / per_row);
+  const int64_t per_row = batch * (cap * (kGW * 2 + width * 2 + p.tt * 4) + kHeadsMax * 4);
+  p.rows = std::min<int64_t>(groups, (budget - p.plan_bytes - 4 * 256) / per_row);
   if (p.rows < 1) return p;
   p.g_bytes = al(batch * p.rows * cap * kGW * 2);
   p.c_bytes = al(batch * p.rows * cap * width * 2);
   p.delta_bytes = al(batch * p.rows * kHeadsMax * 4);
   p.mass_bytes = al(batch * p.rows * p.tt * cap * 4);
-  p.total = p.plan_bytes + p.rows * per_row + 5 * 256;  // (at least the parts; the same rows for this budget)
+  p.total = p.plan_bytes + p.rows * per_row + 4 * 256;  // (at least the parts; the same rows for this budget)
   return p;
 }
 
@@ -1132,18 +1090,8 @@ extern "C" int64_t dsa_sparse_mla_bwd_workspace_size(int64_t batch, int64_t s_q,
 }
 
 namespace dsa {
-// delta and d sink of the tokens [t0, t0 + nt) of every batch element
-static int launch_sink_delta(const void* out, const void* dout, const float* smax, const float* ssum,
-                             const float* sinks, float* dsink, float* dbuf, float* pdbuf, int64_t batch, int64_t s_q,
-                             int64_t n_heads, int t0, int nt, hipStream_t st) {
-  {
-    const int64_t groups = batch * nt * n_heads;
-    const TimedLaunch tl("bwd_delta_kernel", st);
-    bwd_delta_kernel<<<(unsigned)((groups * 16 + 255) / 256), 256, 0, st>>>(
-        (const uint16_t*)out, (const uint16_t*)dout, dbuf, groups, (int)s_q, (int)n_heads, t0, nt, sinks, smax, ssum,
-        pdbuf);
-    if (int rc = check_launch("dsa_sparse_mla_bwd(delta)")) return rc;
-  }
+// d sink of nt tokens of every batch element, from the parts the score kernel left
+static int launch_sink_sum(const float* pdbuf, float* dsink, int64_t batch, int64_t n_heads, int nt, hipStream_t st) {
   const TimedLaunch tl("sink_colsum_kernel", st);
   sink_colsum_kernel<<<(unsigned)n_heads, 256, 0, st>>>(pdbuf, batch * nt, (int)n_heads, dsink);
   return check_launch("dsa_sparse_mla_bwd(sink)");
@@ -1153,18 +1101,16 @@ static int launch_sink_delta(const void* out, const void* dout, const float* sma
 template <bool kPack>
 static int launch_pair_kernels(dim3 ga, int hgroups, const void* q, const void* kv, const int32_t* indices,
                                const void* out, const void* dout, const float* softmax_max, const float* softmax_sum,
-                               const float* dbuf, uint16_t* gbuf, uint16_t* cbuf, void* dq, float* mass, int64_t s_q,
+                               float* pdbuf, uint16_t* gbuf, uint16_t* cbuf, void* dq, float* mass, int64_t s_q,
                                int64_t s_kv, int64_t n_heads, bool rope, int64_t topk, float scale, int64_t q_offset,
                                int r0, int rows, const float* sinks, const PackView& pk, hipStream_t st) {
   {
     static const char* const names[2][2] = {{"bwd_sdp_kernel<512>", "bwd_sdp_kernel<512, packed>"},
                                             {"bwd_sdp_kernel", "bwd_sdp_kernel<packed>"}};
     const TimedLaunch tl(names[rope][kPack], st);
-    // with no sink, delta is formed inside (the sink's gradient needs the delta pass)
-    auto* kern = sinks ? (rope ? bwd_sdp_kernel<kDqk, false, kPack> : bwd_sdp_kernel<kDv, false, kPack>)
-                       : (rope ? bwd_sdp_kernel<kDqk, true, kPack> : bwd_sdp_kernel<kDv, true, kPack>);
+    auto* kern = rope ? bwd_sdp_kernel<kDqk, kPack> : bwd_sdp_kernel<kDv, kPack>;
     kern<<<ga, 64 * kSdpWaves, 0, st>>>((const uint16_t*)q, (const uint16_t*)kv, indices, (const uint16_t*)dout,
-                                        (const uint16_t*)out, softmax_max, softmax_sum, dbuf, gbuf, mass, (int)s_q,
+                                        (const uint16_t*)out, softmax_max, softmax_sum, sinks, pdbuf, gbuf, mass, (int)s_q,
                                         (int)s_kv, (int)n_heads, (int)topk, scale, q_offset, r0, pk);
   }
   if (int rc = check_launch("dsa_sparse_mla_bwd(sdp)")) return rc;
@@ -1204,21 +1150,18 @@ static int sparse_mla_bwd_packed(const void* q, const void* kv, const int32_t* i
   char* p = ws + plan.plan_bytes;
   uint16_t* gbuf = (uint16_t*)p;
   uint16_t* cbuf = (uint16_t*)(p + plan.g_bytes);
-  float* dbuf = (float*)(p + plan.g_bytes + plan.c_bytes);
-  float* pdbuf = (float*)(p + plan.g_bytes + plan.c_bytes + plan.delta_bytes);
-  if (mass) pk.mass = (float*)(p + plan.g_bytes + plan.c_bytes + 2 * plan.delta_bytes);
+  float* pdbuf = (float*)(p + plan.g_bytes + plan.c_bytes);
+  if (mass) pk.mass = (float*)(p + plan.g_bytes + plan.c_bytes + plan.delta_bytes);
   const int hgroups = plan.tt * pk.hp <= kHG ? 1 : 2;  // 64-row halves of the workgroup in use
   for (int64_t g0 = 0; g0 < pk.groups; g0 += plan.rows) {
     const int n = (int)std::min<int64_t>(plan.rows, pk.groups - g0);
     const int t0 = (int)(g0 * plan.tt), nt = (int)std::min<int64_t>((int64_t)n * plan.tt, s_q - t0);
-    if (sinks)
-      if (int rc = launch_sink_delta(out, dout, softmax_max, softmax_sum, sinks, dsink, dbuf, pdbuf, batch, s_q,
-                                     n_heads, t0, nt, st))
-        return rc;
     if (int rc = launch_pair_kernels<true>(dim3((unsigned)n, 1, (unsigned)batch), hgroups, q, kv, indices, out, dout,
-                                           softmax_max, softmax_sum, dbuf, gbuf, cbuf, dq, nullptr, s_q, s_kv, n_heads,
+                                           softmax_max, softmax_sum, pdbuf, gbuf, cbuf, dq, nullptr, s_q, s_kv, n_heads,
                                            d_qk == kDqk, topk, scale, q_offset, (int)g0, n, sinks, pk, st))
       return rc;
+    if (sinks)
+      if (int rc = launch_sink_sum(pdbuf, dsink, batch, n_heads, nt, st)) return rc;
     if (mass)
       if (int rc = pack_mass_gather(pk, mass, batch, s_q, topk, g0, n, st)) return rc;
     if (int rc = pack_dkv_reduce(pk, cbuf, dkv_accum, batch, s_kv, d_qk, g0, n, st)) return rc;
@@ -1285,20 +1228,18 @@ static int sparse_mla_bwd_impl(const void* q, const void* kv, const int32_t* ind
   uint16_t* cbuf = (uint16_t*)(ws + al(plan.g_bytes));
   int* pairs = (int*)(ws + al(plan.g_bytes) + al(plan.c_bytes));
   int* counts = (int*)(ws + al(plan.g_bytes) + al(plan.c_bytes) + al(plan.pairs_bytes));
-  float* dbuf = (float*)(ws + al(plan.g_bytes) + al(plan.c_bytes) + al(plan.pairs_bytes) + al(plan.csr_bytes));
-  float* pdbuf = (float*)((char*)dbuf + al(plan.delta_bytes));  // the sink's per-(row, head) gradient parts
+  // the sink's per-(row, head) gradient parts
+  float* pdbuf = (float*)(ws + al(plan.g_bytes) + al(plan.c_bytes) + al(plan.pairs_bytes) + al(plan.csr_bytes));
 
   for (int64_t r0 = 0; r0 < s_q; r0 += plan.rows) {
     const int rows = (int)std::min<int64_t>(plan.rows, s_q - r0);
-    if (sinks)
-      if (int rc = launch_sink_delta(out, dout, softmax_max, softmax_sum, sinks, dsink, dbuf, pdbuf, batch, s_q,
-                                     n_heads, (int)r0, rows, st))
-        return rc;
     dim3 ga((unsigned)rows, 1, (unsigned)batch);
-    if (int rc = launch_pair_kernels<false>(ga, (int)hgroups, q, kv, indices, out, dout, softmax_max, softmax_sum, dbuf,
+    if (int rc = launch_pair_kernels<false>(ga, (int)hgroups, q, kv, indices, out, dout, softmax_max, softmax_sum, pdbuf,
                                             gbuf, cbuf, dq, mass, s_q, s_kv, n_heads, rope, topk, scale, q_offset,
                                             (int)r0, rows, sinks, PackView(), st))
       return rc;
+    if (sinks)
+      if (int rc = launch_sink_sum(pdbuf, dsink, batch, n_heads, rows, st)) return rc;
     // a prebuilt CSR of every row serves a one-chunk plan; otherwise each chunk builds its own
     const bool prebuilt = csr && rows == s_q;
     for (int b = 0; b < (int)batch; ++b) {

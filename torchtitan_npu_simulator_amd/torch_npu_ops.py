@@ -1078,6 +1078,15 @@ def v4_attention_indices(B, S, device, *, win_left=127, win_right=0, cmp_ratio=1
     offset by S (GetCompressTopkIdxs, :483-488; the ratio-128 layers).
     """
     W = win_left + win_right + 1
+    sel = cmp_ratio > 1 and n_cmp > 0
+    if torch.device(device).type == "cuda" and W > 0 and B > 0 and S > 0 and (not sel or cmp_indices is None or (
+            cmp_indices.is_cuda and cmp_indices.dtype == torch.int32 and cmp_indices.shape[:-1] == (B, S))):
+        n_sel = 0 if not sel else n_cmp if cmp_indices is None else cmp_indices.shape[-1]
+        ci = cmp_indices.contiguous() if sel and cmp_indices is not None and n_sel else None
+        out = torch.empty(B, S, W + n_sel, dtype=torch.int32, device=device)
+        check(load_library().dsa_v4_indices(ptr(ci), ptr(out), B, S, int(win_left), W, int(cmp_ratio), n_sel,
+                                            stream_of(out.device)), "dsa_v4_indices")
+        return out
     s_pos = torch.arange(S, device=device).view(S, 1)
     w = s_pos - win_left + torch.arange(W, device=device).view(1, W)
     w = torch.where((w >= 0) & (w < S), w, torch.full_like(w, -1))
