@@ -269,7 +269,9 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream_of(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """Raw handle of the current stream of ``device`` (without building a Stream object)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def require_gpu_tensor(t: torch.Tensor, name: str) -> None:

@@ -899,10 +899,13 @@ class _SparseFlashAttention(torch.autograd.Function):
         ctx.split = (q_nope.shape[-1], q_pe.shape[-1])
         ctx.kv_shape = kv.shape
         ctx.mark_non_differentiable(smax, ssum)
+        ctx.set_materialize_grads(False)  # (no zero gradients of smax and ssum)
         return out, smax, ssum
 
     @staticmethod
     def backward(ctx, dout, _dmax, _dsum):
+        if dout is None:
+            return (None,) * 7
         q, kv3, indices, out, smax, ssum = ctx.saved_tensors
         dq, dkv = sparse_mla_bwd(q, kv3, indices, out, dout.contiguous(), smax, ssum, ctx.scale, q_offset=ctx.q_offset)
         dnope, dpe = ctx.split
@@ -960,10 +963,13 @@ class _SparseFlashAttentionLinked(torch.autograd.Function):
         link.scale = scale
         link.q_offset = q_offset
         ctx.mark_non_differentiable(smax, ssum)
+        ctx.set_materialize_grads(False)  # (no zero gradients of smax and ssum)
         return out, smax, ssum
 
     @staticmethod
     def backward(ctx, dout, _dmax, _dsum):
+        if dout is None:
+            return (None,) * 8
         q, kv3, indices, out, smax, ssum = ctx.saved_tensors
         dq, dkv, mass = sparse_mla_bwd(q, kv3, indices, out, dout.contiguous(), smax, ssum, ctx.scale,
                                        q_offset=ctx.q_offset, return_mass=True)
@@ -996,10 +1002,13 @@ class _SparseFlashAttentionTND(torch.autograd.Function):
         ctx.split = (q_nope.shape[-1], q_pe.shape[-1])
         ctx.kv_shape = kv.shape
         ctx.mark_non_differentiable(smax, ssum)
+        ctx.set_materialize_grads(False)  # (no zero gradients of smax and ssum)
         return out, smax, ssum
 
     @staticmethod
     def backward(ctx, dout, _dmax, _dsum):
+        if dout is None:
+            return (None,) * 8
         q, kv2, indices, out, smax, ssum = ctx.saved_tensors
         dq, dkv = sparse_mla_bwd_varlen(q, kv2, indices, out, dout.contiguous(), smax, ssum, ctx.scale, *ctx.cu)
         dnope, _ = ctx.split
@@ -1229,31 +1238,44 @@ def npu_sparse_attn_sharedkv_metadata(
     ``npu_sparse_attn_sharedkv`` to check against its own arguments; the host copy of the
     record rides on the tensor, so the check reads no device memory.
     """
-    if num_heads_kv != 1:
-        raise NotImplementedError(f"num_heads_kv={num_heads_kv}: the shared KV has one head")
-    if ori_mask_mode != 4 or cmp_mask_mode != 3:
-        raise NotImplementedError("mask modes: band window (4) over ori_kv, causal (3) over cmp_kv")
+    rec = _sharedkv_record(num_heads_q, num_heads_kv, head_dim, batch_size, max_seqlen_q, max_seqlen_kv, ori_topk,
+                           cmp_topk, cmp_ratio, ori_mask_mode, cmp_mask_mode, ori_win_left, ori_win_right, layout_q,
+                           layout_kv, has_ori_kv, has_cmp_kv)
     for name, t in (("seqused_ori_kv", seqused_ori_kv), ("seqused_cmp_kv", seqused_cmp_kv),
                     ("seqused_q", seqused_q), ("seqused_kv", seqused_kv)):
         if t is not None and t.numel():
             raise NotImplementedError(f"{name} (per-batch used lengths) is not supported")
     if device is None:
         device = cu_seqlens_q.device if cu_seqlens_q is not None else torch.device("cuda", torch.cuda.current_device())
-    rec = [_SHAREDKV_MAGIC, 1, int(num_heads_q), int(num_heads_kv), int(head_dim), int(batch_size),
-           int(max_seqlen_q), int(max_seqlen_kv), int(ori_topk), int(cmp_topk), int(cmp_ratio), int(ori_mask_mode),
-           int(cmp_mask_mode), int(ori_win_left), int(ori_win_right), _LAYOUT_CODES.get(str(layout_q), 0),
-           _LAYOUT_CODES.get(str(layout_kv), 0), int(bool(has_ori_kv)), int(bool(has_cmp_kv))]
     meta = torch.zeros(1024, dtype=torch.int32)
     meta[: len(rec)] = torch.tensor(rec, dtype=torch.int32)
     meta = meta.to(device)
-    meta._dsa_record = tuple(rec)
+    meta._dsa_record = rec
     return meta
+
+
+def _sharedkv_record(num_heads_q, num_heads_kv, head_dim, batch_size, max_seqlen_q, max_seqlen_kv, ori_topk, cmp_topk,
+                     cmp_ratio, ori_mask_mode, cmp_mask_mode, ori_win_left, ori_win_right, layout_q, layout_kv,
+                     has_ori_kv, has_cmp_kv):
+    """The problem description of npu_sparse_attn_sharedkv_metadata, as a tuple of ints."""
+    if num_heads_kv != 1:
+        raise NotImplementedError(f"num_heads_kv={num_heads_kv}: the shared KV has one head")
+    if ori_mask_mode != 4 or cmp_mask_mode != 3:
+        raise NotImplementedError("mask modes: band window (4) over ori_kv, causal (3) over cmp_kv")
+    return (_SHAREDKV_MAGIC, 1, int(num_heads_q), int(num_heads_kv), int(head_dim), int(batch_size),
+            int(max_seqlen_q), int(max_seqlen_kv), int(ori_topk), int(cmp_topk), int(cmp_ratio), int(ori_mask_mode),
+            int(cmp_mask_mode), int(ori_win_left), int(ori_win_right), _LAYOUT_CODES.get(str(layout_q), 0),
+            _LAYOUT_CODES.get(str(layout_kv), 0), int(bool(has_ori_kv)), int(bool(has_cmp_kv)))
 
 
 def _check_sharedkv_metadata(metadata, query, cmp_kv, cmp_ratio, ori_win_left, ori_win_right):
     rec = getattr(metadata, "_dsa_record", None) if metadata is not None else None
     if rec is None:
         return
+    _check_sharedkv_record(rec, query, cmp_kv, cmp_ratio, ori_win_left, ori_win_right)
+
+
+def _check_sharedkv_record(rec, query, cmp_kv, cmp_ratio, ori_win_left, ori_win_right):
     if query.dim() == 3:  # TND: [T, N, D]; the record's batch size counts sequences
         H, D = query.shape[1:]
         B = rec[5]
@@ -1525,11 +1547,12 @@ class SparseAttnSharedKV(torch.autograd.Function):
         tnd = _check_sharedkv_args(layout_q, layout_kv, ori_sparse_indices, (),
                                    (cu_seq_lens_q, cu_seq_lens_ori_kv, cu_seq_lens_cmp_kv), ori_mask_mode,
                                    cmp_mask_mode)
-        metadata = npu_sparse_attn_sharedkv_metadata(
-            cu_seq_lens_q, None, None, None, None, num_heads_q, num_heads_kv, head_dim, batch_size, max_seq_len_q,
-            max_seq_len_kv, 0, topk, cmp_ratio, ori_mask_mode, cmp_mask_mode, ori_win_left, ori_win_right, layout_q,
-            layout_kv, ori_kv is not None, cmp_kv is not None, device=query.device)
-        _check_sharedkv_metadata(metadata, query, cmp_kv, cmp_ratio, ori_win_left, ori_win_right)
+        # (the metadata op's checks on its record; its device tensor has no reader here)
+        _check_sharedkv_record(
+            _sharedkv_record(num_heads_q, num_heads_kv, head_dim, batch_size, max_seq_len_q, max_seq_len_kv, 0, topk,
+                             cmp_ratio, ori_mask_mode, cmp_mask_mode, ori_win_left, ori_win_right, layout_q, layout_kv,
+                             ori_kv is not None, cmp_kv is not None),
+            query, cmp_kv, cmp_ratio, ori_win_left, ori_win_right)
         # the kernels' operands are kept for backward (the bf16 path pads query rows to 512)
         geo = _sharedkv_tnd_args(cu_seq_lens_q, cu_seq_lens_ori_kv, cu_seq_lens_cmp_kv, None, cmp_kv,
                                  cmp_ratio) if tnd else None
