@@ -297,6 +297,17 @@ int dsa_sparse_mla_bwd_ex(const void* q, const void* kv, const int32_t* indices,
 int dsa_attn_mass(const void* q, const void* kv, const int32_t* indices, const float* softmax_max,
                   const float* softmax_sum, float* mass, int dtype, int64_t batch, int64_t s_q, int64_t s_kv,
                   int64_t n_heads, int64_t d_qk, int64_t topk, float scale, int64_t q_offset, void* stream);
+/*
+ * The same with a caller workspace of dsa_attn_mass_workspace_size() bytes (16-byte aligned).
+ * The size is 0 where it has no use; with fewer bytes, or none, the call runs as dsa_attn_mass.
+ * bf16 calls of at most 64 heads use it to let several consecutive tokens share a workgroup.
+ */
+int64_t dsa_attn_mass_workspace_size(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
+                                     int64_t topk, int64_t q_offset);
+int dsa_attn_mass_ws(const void* q, const void* kv, const int32_t* indices, const float* softmax_max,
+                     const float* softmax_sum, float* mass, int dtype, int64_t batch, int64_t s_q, int64_t s_kv,
+                     int64_t n_heads, int64_t d_qk, int64_t topk, float scale, int64_t q_offset, void* workspace,
+                     int64_t workspace_bytes, void* stream);
 
 /*
  * Indexer KL loss and its gradients (reference: DSAIndexerLoss.forward,

@@ -514,11 +514,20 @@ int fwd_splits(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_
 // two workgroups share a CU.  Each wave sums P over its 32 heads (permlane16 swap, then
 // DPP exchanges), the four waves' sums meet in LDS behind the block's barrier, and wave 0
 // stores the block's 128-byte row segment at the start of the next iteration.
-template <int kD>  // row width of Q and KV: 576 (latent + rope) or 512 (no rope)
+// kPack (attn_pack.h): the workgroup's 128 rows are (token, head) pairs of pk.tt tokens over the
+// union of their keys; a row masks the keys its token did not select, each half of a wave's 32
+// rows (one token: hp is a multiple of 16) is summed by itself, and the sums go to pk.mass by
+// union slot, from where pack_mass_gather takes the tokens' own slots.  With few heads the
+// one-token form computes 128 rows per token all the same.  Top-2048, kernel alone: 2500
+// tokens, 64 heads 547 us -> 337 with plan and gather; 1500 tokens, 16 heads 200 -> 101; 600
+// tokens, 32 heads, top-512 49 -> 47 (the forward's rule, pack_tokens, is kept as it is: its
+// plan costs the same here).
+template <int kD, bool kPack>  // kD, row width of Q and KV: 576 (latent + rope) or 512 (no rope)
 __global__ void __launch_bounds__(kFwdThreads, 2)
 attn_mass_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv,
                       const int32_t* __restrict__ idx, const float* __restrict__ smax, const float* __restrict__ ssum,
-                      float* __restrict__ mass, int S, int s_kv, int H, int K, float scale_log2, int64_t q_offset) {
+                      float* __restrict__ mass, int S, int s_kv, int H, int K, float scale_log2, int64_t q_offset,
+                      PackView pk, int g0) {
   using Gather = RowGather<kFwdWaves, kD>;
   using Geo = GatherGeomT<kD>;
   constexpr int kPer = Gather::kMaxPerWave;
@@ -526,26 +535,44 @@ attn_mass_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict
   constexpr int kKS = kD / 16;  // MFMA k-steps of S^T (36 | 32)
   __shared__ u32x4 tile[2][kTC];
   __shared__ int sidx[GatherGeom::kRing][Gather::kRingInts];
-  __shared__ float part[2][kFwdWaves][kBN];  // [block parity][wave][key]: per-wave head sums
+  constexpr int kParts = kPack ? 2 * kFwdWaves : kFwdWaves;
+  __shared__ float part[2][kParts][kBN];  // [block parity][wave | half wave][key]: head sums
   __shared__ int sh_last;
 
-  const int tok = blockIdx.x, b = blockIdx.z, tid = threadIdx.x;
+  const int b = blockIdx.z, tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int n = lane & 31, h = lane >> 5;  // MFMA column (head / key row) and k half
-  const int head = blockIdx.y * kFwdHeads + wave * 32 + n;
-  const bool hok = head < H;
+  const int lg = (int)(gridDim.x - 1u - blockIdx.x);  // (packed) group within the chunk, longest rows first
+  const int grp = kPack ? g0 + lg : 0;
+  int tok = blockIdx.x, head = blockIdx.y * kFwdHeads + wave * 32 + n;
+  bool hok = head < H;
+  if constexpr (kPack) {
+    int t;
+    pack_row(pk, wave * 32 + n, t, head);
+    tok = grp * pk.tt + t;
+    hok = t < pk.tt && tok < S && head < H;
+    if (!hok) tok = grp * pk.tt;  // (a token that exists)
+  }
   const int64_t row_id = (int64_t)b * S + tok;
   const int64_t hrow = row_id * H + (hok ? head : 0);
-  const int32_t* ridx = idx + row_id * K;
-  float* mrow = mass + row_id * K;
-  const int64_t limit = tok + q_offset;
+  const int64_t pgrp = (int64_t)b * pk.groups + grp;
+  const int32_t* ridx = kPack ? pk.idx + pgrp * pk.cap : idx + row_id * K;
+  if constexpr (kPack) K = pk.cap;
+  float* mrow = kPack ? pk.mass + ((int64_t)b * gridDim.x + lg) * pk.tt * pk.cap : mass + row_id * K;
+  const int64_t limit = kPack ? (int64_t)s_kv : tok + q_offset;  // (packed: the plan applied the causal rule)
+  // the tokens of the wave's rows 0..15 and 16..31
+  const pack_word *mask_lo = nullptr, *mask_hi = nullptr;
+  if constexpr (kPack) {
+    mask_lo = pack_mask_row(pk, pgrp, wave * 32);
+    mask_hi = pack_mask_row(pk, pgrp, wave * 32 + 16);
+  }
   const uint16_t* kvb = kv + (int64_t)b * s_kv * kD;
 
   // the row's slot indices (block count), the ring entries of blocks 0..2 (wave 0, DMA),
   // the head's Q row and row statistics are requested together (unconditional loads from
   // head 0's row for absent heads, whose lse2 is then +inf)
   int vidx[kIdxU];
-  load_row_indices(ridx, K, vidx);
+  if constexpr (!kPack) load_row_indices(ridx, K, vidx);
   if (wave == 0) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) Gather::issue_idx(ridx, K, i, sidx[i], lane);  // clamped to slot K-1
@@ -557,8 +584,8 @@ attn_mass_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict
     for (int s = 0; s < kKS; ++s) qb[s] = qh[2 * s + h];
   }
   const float mx = smax[hrow], sm = ssum[hrow];
-  const int nblk = count_row_blocks(ridx, K, s_kv, limit, vidx, &sh_last);
-  if (blockIdx.y == 0)  // slots past the last usable block hold no mass
+  const int nblk = kPack ? (pk.count[pgrp] + kBN - 1) / kBN : count_row_blocks(ridx, K, s_kv, limit, vidx, &sh_last);
+  if (!kPack && blockIdx.y == 0)  // slots past the last usable block hold no mass
     for (int j = nblk * kBN + tid; j < K; j += kFwdThreads) mrow[j] = 0.f;
   if (nblk == 0) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the ring DMA has landed before the LDS is released
@@ -577,7 +604,7 @@ attn_mass_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict
   const typename Gather::PackedLanes gl = Gather::packed_lanes(wave, lane);
   if (wave == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // ring entries 0..2 landed
   __syncthreads();
-  uint32_t vm_cur = Gather::ring_valid(sidx[0], lane, lim, K);
+  uint32_t vm_cur = kPack ? 0u : Gather::ring_valid(sidx[0], lane, lim, K);
 #pragma unroll
   for (int i = 0; i < kPer; ++i) Gather::issue_slot(kvb, &tile[0][0], i, wave, Gather::ring_slot(sidx[0], i, gl), gl, lim, K);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -591,7 +618,7 @@ attn_mass_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict
   // instruction per batch (the forward's schedule); returns the next block's validity bits
   auto qk = [&](const lds_char* tb, u32x4* dst_tile, const int* ring, int rows_left, f32x16& sacc)
       __attribute__((always_inline)) {
-    const uint32_t vm_n = Gather::ring_valid(ring, lane, lim, rows_left);
+    const uint32_t vm_n = kPack ? 0u : Gather::ring_valid(ring, lane, lim, rows_left);
     uint32_t raw_next = Gather::ring_slot(ring, 0, gl);
     sacc = (f32x16){0.f};
     u32x4 a[2][kQBatch];
@@ -641,12 +668,14 @@ attn_mass_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict
       pv[v] = ok ? __builtin_amdgcn_exp2f(sacc[v] * scale_log2 - lse2) : 0.f;
     }
     const bool odd = (lane >> 4) & 1;
+    if constexpr (!kPack)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {  // even rows keep value j, odd rows j + 8
-      const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(pv[j]), __float_as_uint(pv[j + 8]), false, false);
-      const float even_sum = pv[j] + __uint_as_float(r[1]), odd_sum = pv[j + 8] + __uint_as_float(r[0]);
-      pv[j] = odd ? odd_sum : even_sum;
-    }
+      for (int j = 0; j < 8; ++j) {  // even rows keep value j, odd rows j + 8
+        const auto r =
+            __builtin_amdgcn_permlane16_swap(__float_as_uint(pv[j]), __float_as_uint(pv[j + 8]), false, false);
+        const float even_sum = pv[j] + __uint_as_float(r[1]), odd_sum = pv[j + 8] + __uint_as_float(r[0]);
+        pv[j] = odd ? odd_sum : even_sum;
+      }
     auto bstep = [&](auto mc, int nh) __attribute__((always_inline)) {
       constexpr int m = decltype(mc)::value;
       const uint32_t up = ((lane & m) != 0) ? 0xffffffffu : 0u;
@@ -658,6 +687,15 @@ attn_mass_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict
         pv[j] = keep + lane_xor<m>(send);
       }
     };
+    if constexpr (kPack) {  // lane bits 3..0 halve the 16 values: lane l ends with value l & 15
+      bstep(std::integral_constant<int, 8>{}, 8);
+      bstep(std::integral_constant<int, 4>{}, 4);
+      bstep(std::integral_constant<int, 2>{}, 2);
+      bstep(std::integral_constant<int, 1>{}, 1);
+      const int r = lane & 15;
+      part[pb][2 * wave + odd][8 * (r >> 2) + 4 * h + (r & 3)] = pv[0];
+      return;
+    }
     bstep(std::integral_constant<int, 8>{}, 4);
     bstep(std::integral_constant<int, 4>{}, 2);
     bstep(std::integral_constant<int, 2>{}, 1);
@@ -671,6 +709,16 @@ attn_mass_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict
   // block fb's four wave sums -> global (its partials were published by the barrier that
   // ended its iteration); several head groups add into a zeroed row
   auto flush = [&](int fb) __attribute__((always_inline)) {
+    if constexpr (kPack) {  // 32 lanes per token, its hp / 16 half waves in order
+      const int t = tid >> 5, key = tid & (kBN - 1);
+      if (t < pk.tt) {
+        const int u0 = t * (pk.hp >> 4);
+        float s = part[fb & 1][u0][key];
+        for (int u = 1; u < pk.hp >> 4; ++u) s += part[fb & 1][u0 + u][key];
+        mrow[(int64_t)t * pk.cap + fb * kBN + key] = s;
+      }
+      return;
+    }
     if (wave == 0 && lane < kBN) {
       const int pb = fb & 1;
       const float t = (part[pb][0][lane] + part[pb][1][lane]) + (part[pb][2][lane] + part[pb][3][lane]);
@@ -689,11 +737,16 @@ attn_mass_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict
     if (blk > 0) flush(blk - 1);
     if (wave == 0 && blk + 3 < nblk)
       Gather::issue_idx(ridx, K, blk + 3, sidx[(blk + 3) & (GatherGeom::kRing - 1)], lane);
+    uint32_t vm_lo = 0u, vm_hi = 0u;
+    if constexpr (kPack) {
+      vm_lo = mask_lo[blk];
+      vm_hi = mask_hi[blk];
+    }
     f32x16 sacc;
     // ring entry blk+1 landed during iteration blk-2 (or before the loop)
     const uint32_t vm_next = qk(lds_bytes(&tile[blk & 1][0]), &tile[(blk + 1) & 1][0],
                                 sidx[(blk + 1) & (GatherGeom::kRing - 1)], K - (blk + 1) * kBN, sacc);
-    block_mass(sacc, vm_cur, blk & 1);
+    block_mass(sacc, kPack ? (n < 16 ? vm_lo : vm_hi) : vm_cur, blk & 1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // block blk+1 and ring entry blk+3 landed
     __syncthreads();
     vm_cur = vm_next;
@@ -825,10 +878,34 @@ attn_mass_f32_kernel(const float* __restrict__ q, const float* __restrict__ kv, 
 
 }  // namespace dsa
 
-extern "C" int dsa_attn_mass(const void* q, const void* kv, const int32_t* indices, const float* softmax_max,
+namespace dsa {
+// Workspace of the packed mass: the plan and the head sums of a chunk of groups by union slot,
+// [batch][groups of the chunk][tt][cap] fp32, at most kMassBudget or one group per element.
+constexpr int64_t kMassBudget = 1LL << 29;
+static int64_t mass_chunk_groups(int64_t batch, int64_t s_q, int64_t topk, int tt) {
+  const int64_t per = batch * tt * pack_cap(topk, tt) * 4;
+  return std::max<int64_t>(1, std::min<int64_t>(pack_groups(s_q, tt), kMassBudget / per));
+}
+static int64_t mass_workspace_bytes(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
+                                    int64_t topk, int64_t q_offset) {
+  if (dtype != DSA_BF16 || topk <= 0) return 0;
+  const int tt = pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset);
+  if (tt <= 1) return 0;
+  return pack_plan_bytes(batch, s_q, s_kv, topk, tt, true) +
+         mass_chunk_groups(batch, s_q, topk, tt) * batch * tt * pack_cap(topk, tt) * 4;
+}
+}  // namespace dsa
+
+extern "C" int64_t dsa_attn_mass_workspace_size(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
+                                                int64_t topk, int64_t q_offset) {
+  if (batch <= 0 || s_q <= 0 || s_kv <= 0) return 0;
+  return dsa::mass_workspace_bytes(dtype, batch, s_q, s_kv, n_heads, topk, q_offset);
+}
+
+extern "C" int dsa_attn_mass_ws(const void* q, const void* kv, const int32_t* indices, const float* softmax_max,
                              const float* softmax_sum, float* mass, int dtype, int64_t batch, int64_t s_q, int64_t s_kv,
                              int64_t n_heads, int64_t d_qk, int64_t topk, float scale, int64_t q_offset,
-                             void* stream) {
+                             void* workspace, int64_t workspace_bytes, void* stream) {
   using namespace dsa;
   if (!q || !kv || !indices || !softmax_max || !softmax_sum || !mass)
     return set_error(DSA_ERR_INVALID_ARG, "dsa_attn_mass: null pointer");
@@ -842,16 +919,38 @@ extern "C" int dsa_attn_mass(const void* q, const void* kv, const int32_t* indic
       return set_error(DSA_ERR_UNSUPPORTED, "dsa_attn_mass: bf16 path needs d_qk = 576 or 512 (got %lld)", (long long)d_qk);
     const int64_t max_rows = d_qk == kDqk ? GatherGeomT<kDqk>::kMaxRows : GatherGeomT<kDv>::kMaxRows;
     if (s_kv > max_rows) return set_error(DSA_ERR_UNSUPPORTED, "dsa_attn_mass: S_kv > %lld", (long long)max_rows);
+    const int64_t need = workspace ? mass_workspace_bytes(dtype, batch, s_q, s_kv, n_heads, topk, q_offset) : 0;
+    if (need > 0 && workspace_bytes >= need && (uintptr_t)workspace % 16 == 0) {
+      const int tt = pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset);
+      PackView pk;
+      if (int rc = pack_plan_build(indices, batch, s_q, s_kv, n_heads, topk, q_offset, tt, true, workspace, st, &pk))
+        return rc;
+      pk.mass = (float*)((char*)workspace + pack_plan_bytes(batch, s_q, s_kv, topk, tt, true));
+      const int64_t chunk = mass_chunk_groups(batch, s_q, topk, tt);
+      for (int64_t g0 = 0; g0 < pk.groups; g0 += chunk) {
+        const int64_t n = std::min<int64_t>(chunk, pk.groups - g0);
+        {
+          auto kern = d_qk == kDqk ? attn_mass_bf16_kernel<kDqk, true> : attn_mass_bf16_kernel<kDv, true>;
+          const TimedLaunch tl(d_qk == kDqk ? "attn_mass_bf16_kernel<packed>" : "attn_mass_bf16_kernel<512, packed>", st);
+          kern<<<dim3((unsigned)n, 1, (unsigned)batch), kFwdThreads, 0, st>>>(
+              (const uint16_t*)q, (const uint16_t*)kv, indices, softmax_max, softmax_sum, mass, (int)s_q, (int)s_kv,
+              (int)n_heads, (int)topk, scale * kLog2e, q_offset, pk, (int)g0);
+        }
+        if (int rc = pack_mass_gather(pk, mass, batch, s_q, topk, g0, n, st)) return rc;
+      }
+      return check_launch("dsa_attn_mass(bf16, packed)");
+    }
     const unsigned hgroups = ceil_div(n_heads, kFwdHeads);
     if (hgroups > 1) {  // partial sums from several head groups accumulate into a zeroed buffer
       if (hipMemsetAsync(mass, 0, (size_t)(batch * s_q * topk) * 4, st) != hipSuccess)
         return set_error(DSA_ERR_LAUNCH, "dsa_attn_mass: memset failed");
     }
     dim3 grid((unsigned)s_q, hgroups, (unsigned)batch);
-    auto kern = d_qk == kDqk ? attn_mass_bf16_kernel<kDqk> : attn_mass_bf16_kernel<kDv>;
+    auto kern = d_qk == kDqk ? attn_mass_bf16_kernel<kDqk, false> : attn_mass_bf16_kernel<kDv, false>;
     const TimedLaunch tl(d_qk == kDqk ? "attn_mass_bf16_kernel" : "attn_mass_bf16_kernel<512>", st);
     kern<<<grid, kFwdThreads, 0, st>>>((const uint16_t*)q, (const uint16_t*)kv, indices, softmax_max, softmax_sum, mass,
-                                       (int)s_q, (int)s_kv, (int)n_heads, (int)topk, scale * kLog2e, q_offset);
+                                       (int)s_q, (int)s_kv, (int)n_heads, (int)topk, scale * kLog2e, q_offset,
+                                       PackView{}, 0);
     return check_launch("dsa_attn_mass(bf16)");
   }
   if (dtype == DSA_F32) {
@@ -863,6 +962,14 @@ extern "C" int dsa_attn_mass(const void* q, const void* kv, const int32_t* indic
     return check_launch("dsa_attn_mass(f32)");
   }
   return set_error(DSA_ERR_UNSUPPORTED, "dsa_attn_mass: dtype %d", dtype);
+}
+
+extern "C" int dsa_attn_mass(const void* q, const void* kv, const int32_t* indices, const float* softmax_max,
+                             const float* softmax_sum, float* mass, int dtype, int64_t batch, int64_t s_q, int64_t s_kv,
+                             int64_t n_heads, int64_t d_qk, int64_t topk, float scale, int64_t q_offset,
+                             void* stream) {
+  return dsa_attn_mass_ws(q, kv, indices, softmax_max, softmax_sum, mass, dtype, batch, s_q, s_kv, n_heads, d_qk, topk,
+                          scale, q_offset, nullptr, 0, stream);
 }
 
 namespace dsa {

@@ -743,7 +743,7 @@ def sparse_mla_bwd(q, kv, indices, out, dout, smax, ssum, scale, *, q_offset=0, 
 
 
 def attn_mass(q, kv, indices, smax, ssum, scale, *, q_offset=0):
-    """Head-summed softmax mass [B,S,K] at the selected slots (dsa_attn_mass)."""
+    """Head-summed softmax mass [B,S,K] at the selected slots (dsa_attn_mass_ws)."""
     lib = load_library()
     B, S, H, D = q.shape
     s_kv = kv.shape[1]
@@ -752,10 +752,13 @@ def attn_mass(q, kv, indices, smax, ssum, scale, *, q_offset=0):
     kv = kv.contiguous()
     indices = indices.reshape(B, S, K).to(torch.int32).contiguous()
     mass = torch.empty(B, S, K, dtype=torch.float32, device=q.device)
+    dt = _lib.dtype_code(q.dtype)
+    ws_bytes = int(lib.dsa_attn_mass_workspace_size(dt, B, S, s_kv, H, K, int(q_offset)))
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
     check(
-        lib.dsa_attn_mass(ptr(q), ptr(kv), ptr(indices), ptr(smax.contiguous()), ptr(ssum.contiguous()), ptr(mass),
-                          _lib.dtype_code(q.dtype), B, S, s_kv, H, D, K, float(scale), int(q_offset),
-                          stream_of(q.device)),
+        lib.dsa_attn_mass_ws(ptr(q), ptr(kv), ptr(indices), ptr(smax.contiguous()), ptr(ssum.contiguous()), ptr(mass),
+                             dt, B, S, s_kv, H, D, K, float(scale), int(q_offset), ptr(ws), ws_bytes,
+                             stream_of(q.device)),
         "dsa_attn_mass",
     )
     return mass
@@ -850,8 +853,10 @@ def attn_mass_varlen(q, kv, indices, smax, ssum, scale, cu_seqlens_q, cu_seqlens
     lib = load_library()
     T, H, D = q.shape
     kv = kv.reshape(kv.shape[0], kv.shape[-1]).contiguous()
-    g = _varlen_global(indices, cu_seqlens_q, cu_seqlens_kv, T, kv.shape[0], q.device)
-    if g is not None:  # device bounds: one launch over the batch
+    packed = q.dtype == torch.bfloat16 and T > 0 and lib.dsa_attn_mass_workspace_size(
+        _lib.DSA_BF16, 1, T, kv.shape[0], H, indices.shape[-1], _NO_MASK_OFFSET) > 0
+    g = _varlen_global(indices, cu_seqlens_q, cu_seqlens_kv, T, kv.shape[0], q.device, packed)
+    if g is not None:  # device bounds, packed tokens: one launch over the batch
         return attn_mass(q.unsqueeze(0), kv.unsqueeze(0), g.unsqueeze(0), smax.unsqueeze(0), ssum.unsqueeze(0), scale,
                          q_offset=_NO_MASK_OFFSET)[0]
     cu_q, cu_k, n_seq = _varlen_seqs(cu_seqlens_q, cu_seqlens_kv, T, kv.shape[0])
