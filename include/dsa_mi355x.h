@@ -487,6 +487,10 @@ int dsa_mla_absorb_wgrad(const void* a, int64_t lda, const void* b, int64_t ldb,
 int dsa_mla_absorb(const void* a, int64_t lda, const void* wt, void* c, int64_t ldc, const void* append,
                    int64_t ld_append, int64_t append_width, int64_t tokens, int64_t heads, int64_t k, int64_t n,
                    void* stream);
+/* The same products with the weight as it is, w [heads, k, n]. */
+int dsa_mla_absorb_rows(const void* a, int64_t lda, const void* w, void* c, int64_t ldc, const void* append,
+                        int64_t ld_append, int64_t append_width, int64_t tokens, int64_t heads, int64_t k, int64_t n,
+                        void* stream);
 
 /*
  * Packed varlen ("TND") metadata built on the device (reference: build_smla_attention_masks,

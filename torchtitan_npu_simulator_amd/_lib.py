@@ -111,6 +111,7 @@ _SIGNATURES = {
     "dsa_indexer_prep": ([_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i32, _i32, _vp],
                          _i32),
     "dsa_mla_absorb": ([_vp, _i64, _vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp], _i32),
+    "dsa_mla_absorb_rows": ([_vp, _i64, _vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp], _i32),
     "dsa_mla_absorb_wgrad_workspace_size": ([_i64, _i64], _i64),
     "dsa_mla_absorb_wgrad": ([_vp, _i64, _vp, _i64, _vp, _i32, _i32, _i64, _i64, _vp, _i64, _vp], _i32),
     "dsa_tnd_metadata": ([_vp, _i32, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp], _i32),

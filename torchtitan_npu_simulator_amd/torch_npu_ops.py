@@ -2102,23 +2102,31 @@ def mla_absorb(a, wt, *, append=None):
     a [..., H, K] bf16 (rows may be a strided view, e.g. the first 512 columns of a 576-wide
     gradient), wt [H, N, K] bf16, append [..., H, E] or None; (K, N) = (128, 512) or
     (512, 128).  Returns c [..., H, N + E] bf16, contiguous."""
+    return _absorb(a, wt, append, k_rows=False)
+
+
+def _absorb(a, wt, append, *, k_rows):
+    """``mla_absorb``, or with ``k_rows`` the same for a weight [H, K, N] (dsa_mla_absorb_rows)."""
     lib = load_library()
     require_gpu_tensor(a, "a")
     a, lda = _rows_view(a.to(torch.bfloat16))
     H, K = a.shape[-2], a.shape[-1]
-    N = wt.shape[1]
-    if wt.shape != (H, N, K):
+    N = wt.shape[2 if k_rows else 1]
+    if wt.shape != ((H, K, N) if k_rows else (H, N, K)):
         raise ValueError(f"weight {tuple(wt.shape)} does not fit rows [.., {H}, {K}]")
     lead = a.shape[:-2]
     tokens = math.prod(lead)
     wt = wt.to(torch.bfloat16).contiguous()
+    if k_rows and wt.data_ptr() % 16:  # (a slice of a larger buffer: the kernel reads 16 bytes at a time)
+        wt = wt.clone()
     E, lde = 0, 0
     if append is not None:
         append, lde = _rows_view(append.to(torch.bfloat16))
         E = append.shape[-1]
     out = torch.empty(*lead, H, N + E, dtype=torch.bfloat16, device=a.device)
-    check(lib.dsa_mla_absorb(ptr(a), lda, ptr(wt), ptr(out), N + E, ptr(append), lde, E, tokens, H, K, N,
-                             stream_of(a.device)), "dsa_mla_absorb")
+    entry = lib.dsa_mla_absorb_rows if k_rows else lib.dsa_mla_absorb
+    check(entry(ptr(a), lda, ptr(wt), ptr(out), N + E, ptr(append), lde, E, tokens, H, K, N, stream_of(a.device)),
+          "dsa_mla_absorb")
     return out
 
 
@@ -2143,8 +2151,7 @@ def _absorb_wgrad(a, b, dtype, *, wide_rows):
 class _AbsorbQ(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q_nope, q_pe, w_uk):
-        wt = w_uk.transpose(1, 2).contiguous()  # [H, 512, 128]
-        q = mla_absorb(q_nope, wt, append=q_pe)
+        q = _absorb(q_nope, w_uk, q_pe, k_rows=True)
         ctx.save_for_backward(q_nope, w_uk)
         ctx.rope = q_pe.shape[-1]
         return q
@@ -2169,8 +2176,7 @@ class _AbsorbQ(torch.autograd.Function):
 class _AbsorbOut(torch.autograd.Function):
     @staticmethod
     def forward(ctx, out, w_uv_t):
-        wt = w_uv_t.transpose(1, 2).contiguous()  # [H, 128, 512]
-        y = mla_absorb(out, wt)
+        y = _absorb(out, w_uv_t, None, k_rows=True)
         ctx.save_for_backward(out, w_uv_t)
         return y
 
