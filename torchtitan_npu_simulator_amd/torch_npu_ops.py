@@ -670,8 +670,8 @@ def take_attn_mass(q, kv, indices, smax, ssum, scale, q_offset=0):
     exactly these inputs (same tensors, unchanged since), or None; the entry is used once.
 
     ``npu_sparse_flash_attention``'s backward forms P for every (row, head, slot) anyway, so
-    it keeps the mass (``bwd_sdp_kernel`` writes it; bitwise equal to ``dsa_attn_mass`` on
-    the same inputs) for the indexer KL op that a torch_npu-style layer calls next with the
+    it keeps the mass (``bwd_sdp_kernel`` writes it; equal to ``dsa_attn_mass`` on the same
+    inputs, bitwise unless tokens share workgroups) for the indexer KL op that a torch_npu-style layer calls next with the
     same query, key, indices and softmax statistics (reference converters/kernels/dsa.py:
     159-177 after :238-253).  The entry holds the index and statistics tensors it was made
     for (so their addresses cannot be reused while it lives; softmax statistics belong to
