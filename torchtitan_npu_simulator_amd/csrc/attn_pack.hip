@@ -41,7 +41,10 @@ pack_plan_kernel(const int32_t* __restrict__ indices, int S, int s_kv, int K, in
   uint32_t* mo = mask_out + ((int64_t)b * pk.groups + grp) * pk.tt * pk.words;
 
   for (int i = tid; i < nw + pk.tt * pk.words; i += kPlanThreads) lds[i] = 0u;
-  if (tid == 0) sh_dup = 0;
+  if (tid == 0) {
+    sh_dup = 0;
+    if (pk.suspect) pk.suspect[(int64_t)b * pk.groups + grp] = 0;
+  }
   __syncthreads();
   // every load of a batch is issued before the first use
   constexpr int kU = 8;
@@ -293,7 +296,7 @@ int pack_tokens(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64
 int64_t pack_plan_bytes(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int tt, bool backward) {
   const int64_t g = pack_groups(s_q, tt) * batch, cap = pack_cap(topk, tt);
   return al256(g * cap * 4) + al256(g * tt * (cap / 32) * 4) + al256(g * 4) +
-         (backward ? al256(batch * s_q * topk * 2) + al256(g * ((s_kv + 31) / 32) * 8) + al256(g * 4) : 0);
+         (backward ? al256(batch * s_q * topk * 2) + al256(g * ((s_kv + 31) / 32) * 8) + 2 * al256(g * 4) : 0);
 }
 
 int pack_plan_build(const int32_t* indices, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t topk,
@@ -319,6 +322,7 @@ int pack_plan_build(const int32_t* indices, int64_t batch, int64_t s_q, int64_t 
     pk.pos = (uint16_t*)take(batch * s_q * topk * 2);
     pk.sel = (uint2*)take(g * pk.key_words * 8);
     pk.distinct = (int32_t*)take(g * 4);
+    pk.suspect = (int32_t*)take(g * 4);
   }
   const int64_t nw = pk.key_words;
   const size_t lds = (size_t)(nw * 4 + (int64_t)tt * pk.words * 4 + (nw * 2 + 3) / 4 * 4);

@@ -602,8 +602,9 @@ bwd_dqk_kernel(const uint16_t* __restrict__ kv, const int32_t* __restrict__ idx,
     u32x4 av[2][2];
     read_kt(av[0], wt);
     // dS^T operands of the wave's two head groups.  No masking: the score kernel stores
-    // dS = P (dP - delta) with P = 0 exactly at every unusable slot and absent head, and the
-    // rows gathered for those slots (row 0) are finite, so they add exact zeros.
+    // dS = P (dP - delta) with P = 0 exactly at every unusable slot and absent head, which
+    // adds exact zeros while the row gathered for such a slot (row 0; packed, also the keys of
+    // the group's other tokens, see the epilogue) is finite.
     u32x4 bs[2][2];
 #pragma unroll
     for (int gg = 0; gg < 2; ++gg)
@@ -648,21 +649,72 @@ bwd_dqk_kernel(const uint16_t* __restrict__ kv, const int32_t* __restrict__ idx,
 #pragma unroll
     for (int gg = 0; gg < 2; ++gg) {
       int hd = 32 * (2 * hh2 + gg) + n;
+      bool put = hd < H, redo = false;
       if constexpr (kPack) {  // (token, head) of the row, as an offset of whole heads from the group's first
-        int t;
-        pack_row(pk, hd, t, hd);
-        if (t >= pk.tt || tok * pk.tt + t >= S || hd >= H) continue;
-        hd += t * H;
-      } else {
-        if (hd >= H) continue;
-      }
-      uint2* drow = reinterpret_cast<uint2*>(dq + (row_id * H + hd) * kD);
+        int t_;
+        pack_row(pk, hd, t_, hd);
+        put = t_ < pk.tt && tok * pk.tt + t_ < S && hd < H;
+        hd += t_ * H;
+        // a key of another token may have spoilt the row (attn_pack.h)
+        float nf = 0.f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        uint2 w;
-        w.x = pack_bf16x2(dqa[t][gg][4 * j], dqa[t][gg][4 * j + 1]);
-        w.y = pack_bf16x2(dqa[t][gg][4 * j + 2], dqa[t][gg][4 * j + 3]);
-        drow[(32 * dt + 8 * j + 4 * h) / 4] = w;
+        for (int v = 0; v < 16; ++v) nf = fmaf(dqa[t][gg][v], 0.f, nf);
+        nf = xor32_sum(nf);
+        redo = put && nf != nf;
+        if (nf != nf) pk.suspect[pgrp] = 1;  // (absent rows' too)
+      }
+      if (put && !redo) {
+        uint2* drow = reinterpret_cast<uint2*>(dq + (row_id * H + hd) * kD);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          uint2 w;
+          w.x = pack_bf16x2(dqa[t][gg][4 * j], dqa[t][gg][4 * j + 1]);
+          w.y = pack_bf16x2(dqa[t][gg][4 * j + 2], dqa[t][gg][4 * j + 3]);
+          drow[(32 * dt + 8 * j + 4 * h) / 4] = w;
+        }
+      }
+      if constexpr (kPack) {
+        // the tile's columns of those rows from their own slots, 16 rows of one token together:
+        // lane = column n, slots of parity h
+        const uint32_t flags = (uint32_t)__ballot(redo);  // (lanes 32 up repeat the rows)
+        for (int half = 0; half < 2; ++half) {
+          const uint32_t todo = flags >> (16 * half) & 0xffffu;
+          if (todo == 0u) continue;
+          const int hl = 32 * (2 * hh2 + gg) + 16 * half;
+          int t_, h0;
+          pack_row(pk, hl, t_, h0);
+          const pack_word* mt = pack_mask_token(pk, pgrp, t_);
+          const uint16_t* gcol = grow + 128 * (hl >> 6) + (hl & 63);
+          float acc[16];
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+          for (int w = 0; w < nblk; ++w) {
+            const uint32_t word = mt[w];
+            if (word == 0u) continue;
+            for (uint32_t bits = word & (h ? 0xaaaaaaaau : 0x55555555u); bits; bits &= bits - 1) {
+              const int slot = 32 * w + __builtin_ctz(bits);
+              const float k = bf16_to_f(kvb[(int64_t)ridx[slot] * kD + 32 * dt + n]);
+              const u32x4* g16 = reinterpret_cast<const u32x4*>(gcol + (int64_t)slot * kGW);
+              const u32x4 g0 = g16[0], g1 = g16[1];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                acc[2 * e] = fmaf(bf16_lo(g0[e]), k, acc[2 * e]);
+                acc[2 * e + 1] = fmaf(bf16_hi(g0[e]), k, acc[2 * e + 1]);
+                acc[8 + 2 * e] = fmaf(bf16_lo(g1[e]), k, acc[8 + 2 * e]);
+                acc[9 + 2 * e] = fmaf(bf16_hi(g1[e]), k, acc[9 + 2 * e]);
+              }
+            }
+            bool dead = true;  // (nothing left to find: a NaN of the rows' own everywhere)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) dead &= !(todo >> i & 1u) || acc[i] != acc[i];
+            if (__ballot(!dead) == 0) break;
+          }
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const float v = xor32_sum(acc[i]);
+            if (h == 0 && (todo >> i & 1u)) dq[((row_id + t_) * H + h0 + i) * kD + 32 * dt + n] = f_to_bf16(v);
+          }
+        }
       }
     }
   }
@@ -714,6 +766,7 @@ bwd_contrib_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ 
   constexpr int kKSteps = 4 * kHGroups;                // 32-row k steps of X (128 rows per head group)
   __shared__ u32x4 lds[2 * kGTChunks + 2 * kStChunks];  // X staging at start; then G tiles + C stages
   __shared__ int sh_last;
+  __shared__ int sh_odd;  // (packed) a value of Q is not finite
 
   const int lr = launch_row();  // local row in chunk
   const int tok = row0 + lr, b = blockIdx.y;
@@ -726,6 +779,7 @@ bwd_contrib_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ 
   int nblk;
   if constexpr (kPack) {
     nblk = (pk.count[pgrp] + kBN - 1) / kBN;
+    if (tid == 0) sh_odd = 0;  // (set past the first barrier below)
   } else {
     int vidx[kIdxU];
     load_row_indices(ridx, K, vidx);
@@ -808,6 +862,15 @@ bwd_contrib_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ 
 #pragma unroll
   for (int kc = 0; kc < 2 * kHGroups; ++kc) {
     __syncthreads();
+    if constexpr (kPack)
+      if ((kc & 1) == 0) {
+        uint32_t x = 0u;  // bit 15 or 31: an exponent of all ones
+#pragma unroll
+        for (int m = 0; m < kXPer; ++m)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) x |= (xraw[kc][m][r] & 0x7f807f80u) + 0x00800080u;
+        if (x & 0x80008000u) sh_odd = 1;
+      }
 #pragma unroll
     for (int m = 0; m < kXPer; ++m) {
       const int i = tid + kCThreads * m;
@@ -944,6 +1007,49 @@ bwd_contrib_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ 
   if (prev_s0 >= 0) {
 #pragma unroll
     for (int m = 0; m < kStSlices; ++m) store_rows(m, prev_s0, step - 1);
+  }
+  if constexpr (kPack) {
+    // (workgroup-uniform) a token's row may have spoilt the rows of keys it did not select.  A value
+    // of dS, P, dO or delta that is not finite shows in dQ (a dO row makes its whole dS row NaN,
+    // weights of 0 included), a Q row perhaps only in Q (a token without usable keys).
+    if (sh_odd || pk.suspect[pgrp]) {
+      __threadfence();
+      __syncthreads();  // the group's C rows are written
+      for (int i = tid; i < nslots * kRC; i += kCThreads) {
+        const int slot = i / kRC, c = i - slot * kRC;
+        u32x4* at = reinterpret_cast<u32x4*>(crow + (int64_t)slot * kD + 8 * c);
+        u32x4 v = *at;
+        uint32_t x = 0u;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x |= (v[r] & 0x7f807f80u) + 0x00800080u;
+        if (!(x & 0x80008000u)) continue;
+        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < pk.tt && tok * pk.tt + t < S; ++t) {  // the tokens that selected the slot
+          if (!(pk.mask[(pgrp * pk.tt + t) * pk.words + (slot >> 5)] >> (slot & 31) & 1u)) continue;
+          bool dead = true;
+#pragma unroll 4
+          for (int head = 0; head < H; ++head) {
+            const int hl = t * pk.hp + head;
+            const uint16_t* ge = grow + (int64_t)slot * kGW + 128 * (hl >> 6) + (hl & 63);
+            const float ds = bf16_to_f(ge[0]), p = bf16_to_f(ge[64]);
+            const int64_t hrow = (row_id + t) * H + head;
+            const u32x4 xq = *reinterpret_cast<const u32x4*>(q + hrow * kD + 8 * c);
+            const u32x4 xd = c < kDv / 8 ? *reinterpret_cast<const u32x4*>(dout + hrow * kDv + 8 * c) : (u32x4){0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              acc[2 * r] = fmaf(p, bf16_lo(xd[r]), fmaf(ds, bf16_lo(xq[r]), acc[2 * r]));
+              acc[2 * r + 1] = fmaf(p, bf16_hi(xd[r]), fmaf(ds, bf16_hi(xq[r]), acc[2 * r + 1]));
+            }
+          }
+#pragma unroll
+          for (int e = 0; e < 8; ++e) dead &= acc[e] != acc[e];
+          if (dead) break;  // (NaN whatever follows)
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = pack_bf16x2(acc[2 * r], acc[2 * r + 1]);
+        *at = v;
+      }
+    }
   }
 }
 

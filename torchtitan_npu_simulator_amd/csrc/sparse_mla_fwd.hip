@@ -396,7 +396,7 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
     hok = t < pk.tt && tk < S && head < H;
     orow = ((int64_t)b * S + tk) * H + head;
   }
-  if (!hok) return;
+  if (!kPack && !hok) return;  // (packed: the whole wave may redo rows below)
   if constexpr (kSplit) {
 #pragma unroll
     for (int dt = 0; dt < kDv / 32; ++dt)
@@ -414,17 +414,29 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
   const float sk2 = sinks ? sinks[head] * kLog2e : -INFINITY;
   const float den = sinks ? ls + exp2f(sk2 - m_ref) : ls;
   const float inv = den > 0.f ? 1.f / den : 0.f;
-  uint2* orp = reinterpret_cast<uint2*>(out + orow * kDv);
+  bool redo = false;
+  if constexpr (kPack) {  // a key of another token may have spoilt the row (attn_pack.h)
+    float nf = 0.f;
 #pragma unroll
-  for (int dt = 0; dt < kDv / 32; ++dt)
+    for (int dt = 0; dt < kDv / 32; ++dt)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      uint2 w;
-      w.x = pack_bf16x2(o[dt][4 * j] * inv, o[dt][4 * j + 1] * inv);
-      w.y = pack_bf16x2(o[dt][4 * j + 2] * inv, o[dt][4 * j + 3] * inv);
-      orp[(32 * dt + 8 * j + 4 * h) / 4] = w;
-    }
-  if (h == 0) {
+      for (int v = 0; v < 16; ++v) nf = fmaf(o[dt][v], 0.f, nf);
+    nf = xor32_sum(nf);
+    redo = hok && !clamped && nf != nf;
+  }
+  if ((!kPack || hok) && !redo) {
+    uint2* orp = reinterpret_cast<uint2*>(out + orow * kDv);
+#pragma unroll
+    for (int dt = 0; dt < kDv / 32; ++dt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        uint2 w;
+        w.x = pack_bf16x2(o[dt][4 * j] * inv, o[dt][4 * j + 1] * inv);
+        w.y = pack_bf16x2(o[dt][4 * j + 2] * inv, o[dt][4 * j + 3] * inv);
+        orp[(32 * dt + 8 * j + 4 * h) / 4] = w;
+      }
+  }
+  if ((!kPack || hok) && h == 0) {
     const float l_true = ls > 0.f ? ls * exp2f(m_ref - m_true) : 0.f;  // sum at the true max
     float m_out = m_true, l_out = l_true;
     if (sinks) {
@@ -434,6 +446,70 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
     smax[orow] = m_out * kLn2;
     // a negative sum marks a row whose logits outgrew the headroom; the fixup pass redoes it
     ssum[orow] = clamped ? -1.f : l_out;
+  }
+  if constexpr (kPack) {
+    // O of those rows from their own slots, with the weights of the pass above (the same
+    // reference, the same rounding of P): 16 rows of one token together, one key at a time,
+    // lane = columns 8 lane .. +7
+    const uint32_t flags = (uint32_t)__ballot(redo);  // (lanes 32 up repeat the rows)
+    for (int half = 0; half < 2; ++half) {
+      const uint32_t todo = flags >> (16 * half) & 0xffffu;
+      if (todo == 0u) continue;
+      int t, h0;
+      pack_row(pk, wave * 32 + 16 * half, t, h0);
+      const pack_word* mt = pack_mask_token(pk, pgrp, t);
+      const int64_t row0 = ((int64_t)b * S + grp * pk.tt + t) * H;
+      u32x4 q8[16];
+      float q1[16], ref[16], acc[16][8];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const uint16_t* qr_ = q + (row0 + min(h0 + i, H - 1)) * kD;
+        q8[i] = *reinterpret_cast<const u32x4*>(qr_ + 8 * lane);
+        q1[i] = kRope ? bf16_to_f(qr_[(kRope ? kDv : 0) + lane]) : 0.f;
+        const float m = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(m_ref), 16 * half + i));
+        ref[i] = m == -INFINITY ? 0.f : m;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[i][e] = 0.f;
+      }
+      for (int w = 0; w < nblk; ++w) {
+        const uint32_t word = mt[w];
+        if (word == 0u) continue;
+        for (uint32_t bits = word; bits; bits &= bits - 1) {
+          const uint16_t* kr = kvb + (int64_t)ridx[32 * w + __builtin_ctz(bits)] * kD;
+          const u32x4 k8 = *reinterpret_cast<const u32x4*>(kr + 8 * lane);
+          const float k1 = kRope ? bf16_to_f(kr[(kRope ? kDv : 0) + lane]) : 0.f;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            float dot = q1[i] * k1;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              dot = fmaf(bf16_hi(q8[i][e]), bf16_hi(k8[e]), fmaf(bf16_lo(q8[i][e]), bf16_lo(k8[e]), dot));
+            const float x = wave_sum(dot) * scale_log2;
+            const float p = bf16_to_f(f_to_bf16(__builtin_amdgcn_exp2f(fminf(x - ref[i], kHeadroom))));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              acc[i][2 * e] = fmaf(p, bf16_lo(k8[e]), acc[i][2 * e]);
+              acc[i][2 * e + 1] = fmaf(p, bf16_hi(k8[e]), acc[i][2 * e + 1]);
+            }
+          }
+        }
+        bool dead = true;  // (nothing left to find: every column is a NaN of the row's own)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (todo >> i & 1u)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) dead &= acc[i][e] != acc[i][e];
+        if (__ballot(!dead) == 0) break;
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float sc = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(inv), 16 * half + i));
+        u32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = pack_bf16x2(acc[i][2 * e] * sc, acc[i][2 * e + 1] * sc);
+        if (todo >> i & 1u) *reinterpret_cast<u32x4*>(out + (row0 + h0 + i) * kDv + 8 * lane) = v;
+      }
+    }
   }
 }
 
