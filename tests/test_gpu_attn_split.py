@@ -67,3 +67,52 @@ def test_split_forward_outgrown_headroom():
     q, kv = q.bfloat16(), kv.bfloat16()
     out, _, _ = ops.sparse_mla_fwd(q.cuda(), kv.cuda(), idx.cuda(), 1.0, q_offset=s_kv)
     assert rel_err(out, O.sparse_mla_fwd(q, kv, idx, 1.0, q_offset=s_kv)[0]) <= TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("where", ["query nan", "query inf", "query -inf", "key nan", "keys of the first half nan",
+                                   "keys of the first half -inf", "last key inf"])
+@pytest.mark.parametrize("sink", [False, True])
+def test_split_forward_not_finite(where, sink):
+    """Rows that are not finite come out of the merge as out of the one-workgroup kernel."""
+    from torchtitan_npu_simulator_amd import _lib
+    from torchtitan_npu_simulator_amd import torch_npu_ops as ops
+
+    H, K, s_kv, inf = 20, 512, 600, float("inf")
+    g = torch.Generator().manual_seed(5)
+    q = torch.randn(1, 2, H, 576, generator=g).bfloat16()
+    kv = torch.randn(1, s_kv, 576, generator=g).bfloat16()
+    idx = rand_indices(2, K, q_offset=s_kv - 2, seed=5)
+    first = idx[0, 0, : K // 2].long()
+    if where == "query nan":
+        q[0, 0, 3, 7] = float("nan")
+    elif where == "query inf":
+        q[0, 0, 3, 7] = inf
+    elif where == "query -inf":  # (every logit the same infinity)
+        kv[..., 9] = 1.0
+        q[0, 0, 3, 9], q[0, 0, 4, 9] = -inf, inf
+    elif where == "key nan":
+        kv[0, idx[0, 0, 300].long()] = float("nan")
+    elif where == "keys of the first half nan":
+        kv[0, first] = float("nan")
+    elif where == "keys of the first half -inf":
+        q[..., 9] = q[..., 9].abs() + 0.1
+        kv[0, first, 9] = -inf
+    else:
+        kv[0, idx[0, 0, K - 1].long(), 9] = inf
+    sinks = torch.randn(H, generator=g).cuda() if sink else None
+    qd, kvd, idd = q.cuda(), kv.cuda(), idx.cuda()
+    lib = _lib.load_library()
+    assert lib.dsa_sparse_mla_fwd_workspace_size(_lib.DSA_BF16, 1, 2, s_kv, H, K, s_kv - 2) > 0
+    got = ops.sparse_mla_fwd(qd, kvd, idd, 576 ** -0.5, q_offset=s_kv - 2, sinks=sinks)
+    one = [torch.empty_like(t) for t in got]
+    _lib.check(lib.dsa_sparse_mla_fwd_ws(
+        _lib.ptr(qd), _lib.ptr(kvd), _lib.ptr(idd), _lib.ptr(sinks), *(_lib.ptr(t) for t in one), _lib.DSA_BF16, 1, 2,
+        s_kv, H, 576, 512, K, 576 ** -0.5, s_kv - 2, None, 0, _lib.stream_of(qd.device)), "fwd")
+    for a, b in zip(got, one):
+        a, b = a.float(), b.float()
+        ok = torch.isfinite(b)
+        assert torch.equal(a[~ok].nan_to_num(2.0, 1.0, -1.0), b[~ok].nan_to_num(2.0, 1.0, -1.0))
+        # (where O is a NaN the sum holds the NaN logits' weights, which depend on the reference)
+        ok &= ~torch.isnan(one[0].float()).any(-1).reshape(ok.shape[:3] + (1,) * (ok.dim() - 3))
+        assert torch.allclose(a[ok], b[ok], rtol=2e-2, atol=2e-2)

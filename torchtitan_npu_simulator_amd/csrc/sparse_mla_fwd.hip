@@ -51,7 +51,8 @@ constexpr int kLatSteps = kDv / 16;            // 32 latent k-steps (Q in regist
 enum class FwdMode { kPlain, kPack, kSplit };
 
 // partial results of one row and split: O [512], then the reference max, the true max (base 2,
-// -inf: no key), the sum at the reference and whether a logit outgrew the headroom
+// -inf: no key, or no logit above -inf), the sum at the reference and a flag: 1, a logit outgrew
+// the headroom; -1, the split holds no block and left no O
 constexpr int kPartFloats = kDv + 4;
 
 template <int kD, FwdMode kMode>
@@ -132,7 +133,7 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
     const int b1 = __builtin_amdgcn_readfirstlane(nblk * (split + 1) / n_split);
     part += ((row_id * H + (hok ? head : 0)) * n_split + split) * kPartFloats;
     if (b1 == b0) {
-      if (hok && h == 0) *reinterpret_cast<float4*>(part + kDv) = make_float4(-INFINITY, -INFINITY, 0.f, 0.f);
+      if (hok && h == 0) *reinterpret_cast<float4*>(part + kDv) = make_float4(-INFINITY, -INFINITY, 0.f, -1.f);
       return;
     }
     bofs = b0;
@@ -515,7 +516,10 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
 
 // Merges the splits of a row (one wave per row, lane l = columns 8 l .. +7):
 //   O = sum_s 2^(m_s - M) O_s / (sum_s 2^(m_s - M) l_s + 2^(sink - M)),  M = max m_s,
-// in fp32, with the statistics as the one-pass epilogue writes them.
+// in fp32, with the statistics as the one-pass epilogue writes them.  Logits that are not finite
+// come out as there: a NaN logit weighs 2^kHeadroom whatever the reference is, so a split
+// of NaN logits alone (no reference, but a sum) counts as it is; a reference of +inf outweighs
+// every other split, and a split of logits of -inf alone adds 0 times its O.
 __global__ void __launch_bounds__(256)
 fwd_combine_kernel(const float* __restrict__ part, uint16_t* __restrict__ out, float* __restrict__ smax,
                    float* __restrict__ ssum, int64_t rows, int H, int n_split, const float* __restrict__ sinks) {
@@ -524,13 +528,17 @@ fwd_combine_kernel(const float* __restrict__ part, uint16_t* __restrict__ out, f
   if (row >= rows) return;
   const float* p = part + row * n_split * kPartFloats;
   // lane s holds split s's statistics (at most 64 splits)
-  float4 st = make_float4(-INFINITY, -INFINITY, 0.f, 0.f);
+  float4 st = make_float4(-INFINITY, -INFINITY, 0.f, -1.f);
   if (lane < n_split) st = *reinterpret_cast<const float4*>(p + (int64_t)lane * kPartFloats + kDv);
   const float M = wave_max(st.x), mt = wave_max(st.y);
   const float sk2 = sinks ? sinks[row % H] * kLog2e : -INFINITY;
-  const float w = st.x == -INFINITY ? 0.f : exp2f(st.x - M);
+  const float w = st.x == -INFINITY ? (st.z > 0.f ? 1.f : 0.f) : st.x == M ? 1.f : exp2f(st.x - M);
   const float ls = wave_sum(w * st.z);
-  const bool clamped = __ballot(st.w != 0.f) != 0;
+  const uint64_t held = __ballot(st.w >= 0.f);
+  // (the one pass takes its reference from the first logits: a later one of +inf outgrows it)
+  const uint64_t ref = __ballot(st.x != -INFINITY);
+  const float first = ref ? __shfl(st.x, __builtin_ctzll(ref), 64) : M;
+  const bool clamped = __ballot(st.w > 0.f) != 0 || (M == INFINITY && first != INFINITY);
   // (no key: M = -inf, every weight and O are 0, and a sink makes the denominator infinite)
   const float den = sinks ? ls + exp2f(sk2 - M) : ls;
   const float inv = den > 0.f ? 1.f / den : 0.f;
@@ -546,8 +554,8 @@ fwd_combine_kernel(const float* __restrict__ part, uint16_t* __restrict__ out, f
     }
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
-      const float ws = s0 + u < n_split ? __shfl(w, s0 + u, 64) : 0.f;
-      if (ws == 0.f) continue;  // (wave-uniform: a split without keys left no O)
+      const float ws = __shfl(w, s0 + u, 64);  // (s0 + u < 64)
+      if (!(held >> (s0 + u) & 1u)) continue;  // (wave-uniform: a split without keys left no O)
 #pragma unroll
       for (int r = 0; r < 8; ++r) acc[r] = fmaf(ws, x[u][r >> 2][r & 3], acc[r]);
     }
