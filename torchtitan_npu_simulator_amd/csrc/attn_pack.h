@@ -19,6 +19,7 @@
 //                     the last to the end of its 32-slot block;
 //   mask[tt][words]   bit j of word j / 32: slot j of idx is selected by the token;
 //   count             used slots;
+//   redo[4]           (cleared by the plan) the rows whose O the forward found not finite, as bits;
 //   pos[tt][K]        (backward) the slot of the token's j-th selection, kPackNoSlot if
 //                     unusable;
 //   sel[word]         (backward, stored word-major over the groups) the union's keys
@@ -33,10 +34,12 @@
 // is a NaN: a row that is not finite would reach every token of its group (earlier tokens,
 // other sequences of a packed batch).  Every sum over the union is therefore looked at once
 // it is complete, and where it is not finite it is formed again from the token's own slots
-// alone (the forward's and bwd_dqk_kernel's epilogues, the end of bwd_contrib_kernel where
-// the group is suspect).  S = 4096, 16 heads, top-2048, forward + backward: the look costs
-// 1.631 -> 1.639 ms; with one NaN key that half of the tokens select the sums again take
-// 17 ms (forward) and 19 ms (backward), with every key NaN 0.5 and 3 ms.
+// alone (O by the forward's fixup pass, dQ in bwd_dqk_kernel's epilogue, dKV at the end of
+// bwd_contrib_kernel where the group is suspect).  The look takes 2 us of 430 in the forward
+// kernel and in the backward's (6080 tokens, 32 heads, top-1024); S = 4096, 16 heads,
+// top-2048 with one NaN key that half of the tokens select: the sums again take 7 ms
+// (forward; formed in the kernel's own epilogue 17 ms, and 3 % of its time on finite data for
+// the registers) and 19 ms (backward).
 #pragma once
 #include "dsa_common.h"
 
@@ -50,6 +53,7 @@ struct PackView {
   const int32_t* idx = nullptr;    // [batch][groups][cap]
   const uint32_t* mask = nullptr;  // [batch][groups][tt][words]
   const int32_t* count = nullptr;  // [batch][groups]
+  uint32_t* redo = nullptr;        // [batch][groups][4]
   uint16_t* pos = nullptr;         // [batch][S][K], backward only as the next two
   uint2* sel = nullptr;            // [batch][key words][groups]
   int32_t* distinct = nullptr;     // [batch][groups]

@@ -41,6 +41,7 @@ pack_plan_kernel(const int32_t* __restrict__ indices, int S, int s_kv, int K, in
   uint32_t* mo = mask_out + ((int64_t)b * pk.groups + grp) * pk.tt * pk.words;
 
   for (int i = tid; i < nw + pk.tt * pk.words; i += kPlanThreads) lds[i] = 0u;
+  if (tid < 4) pk.redo[((int64_t)b * pk.groups + grp) * 4 + tid] = 0u;
   if (tid == 0) {
     sh_dup = 0;
     if (pk.suspect) pk.suspect[(int64_t)b * pk.groups + grp] = 0;
@@ -295,7 +296,7 @@ int pack_tokens(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64
 
 int64_t pack_plan_bytes(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int tt, bool backward) {
   const int64_t g = pack_groups(s_q, tt) * batch, cap = pack_cap(topk, tt);
-  return al256(g * cap * 4) + al256(g * tt * (cap / 32) * 4) + al256(g * 4) +
+  return al256(g * cap * 4) + al256(g * tt * (cap / 32) * 4) + al256(g * 4) + al256(g * 16) +
          (backward ? al256(batch * s_q * topk * 2) + al256(g * ((s_kv + 31) / 32) * 8) + 2 * al256(g * 4) : 0);
 }
 
@@ -318,6 +319,7 @@ int pack_plan_build(const int32_t* indices, int64_t batch, int64_t s_q, int64_t 
   int32_t* idx = (int32_t*)take(g * pk.cap * 4);
   uint32_t* mask = (uint32_t*)take(g * tt * pk.words * 4);
   int32_t* count = (int32_t*)take(g * 4);
+  pk.redo = (uint32_t*)take(g * 16);
   if (backward) {
     pk.pos = (uint16_t*)take(batch * s_q * topk * 2);
     pk.sel = (uint2*)take(g * pk.key_words * 8);

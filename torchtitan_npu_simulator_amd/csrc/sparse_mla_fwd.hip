@@ -397,7 +397,7 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
     hok = t < pk.tt && tk < S && head < H;
     orow = ((int64_t)b * S + tk) * H + head;
   }
-  if (!kPack && !hok) return;  // (packed: the whole wave may redo rows below)
+  if (!kPack && !hok) return;
   if constexpr (kSplit) {
 #pragma unroll
     for (int dt = 0; dt < kDv / 32; ++dt)
@@ -412,32 +412,28 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
   // the row's denominator: O = acc / (ls + 2^(sink2 - m_ref)), and the row statistics
   // become (m2, s2) = (max(m, sink), sum e^(x - m2) + e^(sink - m2)); with no valid key
   // (m_ref = -inf) the sink term is +inf and O stays 0
-  const float sk2 = sinks ? sinks[head] * kLog2e : -INFINITY;
+  const float sk2 = sinks ? sinks[hok ? head : 0] * kLog2e : -INFINITY;
   const float den = sinks ? ls + exp2f(sk2 - m_ref) : ls;
   const float inv = den > 0.f ? 1.f / den : 0.f;
-  bool redo = false;
-  if constexpr (kPack) {  // a key of another token may have spoilt the row (attn_pack.h)
-    float nf = 0.f;
+  float nf = 0.f;  // (packed) 0, or a NaN
+  const bool put = !kPack || hok;
+  uint2* orp = reinterpret_cast<uint2*>(out + orow * kDv);
 #pragma unroll
-    for (int dt = 0; dt < kDv / 32; ++dt)
+  for (int dt = 0; dt < kDv / 32; ++dt)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) nf = fmaf(o[dt][v], 0.f, nf);
+    for (int j = 0; j < 4; ++j) {
+      uint2 w;
+      w.x = pack_bf16x2(o[dt][4 * j] * inv, o[dt][4 * j + 1] * inv);
+      w.y = pack_bf16x2(o[dt][4 * j + 2] * inv, o[dt][4 * j + 3] * inv);
+      if constexpr (kPack) nf = bf16x2_dot(w.y, 0u, bf16x2_dot(w.x, 0u, nf));
+      if (put) orp[(32 * dt + 8 * j + 4 * h) / 4] = w;
+    }
+  if constexpr (kPack) {  // a key of another token may have spoilt the row (attn_pack.h): the fixup pass redoes it
     nf = xor32_sum(nf);
-    redo = hok && !clamped && nf != nf;
+    const uint32_t redo = (uint32_t)__ballot(hok && nf != nf);  // (lanes 32 up repeat the rows)
+    if (redo != 0u && lane == 0) pk.redo[pgrp * 4 + wave] = redo;
   }
-  if ((!kPack || hok) && !redo) {
-    uint2* orp = reinterpret_cast<uint2*>(out + orow * kDv);
-#pragma unroll
-    for (int dt = 0; dt < kDv / 32; ++dt)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        uint2 w;
-        w.x = pack_bf16x2(o[dt][4 * j] * inv, o[dt][4 * j + 1] * inv);
-        w.y = pack_bf16x2(o[dt][4 * j + 2] * inv, o[dt][4 * j + 3] * inv);
-        orp[(32 * dt + 8 * j + 4 * h) / 4] = w;
-      }
-  }
-  if ((!kPack || hok) && h == 0) {
+  if (put && h == 0) {
     const float l_true = ls > 0.f ? ls * exp2f(m_ref - m_true) : 0.f;  // sum at the true max
     float m_out = m_true, l_out = l_true;
     if (sinks) {
@@ -447,70 +443,6 @@ sparse_mla_fwd_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __res
     smax[orow] = m_out * kLn2;
     // a negative sum marks a row whose logits outgrew the headroom; the fixup pass redoes it
     ssum[orow] = clamped ? -1.f : l_out;
-  }
-  if constexpr (kPack) {
-    // O of those rows from their own slots, with the weights of the pass above (the same
-    // reference, the same rounding of P): 16 rows of one token together, one key at a time,
-    // lane = columns 8 lane .. +7
-    const uint32_t flags = (uint32_t)__ballot(redo);  // (lanes 32 up repeat the rows)
-    for (int half = 0; half < 2; ++half) {
-      const uint32_t todo = flags >> (16 * half) & 0xffffu;
-      if (todo == 0u) continue;
-      int t, h0;
-      pack_row(pk, wave * 32 + 16 * half, t, h0);
-      const pack_word* mt = pack_mask_token(pk, pgrp, t);
-      const int64_t row0 = ((int64_t)b * S + grp * pk.tt + t) * H;
-      u32x4 q8[16];
-      float q1[16], ref[16], acc[16][8];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const uint16_t* qr_ = q + (row0 + min(h0 + i, H - 1)) * kD;
-        q8[i] = *reinterpret_cast<const u32x4*>(qr_ + 8 * lane);
-        q1[i] = kRope ? bf16_to_f(qr_[(kRope ? kDv : 0) + lane]) : 0.f;
-        const float m = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(m_ref), 16 * half + i));
-        ref[i] = m == -INFINITY ? 0.f : m;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[i][e] = 0.f;
-      }
-      for (int w = 0; w < nblk; ++w) {
-        const uint32_t word = mt[w];
-        if (word == 0u) continue;
-        for (uint32_t bits = word; bits; bits &= bits - 1) {
-          const uint16_t* kr = kvb + (int64_t)ridx[32 * w + __builtin_ctz(bits)] * kD;
-          const u32x4 k8 = *reinterpret_cast<const u32x4*>(kr + 8 * lane);
-          const float k1 = kRope ? bf16_to_f(kr[(kRope ? kDv : 0) + lane]) : 0.f;
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            float dot = q1[i] * k1;
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              dot = fmaf(bf16_hi(q8[i][e]), bf16_hi(k8[e]), fmaf(bf16_lo(q8[i][e]), bf16_lo(k8[e]), dot));
-            const float x = wave_sum(dot) * scale_log2;
-            const float p = bf16_to_f(f_to_bf16(__builtin_amdgcn_exp2f(fminf(x - ref[i], kHeadroom))));
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              acc[i][2 * e] = fmaf(p, bf16_lo(k8[e]), acc[i][2 * e]);
-              acc[i][2 * e + 1] = fmaf(p, bf16_hi(k8[e]), acc[i][2 * e + 1]);
-            }
-          }
-        }
-        bool dead = true;  // (nothing left to find: every column is a NaN of the row's own)
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (todo >> i & 1u)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) dead &= acc[i][e] != acc[i][e];
-        if (__ballot(!dead) == 0) break;
-      }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float sc = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(inv), 16 * half + i));
-        u32x4 v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = pack_bf16x2(acc[i][2 * e] * sc, acc[i][2 * e + 1] * sc);
-        if (todo >> i & 1u) *reinterpret_cast<u32x4*>(out + (row0 + h0 + i) * kDv + 8 * lane) = v;
-      }
-    }
   }
 }
 
@@ -843,15 +775,76 @@ __device__ __forceinline__ float ld_elem(const uint16_t* p, int64_t i) { return 
 __device__ __forceinline__ void st_elem(float* p, int64_t i, float v) { p[i] = v; }
 __device__ __forceinline__ void st_elem(uint16_t* p, int64_t i, float v) { p[i] = f_to_bf16(v); }
 
+// O of a token's heads whose bits from `row0` on are set in redo (and whose logits kept to the
+// headroom), from the token's own slots: a wave takes kN heads and one key at a time, lane =
+// latent columns 8 lane .. +7 and rope column lane.  The statistics hold, as no other token's
+// key ever entered them; weights and products that are not finite come out as in the MFMA kernels.
+__device__ void redo_rows(const uint16_t* q, const uint16_t* kvb, const int32_t* ridx, uint16_t* out, const float* smax,
+                          const float* ssum, int s_kv, int H, int K, int dqk, float scale, int64_t limit,
+                          const uint32_t* redo, int row0) {
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const bool rope = dqk > kDv;
+  constexpr int kN = 2;  // (few registers: the kernel's other workgroups leave at once, eight to a CU)
+  for (int h0 = kN * wave; h0 < H; h0 += 4 * kN) {
+    u32x4 q8[kN];
+    float q1[kN], ref[kN], acc[kN][8];
+    uint32_t todo = 0u;
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+      const int hd = min(h0 + i, H - 1), r = row0 + hd;
+      if (h0 + i < H && (redo[r >> 5] >> (r & 31) & 1u) && !(ssum[hd] < 0.f)) todo |= 1u << i;
+      q8[i] = *reinterpret_cast<const u32x4*>(q + (int64_t)hd * dqk + 8 * lane);
+      q1[i] = rope ? bf16_to_f(q[(int64_t)hd * dqk + kDv + lane]) : 0.f;
+      const float m = smax[hd] * kLog2e;
+      ref[i] = m == -INFINITY ? 0.f : m;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[i][e] = 0.f;
+    }
+    todo = __builtin_amdgcn_readfirstlane(todo);
+    if (todo == 0u) continue;
+    for (int j0 = 0; j0 < K; j0 += 64) {
+      const int key = j0 + lane < K ? ridx[j0 + lane] : -1;
+      for (uint64_t m = __ballot(slot_ok(key, s_kv, limit)); m; m &= m - 1) {
+        const uint16_t* kr = kvb + (int64_t)__builtin_amdgcn_readlane(key, __builtin_ctzll(m)) * dqk;
+        const u32x4 k8 = *reinterpret_cast<const u32x4*>(kr + 8 * lane);
+        const float k1 = rope ? bf16_to_f(kr[kDv + lane]) : 0.f;
+#pragma unroll
+        for (int i = 0; i < kN; ++i) {
+          float dot = q1[i] * k1;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            dot = fmaf(bf16_hi(q8[i][e]), bf16_hi(k8[e]), fmaf(bf16_lo(q8[i][e]), bf16_lo(k8[e]), dot));
+          const float p = exp2f(fminf(wave_sum(dot) * scale * kLog2e - ref[i], kHeadroom));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            acc[i][2 * e] = fmaf(p, bf16_lo(k8[e]), acc[i][2 * e]);
+            acc[i][2 * e + 1] = fmaf(p, bf16_hi(k8[e]), acc[i][2 * e + 1]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kN; ++i)
+      if (todo >> i & 1u) {
+        const float l = ssum[h0 + i], inv = l > 0.f ? 1.f / l : 0.f;
+        u32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = pack_bf16x2(acc[i][2 * e] * inv, acc[i][2 * e + 1] * inv);
+        *reinterpret_cast<u32x4*>(out + (int64_t)(h0 + i) * kDv + 8 * lane) = v;
+      }
+  }
+}
+
 // Exact path (any D, fp32 arithmetic): one workgroup per (token, head).  Serves fp32
 // inputs and, in fixup mode (one workgroup per token, heads looped), recomputes the rows
 // the MFMA kernel flagged with a negative softmax_sum.  Scores are staged in dynamic LDS.
+// In fixup mode over packed tokens (pk.redo) it also redoes the rows flagged there.
 template <typename T>
 __global__ void __launch_bounds__(256)
 sparse_mla_fwd_exact_kernel(const T* __restrict__ q, const T* __restrict__ kv, const int32_t* __restrict__ idx,
                             T* __restrict__ out, float* __restrict__ smax, float* __restrict__ ssum, int S,
                             int s_kv, int H, int K, int dqk, int dv, float scale, int64_t q_offset, int fixup,
-                            const float* __restrict__ sinks) {
+                            const float* __restrict__ sinks, PackView pk) {
   extern __shared__ float sc[];
   __shared__ float red[256];
   const int tok = blockIdx.x, b = blockIdx.z, tid = threadIdx.x;
@@ -863,7 +856,16 @@ sparse_mla_fwd_exact_kernel(const T* __restrict__ q, const T* __restrict__ kv, c
   if (fixup) {  // one parallel test of the row's flags: almost every row has none
     bool any = false;
     for (int hh = tid; hh < H; hh += 256) any |= ssum[row_id * H + hh] < 0.f;
+    const uint32_t* redo = nullptr;  // of the token's group
+    if constexpr (sizeof(T) == 2)
+      if (pk.redo) {
+        redo = pk.redo + ((int64_t)b * pk.groups + tok / pk.tt) * 4;
+        any |= tid < 4 && redo[tid] != 0u;
+      }
     if (!__syncthreads_or(any)) return;
+    if constexpr (sizeof(T) == 2)
+      if (redo) redo_rows(q + row_id * H * dqk, kvb, ridx, out + row_id * H * dv, smax + row_id * H, ssum + row_id * H, s_kv, H,
+                          K, dqk, scale, limit, redo, tok % pk.tt * pk.hp);
   }
   for (int head = h0; head < h1; ++head) {
     const int64_t hr = row_id * H + head;
@@ -1128,7 +1130,7 @@ static int sparse_mla_fwd_impl(const void* q, const void* kv, const int32_t* ind
     const TimedLaunch tl("sparse_mla_fwd_exact_kernel<fixup>", st);
     sparse_mla_fwd_exact_kernel<uint16_t><<<fgrid, 256, sc_bytes, st>>>(
         (const uint16_t*)q, (const uint16_t*)kv, indices, (uint16_t*)out, softmax_max, softmax_sum, (int)s_q,
-        (int)s_kv, (int)n_heads, (int)topk, (int)d_qk, (int)d_v, scale, q_offset, 1, sinks);
+        (int)s_kv, (int)n_heads, (int)topk, (int)d_qk, (int)d_v, scale, q_offset, 1, sinks, pk);
     return check_launch("dsa_sparse_mla_fwd(bf16 fixup)");
   }
   if (dtype == DSA_F32) {
@@ -1139,7 +1141,7 @@ static int sparse_mla_fwd_impl(const void* q, const void* kv, const int32_t* ind
     const TimedLaunch tl("sparse_mla_fwd_exact_kernel<float>", st);
     sparse_mla_fwd_exact_kernel<float><<<grid, 256, sc_bytes, st>>>(
         (const float*)q, (const float*)kv, indices, (float*)out, softmax_max, softmax_sum, (int)s_q, (int)s_kv,
-        (int)n_heads, (int)topk, (int)d_qk, (int)d_v, scale, q_offset, 0, sinks);
+        (int)n_heads, (int)topk, (int)d_qk, (int)d_v, scale, q_offset, 0, sinks, PackView{});
     return check_launch("dsa_sparse_mla_fwd(f32)");
   }
   return set_error(DSA_ERR_UNSUPPORTED, "dsa_sparse_mla_fwd: dtype %d not supported", dtype);
