@@ -15,8 +15,8 @@
 // A group of tt tokens has rows (token, head) at lane row hp * token + head, hp = the head
 // count rounded up to 16.  Its plan is
 //   idx[cap]          the union's keys in ascending order (a key repeated inside one token's
-//                     list appears again at the end, once per extra occurrence), -1 from
-//                     the last to the end of its 32-slot block;
+//                     list appears again at the end, once per extra occurrence, these by key
+//                     and token), -1 from the last to the end of its 32-slot block;
 //   mask[tt][words]   bit j of word j / 32: slot j of idx is selected by the token;
 //   count             used slots;
 //   redo[4]           (cleared by the plan) the rows whose O the forward found not finite, as bits;

@@ -5,6 +5,7 @@
 // scan of the words' bit counts gives every key its slot.  Bound by the two reads of the
 // group's index rows and by the LDS atomics (one per selection and pass).
 #include <algorithm>
+#include <type_traits>
 
 #include "attn_pack.h"
 
@@ -14,23 +15,31 @@ namespace {
 constexpr int kPlanThreads = 512;
 constexpr int kPlanWaves = kPlanThreads / 64;
 constexpr uint32_t kRepeats = 0x80000000u;    // (PackView::sel) the group has repeated slots
-constexpr int64_t kPackMaxKeys = 1 << 17;     // bitmap and word offsets: 24 KB of LDS
+constexpr int64_t kPackMaxKeys = 1 << 17;     // bitmap and word offsets: 24 KB of LDS; 8 v + t of a repeat in 31 bits
 constexpr int64_t kPackMaxMaskWords = 9216;   // 36 KB of LDS
+constexpr int64_t kPlanLds = 63 * 1024;       // dynamic LDS of the plan: the above and room to sort repeats
+constexpr int64_t kSortMax = 4096;
+static_assert(kPackMaxKeys / 32 * 6 + kPackMaxMaskWords * 4 <= kPlanLds, "the plan fits without a sort buffer");
 
 __device__ __forceinline__ bool plan_slot_ok(int v, int s_kv, int64_t limit) {
   return v >= 0 && v < s_kv && (int64_t)v <= limit;
 }
 
+// pairs of a bitonic merge over n elements (half the next power of two)
+__device__ __forceinline__ int len_pairs(int n) { return n > 1 ? 1 << (31 - __clz(n - 1)) : 0; }
+
 __global__ void __launch_bounds__(kPlanThreads)
 pack_plan_kernel(const int32_t* __restrict__ indices, int S, int s_kv, int K, int64_t q_offset, PackView pk,
-                 int32_t* __restrict__ idx_out, uint32_t* __restrict__ mask_out, int32_t* __restrict__ count_out) {
+                 int32_t* __restrict__ idx_out, uint32_t* __restrict__ mask_out, int32_t* __restrict__ count_out,
+                 int sort_cap) {
   extern __shared__ uint32_t lds[];
   __shared__ int wsum[kPlanWaves];
-  __shared__ int sh_dup, sh_n;
+  __shared__ int sh_rep;  // repeats found
   const int nw = (s_kv + 31) >> 5;
   uint32_t* bits = lds;                      // [nw] keys of the union
   uint32_t* mk = lds + nw;                   // [tt][words]
   uint16_t* pre = reinterpret_cast<uint16_t*>(mk + pk.tt * pk.words);  // [nw] slots before the word
+  int32_t* srt = reinterpret_cast<int32_t*>(mk + pk.tt * pk.words + (nw + 1) / 2);  // [sort_cap] repeats
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int grp = (int)(gridDim.x - 1u - blockIdx.x), b = blockIdx.y;  // longest rows first
   const int tok0 = grp * pk.tt, nt = min(pk.tt, S - tok0);
@@ -43,7 +52,7 @@ pack_plan_kernel(const int32_t* __restrict__ indices, int S, int s_kv, int K, in
   for (int i = tid; i < nw + pk.tt * pk.words; i += kPlanThreads) lds[i] = 0u;
   if (tid < 4) pk.redo[((int64_t)b * pk.groups + grp) * 4 + tid] = 0u;
   if (tid == 0) {
-    sh_dup = 0;
+    sh_rep = 0;
     if (pk.suspect) pk.suspect[(int64_t)b * pk.groups + grp] = 0;
   }
   __syncthreads();
@@ -109,39 +118,60 @@ pack_plan_kernel(const int32_t* __restrict__ indices, int S, int s_kv, int K, in
     if (ok) {
       p = slot_of(v);
       const uint32_t bit = 1u << (p & 31);
-      if (atomicOr(&mk[t * pk.words + (p >> 5)], bit) & bit) sh_dup = 1;
+      if (atomicOr(&mk[t * pk.words + (p >> 5)], bit) & bit) io[n + atomicAdd(&sh_rep, 1)] = 8 * v + t;
     }
     if (pk.pos) pk.pos[row0 * K + e] = ok ? (uint16_t)p : kPackNoSlot;
   });
   __syncthreads();
-  if (sh_dup) {
-    // some token lists a key more than once (top-k output never does): one thread walks the
-    // lists in order and gives every repeat its own slot after the union, so the slots do
-    // not depend on the order in which the threads ran (pos keeps the key's first slot,
-    // whose probability is the repeat's too)
-    for (int i = tid; i < pk.tt * pk.words; i += kPlanThreads) mk[i] = 0u;
-    __syncthreads();
-    if (tid == 0) {
-      int m = n;
-      for (int t = 0; t < nt; ++t)
-        for (int j = 0; j < K; ++j) {
-          const int v = src[t * K + j];
-          if (!plan_slot_ok(v, s_kv, (int64_t)(tok0 + t) + q_offset)) continue;
-          int p = slot_of(v);
-          if (mk[t * pk.words + (p >> 5)] >> (p & 31) & 1u) {
-            p = m++;
-            io[p] = v;
+  const int rep = sh_rep;
+  if (rep > 0) {
+    // some token lists a key more than once (top-k output never does).  Every further occurrence
+    // takes a slot of its own after the union, ordered by key and token, so the slots do not
+    // depend on the order in which the threads ran (pos keeps the key's first slot, whose
+    // probability is the repeat's too), and a key's reduction finds its run.  A bitonic sort
+    // in place, every comparison ascending (the first step of a merge pairs mirrored
+    // elements), so places past the last one count as +inf; in LDS where they fit.  1024 tokens,
+    // 16 heads, 256 keys drawn with replacement: forward 330 us with one thread that walked
+    // the lists, 116 now (distinct keys: 82).
+    int32_t* ex = io + n;
+    auto sort = [&](auto* x) __attribute__((always_inline)) {
+      for (int len = 2; len < 2 * rep; len <<= 1)
+        for (int j = len >> 1; j > 0; j >>= 1) {
+          const bool mirror = 2 * j == len;
+          for (int i = tid; i < len_pairs(rep); i += kPlanThreads) {
+            const int o = i & (j - 1), base = 2 * (i - o);
+            const int lo = base + o, hi = mirror ? base + 2 * j - 1 - o : lo + j;
+            if (hi < rep) {
+              const int u = x[lo], w = x[hi];
+              if (u > w) {
+                x[lo] = w;
+                x[hi] = u;
+              }
+            }
           }
-          mk[t * pk.words + (p >> 5)] |= 1u << (p & 31);
+          __syncthreads();
         }
-      sh_n = m;
+    };
+    auto give = [&](int i, int x) {  // the i-th repeat's slot
+      const int t = x & 7, p = n + i;
+      ex[i] = x >> 3;
+      atomicOr(&mk[t * pk.words + (p >> 5)], 1u << (p & 31));
+    };
+    if (rep <= sort_cap) {  // in LDS
+      for (int i = tid; i < rep; i += kPlanThreads) srt[i] = ex[i];
+      __syncthreads();
+      sort(srt);
+      for (int i = tid; i < rep; i += kPlanThreads) give(i, srt[i]);
+    } else {
+      sort(ex);
+      for (int i = tid; i < rep; i += kPlanThreads) give(i, ex[i]);
     }
     __syncthreads();
     if (pk.sel)
       for (int w = tid; w < nw; w += kPlanThreads)
         pk.sel[((int64_t)b * nw + w) * pk.groups + grp] = make_uint2(bits[w], (uint32_t)pre[w] | kRepeats);
     if (pk.distinct && tid == 0) pk.distinct[(int64_t)b * pk.groups + grp] = n;
-    n = sh_n;
+    n += rep;
   }
   const int used = (n + 31) >> 5;
   for (int i = tid; i < pk.tt * used; i += kPlanThreads) {
@@ -198,14 +228,20 @@ pack_dkv_reduce_kernel(PackView pk, const uint16_t* __restrict__ cbuf, float* __
       a[2 * r + 1] += bf16_hi(v[r]);
     }
   };
-  bool any = false;
-  for (int gb = n0; gb < n1; gb += 64) {
-    const uint2 e = gb + lane < n1 ? sel[gb + lane] : make_uint2(0u, 0u);
-    const int slot = (int)(e.y & ~kRepeats) + __popc(e.x & (bit - 1u));
-    uint64_t m = __ballot((e.x & bit) != 0u);
-    any |= m != 0;
+  auto add8_times = [](float (&a)[8], const u32x4& v, float x) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      a[2 * r] = fmaf(x, bf16_lo(v[r]), a[2 * r]);
+      a[2 * r + 1] = fmaf(x, bf16_hi(v[r]), a[2 * r + 1]);
+    }
+  };
+  // adds, for every lane g of m, the row of group gb + g at that lane's slot (that lane's `times`
+  // times), in order, kRows rows in flight
+  auto add_rows = [&](uint64_t m, int gb, int slot, auto timed, float times) __attribute__((always_inline)) {
+    constexpr bool kTimed = decltype(timed)::value;
     while (m) {
       u32x4 v[kRows], w[kRows];
+      float x[kRows];
       int cnt = 0, g = 0;
 #pragma unroll
       for (int u = 0; u < kRows; ++u) {
@@ -215,6 +251,7 @@ pack_dkv_reduce_kernel(PackView pk, const uint16_t* __restrict__ cbuf, float* __
           ++cnt;
         }
         const uint16_t* row = cb + ((int64_t)(gb + g) * pk.cap + __builtin_amdgcn_readlane(slot, g)) * kWidth;
+        if constexpr (kTimed) x[u] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(times), g));
         v[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + 8 * lane));
         if constexpr (kChunks == 72)
           w[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + 512 + 8 * (lane & 7)));
@@ -222,21 +259,51 @@ pack_dkv_reduce_kernel(PackView pk, const uint16_t* __restrict__ cbuf, float* __
 #pragma unroll
       for (int u = 0; u < kRows; ++u)
         if (u < cnt) {
-          add8(acc, v[u]);
-          if constexpr (kChunks == 72) add8(acc2, w[u]);
+          if constexpr (kTimed) {
+            add8_times(acc, v[u], x[u]);
+            if constexpr (kChunks == 72) add8_times(acc2, w[u], x[u]);
+          } else {
+            add8(acc, v[u]);
+            if constexpr (kChunks == 72) add8(acc2, w[u]);
+          }
         }
     }
-    uint64_t rep = __ballot((e.y & kRepeats) != 0u);
-    while (rep) {  // groups with repeated keys: their slots after the union, in order
-      const int g = __builtin_ctzll(rep);
-      rep &= rep - 1;
-      const int64_t pg = (int64_t)b * pk.groups + g0 + gb + g;
-      for (int j = pk.distinct[pg]; j < pk.count[pg]; ++j)
-        if (pk.idx[pg * pk.cap + j] == k) {
-          const uint16_t* row = cb + ((int64_t)(gb + g) * pk.cap + j) * kWidth;
-          add8(acc, *reinterpret_cast<const u32x4*>(row + 8 * lane));
-          if constexpr (kChunks == 72) add8(acc2, *reinterpret_cast<const u32x4*>(row + 512 + 8 * (lane & 7)));
-        }
+  };
+  bool any = false;
+  for (int gb = n0; gb < n1; gb += 64) {
+    const uint2 e = gb + lane < n1 ? sel[gb + lane] : make_uint2(0u, 0u);
+    const int slot = (int)(e.y & ~kRepeats) + __popc(e.x & (bit - 1u));
+    uint64_t m = __ballot((e.x & bit) != 0u);
+    any |= m != 0;
+    add_rows(m, gb, slot, std::false_type{}, 1.f);
+    if (__ballot((e.y & kRepeats) != 0u) == 0) continue;
+    // groups with repeated keys: each lane finds the key's run among its group's slots after the
+    // union (ordered by key and token), and in it the slots of one token after the other, whose
+    // rows are the same: one is read, times their number.  (A walk over every repeat for every
+    // key: backward of 2048 tokens, 16 heads, 1024 keys of which half are key 0 218 ms, now 1.8;
+    // 4096 tokens with 512 keys drawn with replacement 50 -> 1.7 ms; distinct keys 1.0.)
+    const int64_t pg = (int64_t)b * pk.groups + g0 + min(gb + lane, n - 1);
+    const int32_t* list = pk.idx + pg * pk.cap;
+    auto first = [&](int a, int z, auto&& before) {  // the first slot of [a, z) that is not `before`
+      while (a < z) {
+        const int mid = (a + z) >> 1;
+        if (before(mid)) a = mid + 1;
+        else z = mid;
+      }
+      return a;
+    };
+    int lo = 0, hi = 0;
+    if (e.y & kRepeats) {
+      const int end = pk.count[pg];
+      lo = first(pk.distinct[pg], end, [&](int j) { return list[j] < k; });
+      hi = first(lo, end, [&](int j) { return list[j] == k; });
+    }
+    for (int t = 0; t < pk.tt; ++t) {
+      if (__ballot(lo < hi) == 0) break;
+      const uint32_t* bits = pk.mask + (pg * pk.tt + t) * pk.words;
+      const int next = first(lo, hi, [&](int j) { return (bits[j >> 5] >> (j & 31) & 1u) != 0u; });
+      add_rows(__ballot(lo < next), gb, lo, std::true_type{}, (float)(next - lo));
+      lo = next;
     }
   }
   if (any && lane == 0) held = 1;
@@ -327,11 +394,13 @@ int pack_plan_build(const int32_t* indices, int64_t batch, int64_t s_q, int64_t 
     pk.suspect = (int32_t*)take(g * 4);
   }
   const int64_t nw = pk.key_words;
-  const size_t lds = (size_t)(nw * 4 + (int64_t)tt * pk.words * 4 + (nw * 2 + 3) / 4 * 4);
+  const int64_t used = nw * 4 + (int64_t)tt * pk.words * 4 + (nw + 1) / 2 * 4;
+  const int sort_cap = (int)std::min<int64_t>(kSortMax, (kPlanLds - used) / 4);
+  const size_t lds = (size_t)(used + sort_cap * 4);
   {
     const TimedLaunch tl("pack_plan_kernel", st);
     pack_plan_kernel<<<dim3((unsigned)pk.groups, (unsigned)batch), kPlanThreads, lds, st>>>(
-        indices, (int)s_q, (int)s_kv, (int)topk, q_offset, pk, idx, mask, count);
+        indices, (int)s_q, (int)s_kv, (int)topk, q_offset, pk, idx, mask, count, sort_cap);
   }
   pk.idx = idx;
   pk.mask = mask;
