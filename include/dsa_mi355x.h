@@ -245,6 +245,9 @@ int dsa_sparse_mla_bwd(const void* q, const void* kv, const int32_t* indices, co
  * workgroup, which gathers the union of their keys once; bf16 calls of few tokens (generation)
  * to split a token's keys over several workgroups.
  */
+/* (tokens that share a workgroup under that rule, the same for dsa_attn_mass_ws; 1: none do) */
+int dsa_attn_packed_tokens(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t topk,
+                           int64_t q_offset);
 int64_t dsa_sparse_mla_fwd_workspace_size(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
                                           int64_t topk, int64_t q_offset);
 int dsa_sparse_mla_fwd_ws(const void* q, const void* kv, const int32_t* indices, const float* sinks, void* out,

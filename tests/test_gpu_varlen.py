@@ -290,3 +290,29 @@ def test_compressor_tnd_parity(D, r, overlap):
                                     norm_weight=w.to(DEV)).cpu()
     ref_n = O.compressor_pool_tnd(kv, sc, ape, r, bs, pos, overlap=overlap, norm_weight=w, out_dtype=torch.bfloat16)
     assert rel_err(got_n.float(), ref_n) <= 2e-2
+
+
+@pytest.mark.parametrize("H", [16, 128])
+def test_short_batch_is_its_sequences(H):
+    """A batch of few tokens with many keys (host bounds) runs per sequence: neither the batch's
+    token count nor its keys choose another summation order."""
+    from torchtitan_npu_simulator_amd import _lib
+
+    ops, lib = _ops(), _lib.load_library()
+    lens_q, lens_k, K = [60, 1, 30], [900, 700, 30], 512
+    T, Tk = sum(lens_q), sum(lens_k)
+    g = torch.Generator().manual_seed(H)
+    q = torch.randn(T, H, 576, generator=g).bfloat16().to(DEV)
+    kv = torch.randn(Tk, 576, generator=g).bfloat16().to(DEV)
+    idx = _local_indices(lens_q, lens_k, K, seed=2).to(DEV)
+    out, smax, ssum = ops.sparse_mla_fwd_varlen(q, kv, idx, 0.05, _cu(lens_q), _cu(lens_k))
+    cq, ck = _cu(lens_q), _cu(lens_k)
+    for i in range(3):
+        a, b, lq, lk = cq[i], ck[i], lens_q[i], lens_k[i]
+        o = torch.empty(lq, H, 512, dtype=torch.bfloat16, device=DEV)
+        m, s = (torch.empty(lq, H, device=DEV) for _ in range(2))
+        _lib.check(lib.dsa_sparse_mla_fwd(
+            _lib.ptr(q[a:a + lq]), _lib.ptr(kv[b:b + lk]), _lib.ptr(idx[a:a + lq]), _lib.ptr(o), _lib.ptr(m), _lib.ptr(s),
+            _lib.DSA_BF16, 1, lq, lk, H, 576, 512, K, 0.05, lk - lq, _lib.stream_of(DEV)), "dsa_sparse_mla_fwd")
+        assert torch.equal(out[a:a + lq], o)
+        assert torch.equal(smax[a:a + lq], m) and torch.equal(ssum[a:a + lq], s)

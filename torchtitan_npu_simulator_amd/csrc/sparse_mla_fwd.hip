@@ -1156,6 +1156,11 @@ extern "C" int dsa_sparse_mla_fwd(const void* q, const void* kv, const int32_t* 
                                   n_heads, d_qk, d_v, topk, scale, q_offset, nullptr, 0, stream);
 }
 
+extern "C" int dsa_attn_packed_tokens(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
+                                      int64_t topk, int64_t q_offset) {
+  return dtype == DSA_BF16 ? dsa::pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset) : 1;
+}
+
 extern "C" int64_t dsa_sparse_mla_fwd_workspace_size(int dtype, int64_t batch, int64_t s_q, int64_t s_kv,
                                                      int64_t n_heads, int64_t topk, int64_t q_offset) {
   if (batch <= 0 || s_q <= 0 || s_kv <= 0) return 0;

@@ -782,8 +782,8 @@ def sparse_mla_fwd_varlen(q, kv, indices, scale, cu_seqlens_q, cu_seqlens_kv, *,
     require_gpu_tensor(q, "q")
     T, H, D = q.shape
     kv = kv.reshape(kv.shape[0], kv.shape[-1]).contiguous()
-    packed = q.dtype == torch.bfloat16 and T > 0 and lib.dsa_sparse_mla_fwd_workspace_size(
-        _lib.DSA_BF16, 1, T, kv.shape[0], H, indices.shape[-1], _NO_MASK_OFFSET) > 0
+    packed = q.dtype == torch.bfloat16 and T > 0 and lib.dsa_attn_packed_tokens(
+        _lib.DSA_BF16, 1, T, kv.shape[0], H, indices.shape[-1], _NO_MASK_OFFSET) > 1
     g = _varlen_global(indices, cu_seqlens_q, cu_seqlens_kv, T, kv.shape[0], q.device, packed)
     if g is not None:  # device bounds, packed tokens: one launch over the batch
         out, smax, ssum = sparse_mla_fwd(q.unsqueeze(0), kv.unsqueeze(0), g.unsqueeze(0), scale, d_v=d_v,
@@ -853,8 +853,8 @@ def attn_mass_varlen(q, kv, indices, smax, ssum, scale, cu_seqlens_q, cu_seqlens
     lib = load_library()
     T, H, D = q.shape
     kv = kv.reshape(kv.shape[0], kv.shape[-1]).contiguous()
-    packed = q.dtype == torch.bfloat16 and T > 0 and lib.dsa_attn_mass_workspace_size(
-        _lib.DSA_BF16, 1, T, kv.shape[0], H, indices.shape[-1], _NO_MASK_OFFSET) > 0
+    packed = q.dtype == torch.bfloat16 and T > 0 and lib.dsa_attn_packed_tokens(
+        _lib.DSA_BF16, 1, T, kv.shape[0], H, indices.shape[-1], _NO_MASK_OFFSET) > 1
     g = _varlen_global(indices, cu_seqlens_q, cu_seqlens_kv, T, kv.shape[0], q.device, packed)
     if g is not None:  # device bounds, packed tokens: one launch over the batch
         return attn_mass(q.unsqueeze(0), kv.unsqueeze(0), g.unsqueeze(0), smax.unsqueeze(0), ssum.unsqueeze(0), scale,
