@@ -316,3 +316,21 @@ def test_short_batch_is_its_sequences(H):
             _lib.DSA_BF16, 1, lq, lk, H, 576, 512, K, 0.05, lk - lq, _lib.stream_of(DEV)), "dsa_sparse_mla_fwd")
         assert torch.equal(out[a:a + lq], o)
         assert torch.equal(smax[a:a + lq], m) and torch.equal(ssum[a:a + lq], s)
+
+
+@pytest.mark.parametrize("device_bounds", [False, True])
+def test_packed_backward_keeps_no_mass(device_bounds):
+    """The TND KL op computes its own mass, so the backward of a batch leaves none behind."""
+    ops = _ops()
+    lens, H, K = [500, 700], 16, 64
+    T = sum(lens)
+    g = torch.Generator().manual_seed(4)
+    q, dout = (torch.randn(T, H, w, generator=g).bfloat16().to(DEV) for w in (576, 512))
+    kv = torch.randn(T, 576, generator=g).bfloat16().to(DEV)
+    idx = _local_indices(lens, lens, K, seed=3).to(DEV)
+    cu = torch.tensor(_cu(lens), dtype=torch.int32, device=DEV) if device_bounds else _cu(lens)
+    out, smax, ssum = ops.sparse_mla_fwd_varlen(q, kv, idx, 0.05, cu, cu)
+    got = ops.sparse_mla_bwd_varlen(q, kv, idx, out, dout, smax, ssum, 0.05, cu, cu)
+    assert ops._attn_mass_entry is None
+    ref = ops.sparse_mla_bwd_varlen(q, kv, idx, out, dout, smax, ssum, 0.05, cu, cu, return_mass=True)
+    assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])

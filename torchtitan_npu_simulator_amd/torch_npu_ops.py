@@ -686,7 +686,7 @@ def take_attn_mass(q, kv, indices, smax, ssum, scale, q_offset=0):
 
 
 def sparse_mla_bwd(q, kv, indices, out, dout, smax, ssum, scale, *, q_offset=0, workspace_bytes=None,
-                   return_mass=False, sinks=None):
+                   return_mass=False, sinks=None, keep_mass=True):
     """(dq like q, dkv fp32 [B,S_kv,D_qk]) from dsa_sparse_mla_bwd, plus the head-summed
     attention mass [B,S,K] fp32 when ``return_mass`` (bf16 path; the same quantity as
     ``attn_mass``, taken from the probabilities the backward recomputes anyway), plus
@@ -694,6 +694,7 @@ def sparse_mla_bwd(q, kv, indices, out, dout, smax, ssum, scale, *, q_offset=0, 
     then be the statistics sparse_mla_fwd returned with the same sinks).
 
     ``workspace_bytes`` caps the scratch (fewer bytes -> more query-row chunks).
+    ``keep_mass=False``: no mass is written for ``take_attn_mass``.
     """
     global _attn_mass_entry
     lib = load_library()
@@ -704,7 +705,7 @@ def sparse_mla_bwd(q, kv, indices, out, dout, smax, ssum, scale, *, q_offset=0, 
     indices = indices.reshape(B, S, K).to(torch.int32).contiguous()
     # without return_mass the bf16 path still writes the mass (a few % of the score kernel)
     # and keeps it for the indexer KL op of the same layer (take_attn_mass)
-    keep = _share_attn_mass and not return_mass and sinks is None and q.dtype == torch.bfloat16
+    keep = keep_mass and _share_attn_mass and not return_mass and sinks is None and q.dtype == torch.bfloat16
     if keep:
         _attn_mass_entry = None  # (the old mass goes before the new one is allocated)
         keep_key = _attn_mass_key(q, kv, indices, smax, ssum, scale, q_offset)
@@ -820,9 +821,10 @@ def sparse_mla_bwd_varlen(q, kv, indices, out, dout, smax, ssum, scale, cu_seqle
         if workspace_bytes is None else int(workspace_bytes)) == 1
     g = _varlen_global(indices, cu_seqlens_q, cu_seqlens_kv, T, T_kv, q.device, packed)
     if g is not None:  # device bounds, packed tokens: one launch over the batch
+        # (the TND KL op computes its own mass: none is kept for it)
         res = sparse_mla_bwd(q.unsqueeze(0), kv.unsqueeze(0), g.unsqueeze(0), out.unsqueeze(0), dout.unsqueeze(0),
                              smax.unsqueeze(0), ssum.unsqueeze(0), scale, q_offset=_NO_MASK_OFFSET,
-                             workspace_bytes=workspace_bytes, return_mass=return_mass)
+                             workspace_bytes=workspace_bytes, return_mass=return_mass, keep_mass=False)
         return tuple(t[0] for t in res)
     cu_q, cu_k, n_seq = _varlen_seqs(cu_seqlens_q, cu_seqlens_kv, T, T_kv)
     K = indices.shape[-1]
