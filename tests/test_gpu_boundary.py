@@ -317,3 +317,41 @@ def test_kl_op_takes_the_attention_backward_mass(monkeypatch):
     ops.npu_sparse_lightning_indexer_grad_kl_loss(q_nope.detach(), k_nope.detach(), qi, ki, w, idx, smax2, ssum2,
                                                   scale, **kw)
     assert calls == [1]
+
+
+class _Stop(torch.autograd.Function):
+    """Passes its input on and returns no gradient for it."""
+
+    @staticmethod
+    def forward(ctx, x):
+        return x * 1.0
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+@pytest.mark.parametrize("route", ["BSND", "TND", "linked"])
+def test_attention_undefined_output_gradient(route):
+    """An output whose consumer returns no gradient gives zero gradients, as any zero would."""
+    from torchtitan_npu_simulator_amd import torch_npu_ops as ops
+
+    S, H, K = 40, 8, 16
+    q, kv, _, scale = attn_inputs(S, H, seed=1)
+    q, kv = q.to(DEV).requires_grad_(), kv.to(DEV).requires_grad_()
+    idx = rand_indices(S, K, seed=2).to(DEV)
+    if route == "linked":
+        link = ops.MassLink()
+        after = torch.zeros((), device=DEV)
+        out = ops.sparse_flash_attention_linked(q, kv.unsqueeze(2), idx, scale, after, link)[0]
+    else:
+        tnd = route == "TND"
+        qq, kk, ii = (q[0], kv[0].unsqueeze(1), idx[0]) if tnd else (q, kv.unsqueeze(2), idx.unsqueeze(2))
+        lay = dict(layout_query="TND", layout_kv="TND", cu_seqlens_q=[0, S], cu_seqlens_kv=[0, S]) if tnd else {}
+        out = ops.npu_sparse_flash_attention(qq[..., :512], kk[..., :512], kk[..., :512], ii, query_rope=qq[..., 512:],
+                                             key_rope=kk[..., 512:], scale_value=scale, **lay)[0]
+    dq, dkv = torch.autograd.grad(_Stop.apply(out).sum(), [q, kv])
+    assert dq.shape == q.shape and dkv.shape == kv.shape
+    assert not dq.any() and not dkv.any()
+    if route == "linked":
+        assert link.mass is not None

@@ -911,9 +911,9 @@ class _SparseFlashAttention(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout, _dmax, _dsum):
-        if dout is None:
-            return (None,) * 7
         q, kv3, indices, out, smax, ssum = ctx.saved_tensors
+        if dout is None:  # (an undefined gradient is zero, and so are the ones returned)
+            dout = torch.zeros_like(out)
         dq, dkv = sparse_mla_bwd(q, kv3, indices, out, dout.contiguous(), smax, ssum, ctx.scale, q_offset=ctx.q_offset)
         dnope, dpe = ctx.split
         dkv = dkv.to(kv3.dtype).reshape(ctx.kv_shape)
@@ -975,9 +975,9 @@ class _SparseFlashAttentionLinked(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout, _dmax, _dsum):
-        if dout is None:
-            return (None,) * 8
         q, kv3, indices, out, smax, ssum = ctx.saved_tensors
+        if dout is None:
+            dout = torch.zeros_like(out)
         dq, dkv, mass = sparse_mla_bwd(q, kv3, indices, out, dout.contiguous(), smax, ssum, ctx.scale,
                                        q_offset=ctx.q_offset, return_mass=True)
         ctx.link.mass = mass
@@ -1014,9 +1014,9 @@ class _SparseFlashAttentionTND(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout, _dmax, _dsum):
-        if dout is None:
-            return (None,) * 8
         q, kv2, indices, out, smax, ssum = ctx.saved_tensors
+        if dout is None:
+            dout = torch.zeros_like(out)
         dq, dkv = sparse_mla_bwd_varlen(q, kv2, indices, out, dout.contiguous(), smax, ssum, ctx.scale, *ctx.cu)
         dnope, _ = ctx.split
         dkv = dkv.to(kv2.dtype).reshape(ctx.kv_shape)
