@@ -102,3 +102,13 @@ def test_lightning_indexer_workspace_respects_the_score_budget(lib, B, S, s_k):
         assert small <= budget - 4 * s_k + 256 + pieces
     big = ops.lightning_indexer_workspace_bytes(lib, B, S, s_k, 64, 128, fp8, budget=B * S * s_k * 4)
     assert big >= B * S * s_k * 4  # everything in one pass when it fits
+
+
+def test_smallest_workspaces(lib):
+    """A workspace that once held one query row of a problem still does: the sizes are those of
+    the 256-pair reduction segments that a single row has always had."""
+    for b, s, s_kv, d, k, attn, kl in [(1, 4096, 4096, 576, 2048, 3519744, 606464), (1, 64, 64, 576, 64, 113664, 18944),
+                                       (2, 1000, 1000, 512, 256, 809728, 149248), (3, 7, 77, 576, 33, 221696, 27904),
+                                       (1, 1, 5000, 576, 1000, 1779968, 344320)]:
+        assert lib.dsa_sparse_mla_bwd_chunk_rows(b, s, s_kv, d, k, attn) >= 1
+        assert lib.dsa_indexer_kl_grad_chunk_rows(b, s, s_kv, k, kl) >= 1

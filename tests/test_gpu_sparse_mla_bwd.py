@@ -341,3 +341,25 @@ def test_bwd_pair_fill_row_blocks_without_keys_in_a_range(S, K, s_kv, windows):
     sel = idx.flatten().long()
     touched[sel[sel >= 0]] = True
     assert float(dkv[0, ~touched].abs().sum()) == 0.0
+
+
+@pytest.mark.gpu
+def test_smallest_workspace():
+    """One query row per chunk, in the smallest workspace that is taken."""
+    from torchtitan_npu_simulator_amd import _lib
+    from torchtitan_npu_simulator_amd import torch_npu_ops as ops
+
+    S, H, K = 21, 16, 64
+    q, kv, dout, scale = attn_inputs(S, H, seed=3)
+    idx = rand_indices(S, K, seed=3).cuda()
+    q, kv, dout = q.cuda(), kv.cuda(), dout.cuda()
+    out, smax, ssum = ops.sparse_mla_fwd(q, kv, idx, scale)
+    rows, lo, hi = _lib.load_library().dsa_sparse_mla_bwd_chunk_rows, 0, 1 << 30
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        lo, hi = (lo, mid) if rows(1, S, S, 576, K, mid) > 0 else (mid, hi)
+    assert rows(1, S, S, 576, K, hi) == 1
+    full = ops.sparse_mla_bwd(q, kv, idx, out, dout, smax, ssum, scale)
+    part = ops.sparse_mla_bwd(q, kv, idx, out, dout, smax, ssum, scale, workspace_bytes=hi)
+    assert torch.equal(full[0], part[0])
+    assert rel_err(part[1], full[1]) <= 1e-5

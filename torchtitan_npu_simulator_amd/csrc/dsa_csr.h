@@ -424,17 +424,20 @@ __global__ void __launch_bounds__(1024) csr_scan_kernel(const int* __restrict__ 
 // pairs per wave: 256, fewer where those would not fill the chip (a segment costs two partial
 // rows).  150 rows of top-256: the reduction of 576-wide rows 57 us on 150 segments of 256
 // pairs, 12 us on 1200 of 32; 1500 rows of top-1024, 128-wide: 67 us of 256, 56 us of 64.
-inline int csr_seg_shift(int64_t rows, int64_t K) {
+// `coarse` keeps 256: a chunk of one row in a workspace that has no room for more partial rows
+// (with room, one row of top-2048 and 128 heads takes 355 us, coarse 585).
+inline int csr_seg_shift(int64_t rows, int64_t K, bool coarse) {
+  if (coarse) return 8;
   const int64_t pairs = rows * K;
   return pairs >= (1 << 22) ? 8 : pairs >= (1 << 21) ? 7 : pairs >= (1 << 20) ? 6 : 5;
 }
-inline int64_t csr_segments(int64_t rows, int64_t K) {
-  const int sh = csr_seg_shift(rows, K);
+inline int64_t csr_segments(int64_t rows, int64_t K, bool coarse) {
+  const int sh = csr_seg_shift(rows, K, coarse);
   return (rows * K + (1 << sh) - 1) >> sh;
 }
 // the most segments of any chunk of at most `rows` rows
-inline int64_t csr_segments_max(int64_t rows, int64_t K) {
-  const int64_t n = csr_segments(rows, K), few = (rows * K + 31) / 32;
+inline int64_t csr_segments_max(int64_t rows, int64_t K, bool coarse) {
+  const int64_t n = csr_segments(rows, K, coarse), few = coarse ? n : (rows * K + 31) / 32;
   return n > 32768 ? n : few < 32768 ? few : 32768;
 }
 
@@ -586,17 +589,17 @@ csr_partial_fixup_kernel(const int* __restrict__ row_ptr, const int* __restrict_
 // counts and row_ptr (s_kv + 1 ints each), the segment table (one int per segment
 // of the chunk), the [row block][key] count table, the [column chunk][key] chunk offsets
 // and two partial-sum rows per segment (at a 16-byte boundary).
-inline int64_t csr_ws_ints(int64_t s_kv, int64_t rows, int64_t K) {
+inline int64_t csr_ws_ints(int64_t s_kv, int64_t rows, int64_t K, bool coarse = false) {
   const int64_t n_rb = csr_row_blocks_max(s_kv, K, rows);
   const int64_t n_chunks = (n_rb + kColChunk - 1) / kColChunk;
-  const int64_t n_seg = csr_segments_max(rows, K);
+  const int64_t n_seg = csr_segments_max(rows, K, coarse);
   return (2 * (s_kv + 1) + n_seg + (n_rb + n_chunks) * s_kv + 3) / 4 * 4 + 4;  // (+4: the fill's dup flag last)
 }
-inline int64_t csr_part_bytes(int64_t rows, int64_t K, int64_t width) {
-  return csr_segments_max(rows, K) * 2 * width * 4;
+inline int64_t csr_part_bytes(int64_t rows, int64_t K, int64_t width, bool coarse = false) {
+  return csr_segments_max(rows, K, coarse) * 2 * width * 4;
 }
-inline int64_t csr_ws_bytes(int64_t s_kv, int64_t rows, int64_t K, int64_t width) {
-  return csr_ws_ints(s_kv, rows, K) * 4 + csr_part_bytes(rows, K, width);
+inline int64_t csr_ws_bytes(int64_t s_kv, int64_t rows, int64_t K, int64_t width, bool coarse = false) {
+  return csr_ws_ints(s_kv, rows, K, coarse) * 4 + csr_part_bytes(rows, K, width, coarse);
 }
 
 // A built CSR: the key-sorted pair list with its key pointers and segment table.
@@ -609,14 +612,14 @@ struct CsrView {
 // Build the CSR of query rows [row0, row0 + rows) of batch element b: `pairs` holds
 // rows * K ints, csr_ws csr_ws_ints(s_kv, rows, K) ints.
 inline int csr_build(const int32_t* idx, int* pairs, int* csr_ws, int S, int s_kv, int K, int64_t q_offset, int row0,
-                     int rows, int b, hipStream_t st, CsrView* view) {
+                     int rows, int b, hipStream_t st, CsrView* view, bool coarse = false) {
   const int rows_per_wg = csr_rows_per_wg(s_kv, K, rows);
   const int64_t n_rb = ceil_div(rows, rows_per_wg);
   const int64_t n_chunks = ceil_div(n_rb, kColChunk);
   int* counts = csr_ws;
   int* row_ptr = counts + (s_kv + 1);
   int* seg_key = row_ptr + (s_kv + 1);
-  const int64_t n_seg = csr_segments(rows, K);
+  const int64_t n_seg = csr_segments(rows, K, coarse);
   int* table = seg_key + n_seg;
   int* chunk_off = table + n_rb * s_kv;
   const int n_ranges = (int)ceil_div(s_kv, kLdsKeys);
@@ -628,7 +631,7 @@ inline int csr_build(const int32_t* idx, int* pairs, int* csr_ws, int S, int s_k
   const bool vec = K % 4 == 0 && ((uintptr_t)(idx + row_base * K) % 16) == 0;
   const int n_franges = (int)ceil_div(s_kv, kFillKeys);
   const bool staged = n_franges <= kFillRangesMax && n_franges * ceil_div(n_rb, kFillRB) >= kFillStagedMin;
-  int* dup_flag = staged ? csr_ws + csr_ws_ints(s_kv, rows, K) - 1 : nullptr;
+  int* dup_flag = staged ? csr_ws + csr_ws_ints(s_kv, rows, K, coarse) - 1 : nullptr;
   launch_csr_count<false>(vec, (unsigned)cgrid, hist_bytes, st, idx, table, nullptr, nullptr, pairs, S, s_kv, K,
                           q_offset, row0, rows, b, n_ranges, rows_per_wg, dup_flag);
   {
@@ -666,7 +669,8 @@ inline int csr_build(const int32_t* idx, int* pairs, int* csr_ws, int S, int s_k
   }
   {
     const TimedLaunch tl("csr_seg_key_kernel", st);
-    csr_seg_key_kernel<<<ceil_div(s_kv, 256), 256, 0, st>>>(row_ptr, seg_key, s_kv, csr_seg_shift(rows, K));
+    csr_seg_key_kernel<<<ceil_div(s_kv, 256), 256, 0, st>>>(row_ptr, seg_key, s_kv,
+                                                             csr_seg_shift(rows, K, coarse));
   }
   view->pairs = pairs;
   view->row_ptr = row_ptr;
@@ -677,9 +681,9 @@ inline int csr_build(const int32_t* idx, int* pairs, int* csr_ws, int S, int s_k
 // Reduce the contribution rows cbuf[b][row][slot][8 * row_chunks] of the rows a built CSR
 // covers into acc_out[b][key][...]; `part` holds csr_part_bytes(rows, K, 8 * row_chunks).
 inline int csr_reduce_built(const CsrView& v, const uint16_t* cbuf, float* acc_out, float* part, int s_kv, int rows,
-                            int K, int b, int row_chunks, hipStream_t st) {
-  const int sh = csr_seg_shift(rows, K);
-  const unsigned rgrid = ceil_div(csr_segments(rows, K), 4);
+                            int K, int b, int row_chunks, hipStream_t st, bool coarse = false) {
+  const int sh = csr_seg_shift(rows, K, coarse);
+  const unsigned rgrid = ceil_div(csr_segments(rows, K, coarse), 4);
   const TimedLaunch tl(row_chunks == 72   ? "dkv_reduce_kernel<72>"
                        : row_chunks == 64 ? "dkv_reduce_kernel<64>"
                                           : "dkv_reduce_kernel<16>",
@@ -708,14 +712,15 @@ inline int csr_reduce_built(const CsrView& v, const uint16_t* cbuf, float* acc_o
 
 // Build the CSR for query rows [row0, row0 + rows) of batch element b and reduce the
 // contribution rows cbuf[b][row][slot][8 * row_chunks] into acc_out[b][key][...].
-// csr_ws holds csr_ws_bytes(s_kv, rows, K) bytes.
+// csr_ws holds csr_ws_bytes(s_kv, rows, K, 8 * row_chunks, coarse) bytes.
 inline int csr_reduce(const int32_t* idx, const uint16_t* cbuf, float* acc_out, int* pairs, int* csr_ws, int S,
-                      int s_kv, int K, int64_t q_offset, int row0, int rows, int b, int row_chunks, hipStream_t st) {
+                      int s_kv, int K, int64_t q_offset, int row0, int rows, int b, int row_chunks, hipStream_t st,
+                      bool coarse) {
   if (s_kv <= 0 || rows <= 0) return DSA_OK;  // no pairs: the accumulator keeps its contents
   CsrView v;
-  if (int rc = csr_build(idx, pairs, csr_ws, S, s_kv, K, q_offset, row0, rows, b, st, &v)) return rc;
-  float* part = reinterpret_cast<float*>(csr_ws + csr_ws_ints(s_kv, rows, K));
-  return csr_reduce_built(v, cbuf, acc_out, part, s_kv, rows, K, b, row_chunks, st);
+  if (int rc = csr_build(idx, pairs, csr_ws, S, s_kv, K, q_offset, row0, rows, b, st, &v, coarse)) return rc;
+  float* part = reinterpret_cast<float*>(csr_ws + csr_ws_ints(s_kv, rows, K, coarse));
+  return csr_reduce_built(v, cbuf, acc_out, part, s_kv, rows, K, b, row_chunks, st, coarse);
 }
 
 // A prebuilt CSR of every query row of every batch element, shared by the reductions of one

@@ -628,17 +628,27 @@ indexer_kl_generic_kernel(const uint16_t* __restrict__ qi, const uint16_t* __res
 
 struct KlPlan {
   int64_t rows, ck_bytes, pairs_bytes, csr_bytes, total;
+  bool coarse;  // the reduction's segments (dsa_csr.h)
 };
 
-KlPlan plan_kl(int64_t batch, int64_t rows, int64_t s_k, int64_t topk) {
+KlPlan plan_kl(int64_t batch, int64_t rows, int64_t s_k, int64_t topk, bool coarse = false) {
   auto al = [](int64_t x) { return (x + 255) / 256 * 256; };
   KlPlan p{};
   p.rows = rows;
   p.ck_bytes = batch * rows * topk * kD * 2;
   p.pairs_bytes = rows * topk * 4;
-  p.csr_bytes = csr_ws_bytes(s_k, rows, topk, 128);
+  p.csr_bytes = csr_ws_bytes(s_k, rows, topk, 128, coarse);
+  p.coarse = coarse;
   p.total = al(p.ck_bytes) + al(p.pairs_bytes) + al(p.csr_bytes);
   return p;
+}
+
+// the most rows per chunk whose scratch fits (total > bytes: not even one row's does)
+KlPlan fit_kl(int64_t batch, int64_t s_q, int64_t s_k, int64_t topk, int64_t bytes) {
+  const int64_t per_row = batch * topk * kD * 2 + topk * 4;
+  KlPlan p = plan_kl(batch, std::max<int64_t>(1, std::min<int64_t>(s_q, bytes / per_row)), s_k, topk);
+  while (p.total > bytes && p.rows > 1) p = plan_kl(batch, p.rows - 1, s_k, topk);
+  return p.total > bytes ? plan_kl(batch, 1, s_k, topk, true) : p;
 }
 
 constexpr int64_t kKlBudget = 8LL << 30;
@@ -660,10 +670,7 @@ extern "C" int64_t dsa_indexer_kl_grad_chunk_rows(int64_t batch, int64_t s_q, in
                                                   int64_t workspace_bytes) {
   using namespace dsa;
   if (batch <= 0 || s_q <= 0 || s_k <= 0 || topk <= 0 || workspace_bytes <= 0) return 0;
-  const int64_t per_row = batch * topk * kD * 2 + topk * 4;
-  const int64_t rows = std::max<int64_t>(1, std::min<int64_t>(s_q, workspace_bytes / per_row));
-  KlPlan plan = plan_kl(batch, rows, s_k, topk);
-  while (plan.total > workspace_bytes && plan.rows > 1) plan = plan_kl(batch, plan.rows - 1, s_k, topk);
+  const KlPlan plan = fit_kl(batch, s_q, s_k, topk, workspace_bytes);
   return plan.total > workspace_bytes ? 0 : plan.rows;
 }
 
@@ -707,10 +714,7 @@ extern "C" int dsa_indexer_kl_grad_ex(const void* q_idx, const void* k_idx, cons
     return check_launch("dsa_indexer_kl_grad(generic)");
   }
   if (!workspace) return set_error(DSA_ERR_INVALID_ARG, "dsa_indexer_kl_grad: workspace required");
-  const int64_t per_row = batch * topk * kD * 2 + topk * 4;
-  int64_t rows = std::max<int64_t>(1, std::min<int64_t>(s_q, workspace_bytes / per_row));
-  KlPlan plan = plan_kl(batch, rows, s_k, topk);
-  while (plan.total > workspace_bytes && plan.rows > 1) plan = plan_kl(batch, plan.rows - 1, s_k, topk);
+  const KlPlan plan = fit_kl(batch, s_q, s_k, topk, workspace_bytes);
   if (plan.total > workspace_bytes)
     return set_error(DSA_ERR_INVALID_ARG, "dsa_indexer_kl_grad: workspace of %lld bytes is too small",
                      (long long)workspace_bytes);
@@ -734,7 +738,7 @@ extern "C" int dsa_indexer_kl_grad_ex(const void* q_idx, const void* k_idx, cons
     if (int rc = check_launch("dsa_indexer_kl_grad(mfma)")) return rc;
     // a prebuilt CSR of every row (the one the attention backward reduced dKV with) serves a
     // one-chunk plan; otherwise each chunk builds its own
-    const bool prebuilt = pair_csr && rows_c == s_q;
+    const bool prebuilt = pair_csr && rows_c == s_q && !plan.coarse;
     for (int b = 0; b < (int)batch; ++b) {
       if (prebuilt) {
         float* part = reinterpret_cast<float*>(csr + csr_ws_ints(s_k, rows_c, topk));
@@ -742,7 +746,7 @@ extern "C" int dsa_indexer_kl_grad_ex(const void* q_idx, const void* k_idx, cons
                                       rows_c, (int)topk, b, kRowC, st))
           return rc;
       } else if (int rc = csr_reduce(indices, ck, dk_idx_accum, pairs, csr, (int)s_q, (int)s_k, (int)topk, q_offset,
-                                     (int)r0, rows_c, b, kRowC, st)) {
+                                     (int)r0, rows_c, b, kRowC, st, plan.coarse)) {
         return rc;
       }
     }

@@ -1133,11 +1133,13 @@ sink_colsum_kernel(const float* __restrict__ pd, int64_t nrows, int H, float* __
 struct BwdPlan {
   int64_t rows;  // query rows per chunk
   int64_t g_bytes, c_bytes, pairs_bytes, csr_bytes, delta_bytes, total;  // delta_bytes: the sink's parts
+  bool coarse;  // the reduction's segments (dsa_csr.h)
 };
 
 // Scratch per chunk: G and C (bf16, C rows `width` columns), the CSR pair list and
 // offsets, and the sink's gradient parts (fp32 per row and head).
-BwdPlan plan_bwd(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int64_t budget, int64_t width) {
+BwdPlan plan_bwd(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int64_t budget, int64_t width,
+                 bool coarse = false) {
   BwdPlan p{};
   const int64_t per_row = batch * g_slots(topk) * kGW * 2 + batch * topk * (int64_t)(width * 2 + 4) +
                           batch * kHeadsMax * 4 + topk * width / 32;  // (last: CSR segment partials)
@@ -1147,11 +1149,19 @@ BwdPlan plan_bwd(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int64_t
   p.g_bytes = batch * rows * g_slots(topk) * kGW * 2;
   p.c_bytes = batch * rows * topk * width * 2;
   p.pairs_bytes = rows * topk * 4;
-  p.csr_bytes = csr_ws_bytes(s_kv, rows, topk, width);
+  p.csr_bytes = csr_ws_bytes(s_kv, rows, topk, width, coarse);
+  p.coarse = coarse;
   p.delta_bytes = batch * rows * kHeadsMax * 4;
   auto al = [](int64_t x) { return (x + 255) / 256 * 256; };
   p.total = al(p.g_bytes) + al(p.c_bytes) + al(p.pairs_bytes) + al(p.csr_bytes) + al(p.delta_bytes);
   return p;
+}
+
+// the largest chunk whose scratch fits (total > bytes: not even one row's does)
+BwdPlan fit_bwd(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int64_t bytes, int64_t width) {
+  BwdPlan p = plan_bwd(batch, s_q, s_kv, topk, bytes, width);
+  while (p.total > bytes && p.rows > 1) p = plan_bwd(batch, p.rows - 1, s_kv, topk, 0, width);
+  return p.total > bytes ? plan_bwd(batch, 1, s_kv, topk, 0, width, true) : p;
 }
 
 constexpr int64_t kDefaultBudget = 32LL << 30;  // scratch for the G / C chunks (C3 in one chunk)
@@ -1322,9 +1332,7 @@ static int sparse_mla_bwd_impl(const void* q, const void* kv, const int32_t* ind
     return sparse_mla_bwd_packed(q, kv, indices, out, dout, softmax_max, softmax_sum, dq, dkv_accum, mass,
                                  (char*)workspace, pp, batch, s_q, s_kv, n_heads, d_qk, topk, scale, q_offset, sinks,
                                  dsink, st);
-  // choose the largest chunk whose scratch fits the given workspace
-  BwdPlan plan = plan_bwd(batch, s_q, s_kv, topk, workspace_bytes, d_qk);
-  while (plan.total > workspace_bytes && plan.rows > 1) plan = plan_bwd(batch, plan.rows - 1, s_kv, topk, 0, d_qk);
+  const BwdPlan plan = fit_bwd(batch, s_q, s_kv, topk, workspace_bytes, d_qk);
   if (plan.total > workspace_bytes)
     return set_error(DSA_ERR_INVALID_ARG, "dsa_sparse_mla_bwd: workspace of %lld bytes is too small",
                      (long long)workspace_bytes);
@@ -1347,7 +1355,7 @@ static int sparse_mla_bwd_impl(const void* q, const void* kv, const int32_t* ind
     if (sinks)
       if (int rc = launch_sink_sum(pdbuf, dsink, batch, n_heads, rows, st)) return rc;
     // a prebuilt CSR of every row serves a one-chunk plan; otherwise each chunk builds its own
-    const bool prebuilt = csr && rows == s_q;
+    const bool prebuilt = csr && rows == s_q && !plan.coarse;
     for (int b = 0; b < (int)batch; ++b) {
       if (prebuilt) {
         float* part = reinterpret_cast<float*>(counts + csr_ws_ints(s_kv, rows, topk));
@@ -1355,7 +1363,7 @@ static int sparse_mla_bwd_impl(const void* q, const void* kv, const int32_t* ind
                                       (int)topk, b, (int)(d_qk / 8), st))
           return rc;
       } else if (int rc = csr_reduce(indices, cbuf, dkv_accum, pairs, counts, (int)s_q, (int)s_kv, (int)topk, q_offset,
-                                     (int)r0, rows, b, (int)(d_qk / 8), st)) {
+                                     (int)r0, rows, b, (int)(d_qk / 8), st, plan.coarse)) {
         return rc;
       }
     }
@@ -1384,8 +1392,7 @@ extern "C" int64_t dsa_sparse_mla_bwd_chunk_rows(int64_t batch, int64_t s_q, int
                                                  int64_t topk, int64_t workspace_bytes) {
   using namespace dsa;
   if (batch <= 0 || s_q <= 0 || s_kv <= 0 || topk <= 0 || workspace_bytes <= 0) return 0;
-  BwdPlan plan = plan_bwd(batch, s_q, s_kv, topk, workspace_bytes, d_qk);
-  while (plan.total > workspace_bytes && plan.rows > 1) plan = plan_bwd(batch, plan.rows - 1, s_kv, topk, 0, d_qk);
+  const BwdPlan plan = fit_bwd(batch, s_q, s_kv, topk, workspace_bytes, d_qk);
   return plan.total > workspace_bytes ? 0 : plan.rows;
 }
 
