@@ -366,7 +366,8 @@ int dsa_indexer_kl_grad_ex(const void* q_idx, const void* k_idx, const float* w,
  */
 int64_t dsa_pair_csr_size(int64_t batch, int64_t s_q, int64_t s_k, int64_t topk);
 /* 1 where dsa_sparse_mla_bwd{,_ex,_sink} with this workspace runs over packed tokens (bf16, at
- * most 64 heads): it then reduces dKV by its own plan and takes no pair CSR */
+ * most 64 heads, a workspace for a chunk of 192 tokens or all of them): it then reduces dKV by
+ * its own plan and takes no pair CSR */
 int dsa_sparse_mla_bwd_packed(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t d_qk, int64_t topk,
                               int64_t q_offset, int64_t workspace_bytes);
 /* query rows per chunk that a workspace of workspace_bytes gives dsa_sparse_mla_bwd{,_ex}

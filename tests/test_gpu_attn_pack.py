@@ -115,3 +115,35 @@ def test_packed_sink_and_chunks():
         assert rel_err(a, b) <= 1e-5
     for a, b in zip(full, one):
         assert rel_err(a, b) <= 1e-2
+
+
+def test_packed_needs_room():
+    """A workspace that holds only a few groups at a time runs one token per workgroup."""
+    from torchtitan_npu_simulator_amd import _lib
+
+    lib = _lib.load_library()
+    packed, rows = lib.dsa_sparse_mla_bwd_packed, lib.dsa_sparse_mla_bwd_chunk_rows
+    for S, H, K in [(4096, 16, 2048), (4096, 64, 2048), (2048, 64, 512), (700, 16, 64)]:
+        most = int(lib.dsa_sparse_mla_bwd_workspace_size(1, S, S, H, 576, K))
+        assert packed(1, S, S, H, 576, K, 0, most) == 1
+        few = most * 100 // S  # (about a hundred tokens' share)
+        assert packed(1, S, S, H, 576, K, 0, few) == 0 and rows(1, S, S, 576, K, few) >= 1
+
+
+@pytest.mark.gpu
+def test_packed_capped_workspace_results():
+    from torchtitan_npu_simulator_amd import _lib
+    from torchtitan_npu_simulator_amd import torch_npu_ops as ops
+
+    S, H, K = 600, 32, 64
+    g = torch.Generator().manual_seed(9)
+    q, dout = torch.randn(1, S, H, 576, generator=g).bfloat16().cuda(), torch.randn(1, S, H, 512, generator=g).bfloat16().cuda()
+    kv = torch.randn(1, S, 576, generator=g).bfloat16().cuda()
+    idx = rand_indices(S, K, seed=9).cuda()
+    out, smax, ssum = ops.sparse_mla_fwd(q, kv, idx, 576 ** -0.5)
+    most = int(_lib.load_library().dsa_sparse_mla_bwd_workspace_size(1, S, S, H, 576, K))
+    runs = [ops.sparse_mla_bwd(q, kv, idx, out, dout, smax, ssum, 576 ** -0.5, workspace_bytes=b)
+            for b in (most, most // 2, most // 8)]
+    for r in runs[1:]:
+        for a, b in zip(r, runs[0]):
+            assert rel_err(a, b) <= 1e-2

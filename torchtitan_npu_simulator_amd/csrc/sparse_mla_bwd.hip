@@ -1166,6 +1166,13 @@ BwdPlan fit_bwd(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int64_t 
 
 constexpr int64_t kDefaultBudget = 32LL << 30;  // scratch for the G / C chunks (C3 in one chunk)
 
+// Tokens per chunk from which a workspace too small for all of them is packed: a chunk is one
+// workgroup per group, while the one-token kernels put a workgroup per token into it and
+// need no room for a plan.  Packed and one token, ms: S = 4096, 16 heads, top-2048 in 96 MB (8
+// tokens) 168 and 42, 256 MB (56) 25 and 17, 512 MB (128) 11.2 and 9.4; S = 2048, 64 heads,
+// top-512 in 64 MB (66) 4.57 and 4.11, 128 MB (140) 2.33 and 2.31.
+constexpr int64_t kPackMinTokens = 192;
+
 // Scratch of the packed-token backward: the plan, then per chunk of `rows` groups G, C, the
 // sink's gradient parts and the per-token mass.  total = 0: unpacked.
 struct PackBwdPlan {
@@ -1182,7 +1189,7 @@ PackBwdPlan plan_pack_bwd(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_he
   p.plan_bytes = pack_plan_bytes(batch, s_q, s_kv, topk, p.tt, true);
   const int64_t per_row = batch * (cap * (kGW * 2 + width * 2 + p.tt * 4) + kHeadsMax * 4);
   p.rows = std::min<int64_t>(groups, (budget - p.plan_bytes - 4 * 256) / per_row);
-  if (p.rows < 1) return p;
+  if (p.rows < 1 || (p.rows < groups && batch * p.rows * p.tt < kPackMinTokens)) return p;
   p.g_bytes = al(batch * p.rows * cap * kGW * 2);
   p.c_bytes = al(batch * p.rows * cap * width * 2);
   p.delta_bytes = al(batch * p.rows * kHeadsMax * 4);
