@@ -275,10 +275,13 @@ attn_f32_bwd_kernel(const float* __restrict__ q, const float* __restrict__ kv, c
       __syncthreads();
       continue;
     }
-    {  // waves 0, 1: S of key tiles 0, 1; waves 2, 3: dP of them
-      const int kt = wave & 1;
-      const f32x4 x = wave < 2 ? dot_rows(tile + 16 * kt * kLd, qs, 0, dqk, col, g)
-                               : dot_rows(tile + 16 * kt * kLd, dos, 0, dv, col, g);
+    {  // waves 0, 1: S of key tiles 0, 1; waves 2, 3: dP of them.  In two column halves, which
+       // gives S the forward's bits (the rounding of S then cancels in P = exp(S - lse): dQ is off by
+       // 5.4e-7 from fp64, 8.7e-7 with S in one chain) and dP a shorter chain
+      const int kt = wave & 1, d = wave < 2 ? dqk : dv, mid = (d / 16 / 2) * 16;
+      const float* rows = wave < 2 ? qs : dos;
+      const f32x4 x = dot_rows(tile + 16 * kt * kLd, rows, 0, mid, col, g) +
+                      dot_rows(tile + 16 * kt * kLd, rows, mid, d, col, g);
       *reinterpret_cast<f32x4*>(&(wave < 2 ? ps : ds)[col * kPs + 16 * kt + 4 * g]) = x;
     }
     __syncthreads();
