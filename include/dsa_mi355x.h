@@ -245,8 +245,8 @@ int dsa_sparse_mla_bwd(const void* q, const void* kv, const int32_t* indices, co
  * workgroup, which gathers the union of their keys once; bf16 calls of few tokens (generation)
  * to split a token's keys over several workgroups.
  */
-/* (tokens that share a workgroup under that rule, the same for dsa_attn_mass_ws; 1: none do) */
-int dsa_attn_packed_tokens(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t topk,
+/* Tokens that share a workgroup in such a call, or (mass = 1) in dsa_attn_mass_ws; 1: none do. */
+int dsa_attn_packed_tokens(int mass, int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t topk,
                            int64_t q_offset);
 int64_t dsa_sparse_mla_fwd_workspace_size(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
                                           int64_t topk, int64_t q_offset);
@@ -303,7 +303,8 @@ int dsa_attn_mass(const void* q, const void* kv, const int32_t* indices, const f
 /*
  * The same with a caller workspace of dsa_attn_mass_workspace_size() bytes (16-byte aligned).
  * The size is 0 where it has no use; with fewer bytes, or none, the call runs as dsa_attn_mass.
- * bf16 calls of at most 64 heads use it to let several consecutive tokens share a workgroup.
+ * bf16 calls of at most 64 heads use it to let several consecutive tokens share a workgroup,
+ * where that is faster (dsa_attn_packed_tokens).
  */
 int64_t dsa_attn_mass_workspace_size(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
                                      int64_t topk, int64_t q_offset);

@@ -76,3 +76,31 @@ def test_packed_mass_in_chunks():
     _, mx, sm = ops.sparse_mla_fwd(q, kv, idx, 512 ** -0.5)
     plain = _mass(q, kv, idx, mx, sm, 512 ** -0.5, 0, 0)
     torch.testing.assert_close(_mass(q, kv, idx, mx, sm, 512 ** -0.5, 0, need), plain, rtol=2.0 ** -17, atol=1e-30)
+
+
+@pytest.mark.parametrize("B,S,s_kv,H,D,K,repeats", [
+    (1, 700, 700, 64, 576, 512, False),   # two tokens per group, a tail of one, slots past the last key
+    (2, 513, 600, 16, 512, 512, True),    # five tokens, a tail of three, two batch elements, repeats
+    (1, 1030, 500, 1, 576, 515, True),    # one head of 16 rows, an odd slot count
+    (1, 640, 640, 17, 576, 600, False),   # heads padded to 32 rows
+    (2, 300, 900, 40, 512, 513, False)])  # 48 rows per token: a wave's halves belong to two tokens
+def test_packed_mass_long_lists(B, S, s_kv, H, D, K, repeats):
+    """Sizes at which the causal call packs: against the one-token kernel, and in the backward."""
+    from torchtitan_npu_simulator_amd import torch_npu_ops as ops
+    from torchtitan_npu_simulator_amd._lib import DSA_BF16, load_library
+
+    q, kv, idx = _case(B, S, s_kv, H, D, K, S + H, repeats)
+    scale, off = D ** -0.5, s_kv - S if s_kv > S else 0
+    lib = load_library()
+    assert lib.dsa_attn_packed_tokens(1, DSA_BF16, B, S, s_kv, H, K, off) > 1
+    need = int(lib.dsa_attn_mass_workspace_size(DSA_BF16, B, S, s_kv, H, K, off))
+    out, mx, sm = ops.sparse_mla_fwd(q, kv, idx, scale, q_offset=off)
+    plain = _mass(q, kv, idx, mx, sm, scale, off, 0)
+    got = _mass(q, kv, idx, mx, sm, scale, off, need)
+    torch.testing.assert_close(got, plain, rtol=2.0 ** -17, atol=1e-30)
+    assert torch.equal(got == 0, plain == 0)
+    assert torch.equal(ops.attn_mass(q, kv, idx, mx, sm, scale, q_offset=off), got)
+    dout = torch.randn(out.shape, device=DEV).bfloat16()
+    mass = ops.sparse_mla_bwd(q, kv, idx, out, dout, mx, sm, scale, q_offset=off, return_mass=True)[2]
+    # (its scores come from 16 x 16 x 32 matrix steps: fp32 sums in another order)
+    torch.testing.assert_close(mass, plain, rtol=1e-4, atol=1e-7)

@@ -147,3 +147,30 @@ def test_packed_capped_workspace_results():
     for r in runs[1:]:
         for a, b in zip(r, runs[0]):
             assert rel_err(a, b) <= 1e-2
+
+
+def test_packed_where_lists_overlap():
+    """With the causal test, lists that share few keys run one token per workgroup; without it
+    (sequences of a batch, V4 windows) the number of keys says nothing."""
+    from torchtitan_npu_simulator_amd import _lib
+
+    lib = _lib.load_library()
+
+    def tokens(mass, S, s_kv, H, K, off=None):
+        return lib.dsa_attn_packed_tokens(mass, _lib.DSA_BF16, 1, S, s_kv, H, K, s_kv - S if off is None else off)
+
+    def back(S, s_kv, H, K, off=None):
+        return lib.dsa_sparse_mla_bwd_packed(1, S, s_kv, H, 576, K, s_kv - S if off is None else off, 32 << 30)
+
+    assert tokens(0, 4096, 16384, 64, 1024) == 2 and tokens(0, 4096, 32768, 64, 1024) == 1
+    assert tokens(0, 4096, 131072, 16, 1024) == 8 and tokens(0, 4096, 131072, 64, 1024, off=1 << 40) == 2
+    assert back(4096, 16384, 64, 256) == 1 and back(4096, 32768, 64, 256) == 0 and back(1024, 32768, 64, 256) == 1
+    assert back(4096, 65536, 16, 256) == 1 and back(4096, 131072, 16, 256) == 0
+    assert back(4096, 65536, 64, 256, off=1 << 40) == 1
+    assert tokens(1, 1024, 1024, 16, 256) == 1 and tokens(1, 1024, 1024, 16, 512) == 4
+    assert tokens(1, 4096, 4096, 16, 64) == 8 and tokens(1, 4096, 32768, 64, 1024) == 1
+    # a workspace serves the call with and without the causal test
+    for S, s_kv, H, K in [(4096, 32768, 64, 256), (4096, 4096, 16, 512)]:
+        most = int(lib.dsa_sparse_mla_bwd_workspace_size(1, S, s_kv, H, 576, K))
+        assert lib.dsa_sparse_mla_bwd_packed(1, S, s_kv, H, 576, K, s_kv, most) == 1
+        assert lib.dsa_sparse_mla_bwd_chunk_rows(1, S, s_kv, 576, K, most) >= 1

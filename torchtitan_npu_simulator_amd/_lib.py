@@ -52,7 +52,7 @@ _SIGNATURES = {
         [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _i64, _vp],
         _i32,
     ),
-    "dsa_attn_packed_tokens": ([_i32, _i64, _i64, _i64, _i64, _i64, _i64], _i32),
+    "dsa_attn_packed_tokens": ([_i32, _i32, _i64, _i64, _i64, _i64, _i64, _i64], _i32),
     "dsa_sparse_mla_fwd_workspace_size": ([_i32, _i64, _i64, _i64, _i64, _i64, _i64], _i64),
     "dsa_sparse_mla_fwd_ws": (
         [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _i64, _vp, _i64, _vp],

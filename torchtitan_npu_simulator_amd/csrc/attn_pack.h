@@ -20,7 +20,7 @@
 //   mask[tt][words]   bit j of word j / 32: slot j of idx is selected by the token;
 //   count             used slots;
 //   redo[4]           (cleared by the plan) the rows whose O the forward found not finite, as bits;
-//   pos[tt][K]        (backward) the slot of the token's j-th selection, kPackNoSlot if
+//   pos[tt][K]        (mass, backward) the slot of the token's j-th selection, kPackNoSlot if
 //                     unusable;
 //   sel[word]         (backward, stored word-major over the groups) the union's keys
 //                     32 word .. +31 as bits, with the slot of the first of them; bit 31 of
@@ -54,7 +54,7 @@ struct PackView {
   const uint32_t* mask = nullptr;  // [batch][groups][tt][words]
   const int32_t* count = nullptr;  // [batch][groups]
   uint32_t* redo = nullptr;        // [batch][groups][4]
-  uint16_t* pos = nullptr;         // [batch][S][K], backward only as the next two
+  uint16_t* pos = nullptr;         // [batch][S][K]: mass and backward; the next three: backward
   uint2* sel = nullptr;            // [batch][key words][groups]
   int32_t* distinct = nullptr;     // [batch][groups]
   int32_t* suspect = nullptr;      // [batch][groups]
@@ -62,17 +62,21 @@ struct PackView {
   int tt = 1, hp = kPackRows, cap = 0, words = 0, groups = 0, key_words = 0;
 };
 
-// Tokens per group for a problem (1: the unpacked kernels serve it).
-int pack_tokens(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t topk, int64_t q_offset);
 inline int pack_hp(int64_t n_heads) { return (int)((n_heads + 15) / 16 * 16); }
 inline int64_t pack_groups(int64_t s_q, int tt) { return (s_q + tt - 1) / tt; }
 inline int64_t pack_cap(int64_t topk, int tt) { return (topk * tt + 31) / 32 * 32; }
 
-// Workspace of the plan (256-byte aligned parts); backward adds pos, sel, distinct and suspect.
-int64_t pack_plan_bytes(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int tt, bool backward);
+// Parts of the plan: the forward takes idx, mask, count and redo, the mass pos too, the backward
+// all of it.
+enum class PackParts { kForward, kMass, kBackward };
+// Tokens per group for a problem (1: the unpacked kernels serve it).
+int pack_tokens(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t topk, int64_t q_offset,
+                PackParts parts);
+// Workspace of the plan (256-byte aligned parts).
+int64_t pack_plan_bytes(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int tt, PackParts parts);
 // Enqueues the plan into ws and fills *view.
 int pack_plan_build(const int32_t* indices, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t topk,
-                    int64_t q_offset, int tt, bool backward, void* ws, hipStream_t st, PackView* view);
+                    int64_t q_offset, int tt, PackParts parts, void* ws, hipStream_t st, PackView* view);
 // For the n groups from g0 of every batch element:
 // mass[token][j] = view.mass[token's group][token][pos[token][j]] (0 at unusable slots)
 int pack_mass_gather(const PackView& view, float* mass, int64_t batch, int64_t s_q, int64_t topk, int64_t g0, int64_t n,

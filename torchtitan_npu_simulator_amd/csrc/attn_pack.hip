@@ -343,32 +343,65 @@ int64_t al256(int64_t x) { return (x + 255) / 256 * 256; }
 }  // namespace
 
 // Packing never adds gathered blocks (a union is at most the sum of its lists), so it is
-// taken wherever a token leaves half of the workgroup's rows idle or more and the tokens
+// considered wherever a token leaves half of the workgroup's rows idle or more and the tokens
 // would run in two rounds of the 256 CUs or more: ceil(tokens / 256) tokens per group keep
 // one workgroup per CU.  A call with no causal test (q_offset >= s_kv: the sequences of a
 // packed batch on global key rows) packs from 1024 tokens: the union changes the order in
 // which a row's keys are summed, and a shorter batch keeps the results of per-sequence calls
 // bit for bit.
-int pack_tokens(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t topk, int64_t q_offset) {
+//
+// What a group saves over its tokens is the overlap of their lists, about s_kv / (tt topk) for
+// lists drawn at random (top-k lists of neighbours overlap more); the limits below keep calls
+// of a causal test whose random lists were not faster packed on the one-token kernels.  (Without
+// the test a row's keys lie in its own sequence or window, which s_kv says nothing about.)
+// Time of one token over packed, top-k lists at random, 64 | 32 | 16 heads (2 | 4 | 8 tokens):
+//   forward, 4096 tokens, top-1024: s_kv 16384 1.02 | 1.12 | 1.29, 32768 0.98 | 1.07 | 1.15,
+//     131072 0.93 | 1.02 | 1.07.
+//   backward, where every key looks at every group: top-2048, s_kv 16384 1.06 | 1.22 | 1.55,
+//     65536 0.95 | 1.02 | 1.10, 131072 0.87 | 0.96 | 1.04; top-256, 16384 1.03 | 1.14 | 1.28,
+//     65536 0.86 | 0.96 | 1.10; 1024 tokens (512 | 256 | 256 groups), top-1024, 32768 1.02 |
+//     1.08 | 1.10, 65536 0.95 | 1.05 | 1.07, 131072 0.86 | 0.95 | 0.96.
+//   mass, whose one-token form runs two workgroups per CU: 1024 tokens and keys, top-64 0.82 |
+//     0.84 | 0.84, top-512 1.13 | 1.16 | 1.23; 4096 tokens, s_kv 4096, top-256 0.93 | 1.11 | 1.34,
+//     top-2048 1.45 | 2.2 | 3.0; s_kv 32768, top-1024 0.92 | 0.97 | 1.01.
+static bool overlap_pays(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int64_t tt, PackParts parts) {
+  const int64_t tokens = batch * s_q, lists = tt * topk;
+  switch (parts) {
+    case PackParts::kForward:
+      return tt > 2 || s_kv <= std::max<int64_t>(16384, 16 * topk);
+    case PackParts::kBackward:
+      return s_kv <= tt * std::max<int64_t>(8192, 8 * topk) || s_kv * batch * pack_groups(s_q, (int)tt) <= (1 << 24);
+    default:
+      if (topk >= 512 && s_kv <= (tokens >= 2048 ? 2 : 1) * lists) return true;
+      if (tokens >= 8192 && s_kv <= 8 * lists) return true;
+      return tokens >= 2048 && tt > 2 && (s_kv <= 4 * lists || topk <= (tt >= 6 ? 256 : 64));
+  }
+}
+
+int pack_tokens(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t topk, int64_t q_offset,
+                PackParts parts) {
   if (n_heads <= 0 || n_heads > kPackRows / 2 || batch <= 0 || s_q <= 0 || topk <= 0) return 1;
-  if (batch * s_q < (q_offset >= s_kv ? 1024 : 512)) return 1;
+  const bool causal = q_offset < s_kv;
+  if (batch * s_q < (causal ? 512 : 1024)) return 1;
   if (s_kv > kPackMaxKeys) return 1;
   int64_t tt = kPackRows / pack_hp(n_heads);
   tt = std::min<int64_t>(tt, (batch * s_q + 255) / 256);
   tt = std::min<int64_t>(tt, s_q);
   tt = std::min<int64_t>(tt, 65504 / topk);  // slots are 16-bit
   while (tt > 1 && tt * (pack_cap(topk, (int)tt) / 32) > kPackMaxMaskWords) --tt;
-  return (int)std::max<int64_t>(tt, 1);
+  if (tt <= 1 || (causal && !overlap_pays(batch, s_q, s_kv, topk, tt, parts))) return 1;
+  return (int)tt;
 }
 
-int64_t pack_plan_bytes(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int tt, bool backward) {
+int64_t pack_plan_bytes(int64_t batch, int64_t s_q, int64_t s_kv, int64_t topk, int tt, PackParts parts) {
   const int64_t g = pack_groups(s_q, tt) * batch, cap = pack_cap(topk, tt);
   return al256(g * cap * 4) + al256(g * tt * (cap / 32) * 4) + al256(g * 4) + al256(g * 16) +
-         (backward ? al256(batch * s_q * topk * 2) + al256(g * ((s_kv + 31) / 32) * 8) + 2 * al256(g * 4) : 0);
+         (parts != PackParts::kForward ? al256(batch * s_q * topk * 2) : 0) +
+         (parts == PackParts::kBackward ? al256(g * ((s_kv + 31) / 32) * 8) + 2 * al256(g * 4) : 0);
 }
 
 int pack_plan_build(const int32_t* indices, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t topk,
-                    int64_t q_offset, int tt, bool backward, void* ws, hipStream_t st, PackView* view) {
+                    int64_t q_offset, int tt, PackParts parts, void* ws, hipStream_t st, PackView* view) {
   PackView pk;
   pk.tt = tt;
   pk.hp = pack_hp(n_heads);
@@ -387,8 +420,8 @@ int pack_plan_build(const int32_t* indices, int64_t batch, int64_t s_q, int64_t 
   uint32_t* mask = (uint32_t*)take(g * tt * pk.words * 4);
   int32_t* count = (int32_t*)take(g * 4);
   pk.redo = (uint32_t*)take(g * 16);
-  if (backward) {
-    pk.pos = (uint16_t*)take(batch * s_q * topk * 2);
+  if (parts != PackParts::kForward) pk.pos = (uint16_t*)take(batch * s_q * topk * 2);
+  if (parts == PackParts::kBackward) {
     pk.sel = (uint2*)take(g * pk.key_words * 8);
     pk.distinct = (int32_t*)take(g * 4);
     pk.suspect = (int32_t*)take(g * 4);

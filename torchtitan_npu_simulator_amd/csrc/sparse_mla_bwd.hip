@@ -1182,11 +1182,11 @@ struct PackBwdPlan {
 PackBwdPlan plan_pack_bwd(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t topk, int64_t q_offset,
                           int64_t budget, int64_t width) {
   PackBwdPlan p{};
-  p.tt = pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset);
+  p.tt = pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset, PackParts::kBackward);
   if (p.tt <= 1) return p;
   const int64_t cap = pack_cap(topk, p.tt), groups = pack_groups(s_q, p.tt);
   auto al = [](int64_t x) { return (x + 255) / 256 * 256; };
-  p.plan_bytes = pack_plan_bytes(batch, s_q, s_kv, topk, p.tt, true);
+  p.plan_bytes = pack_plan_bytes(batch, s_q, s_kv, topk, p.tt, PackParts::kBackward);
   const int64_t per_row = batch * (cap * (kGW * 2 + width * 2 + p.tt * 4) + kHeadsMax * 4);
   p.rows = std::min<int64_t>(groups, (budget - p.plan_bytes - 4 * 256) / per_row);
   if (p.rows < 1 || (p.rows < groups && batch * p.rows * p.tt < kPackMinTokens)) return p;
@@ -1205,11 +1205,11 @@ extern "C" int64_t dsa_sparse_mla_bwd_workspace_size(int64_t batch, int64_t s_q,
                                                      int64_t d_qk, int64_t topk) {
   if (batch <= 0 || s_q <= 0 || s_kv <= 0 || topk <= 0) return 0;
   const int64_t width = d_qk == dsa::kDv ? dsa::kDv : dsa::kDqk;  // C row width of the bf16 path
-  const dsa::PackBwdPlan pp = dsa::plan_pack_bwd(batch, s_q, s_kv, n_heads, topk, 0, dsa::kDefaultBudget, width);
-  const bool either = pp.total && !dsa::plan_pack_bwd(batch, s_q, s_kv, n_heads, topk, s_kv, dsa::kDefaultBudget,
-                                                      width).total;  // (packed or not by the call's q_offset)
-  if (pp.total && !either) return pp.total;
-  return std::max(pp.total, dsa::plan_bwd(batch, s_q, s_kv, topk, dsa::kDefaultBudget, width).total);
+  // packed or not by the call's q_offset: with the causal test, and without
+  const int64_t causal = dsa::plan_pack_bwd(batch, s_q, s_kv, n_heads, topk, 0, dsa::kDefaultBudget, width).total;
+  const int64_t open = dsa::plan_pack_bwd(batch, s_q, s_kv, n_heads, topk, s_kv, dsa::kDefaultBudget, width).total;
+  if (causal && open) return std::max(causal, open);
+  return std::max(std::max(causal, open), dsa::plan_bwd(batch, s_q, s_kv, topk, dsa::kDefaultBudget, width).total);
 }
 
 namespace dsa {
@@ -1268,7 +1268,7 @@ static int sparse_mla_bwd_packed(const void* q, const void* kv, const int32_t* i
                                  int64_t s_q, int64_t s_kv, int64_t n_heads, int64_t d_qk, int64_t topk, float scale,
                                  int64_t q_offset, const float* sinks, float* dsink, hipStream_t st) {
   PackView pk;
-  if (int rc = pack_plan_build(indices, batch, s_q, s_kv, n_heads, topk, q_offset, plan.tt, true, ws, st, &pk))
+  if (int rc = pack_plan_build(indices, batch, s_q, s_kv, n_heads, topk, q_offset, plan.tt, PackParts::kBackward, ws, st, &pk))
     return rc;
   char* p = ws + plan.plan_bytes;
   uint16_t* gbuf = (uint16_t*)p;

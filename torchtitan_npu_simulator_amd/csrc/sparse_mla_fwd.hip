@@ -536,8 +536,7 @@ int fwd_splits(int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads, int64_
 // union slot, from where pack_mass_gather takes the tokens' own slots.  With few heads the
 // one-token form computes 128 rows per token all the same.  Top-2048, kernel alone: 2500
 // tokens, 64 heads 547 us -> 337 with plan and gather; 1500 tokens, 16 heads 200 -> 101; 600
-// tokens, 32 heads, top-512 49 -> 47 (the forward's rule, pack_tokens, is kept as it is: its
-// plan costs the same here).
+// tokens, 32 heads, top-512 49 -> 47 (pack_tokens says from where it pays).
 template <int kD, bool kPack>  // kD, row width of Q and KV: 576 (latent + rope) or 512 (no rope)
 __global__ void __launch_bounds__(kFwdThreads, 2)
 attn_mass_bf16_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv,
@@ -966,7 +965,9 @@ attn_mass_f32_kernel(const float* __restrict__ q, const float* __restrict__ kv, 
 
 namespace dsa {
 // Workspace of the packed mass: the plan and the head sums of a chunk of groups by union slot,
-// [batch][groups of the chunk][tt][cap] fp32, at most kMassBudget or one group per element.
+// [batch][groups of the chunk][tt][cap] fp32, at most kMassBudget or one group per element.  Its
+// size keeps to the forward's rule; a call that the mass's own rule (pack_tokens) leaves on the
+// one-token kernel has no use for it.
 constexpr int64_t kMassBudget = 1LL << 29;
 static int64_t mass_chunk_groups(int64_t batch, int64_t s_q, int64_t topk, int tt) {
   const int64_t per = batch * tt * pack_cap(topk, tt) * 4;
@@ -975,9 +976,9 @@ static int64_t mass_chunk_groups(int64_t batch, int64_t s_q, int64_t topk, int t
 static int64_t mass_workspace_bytes(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
                                     int64_t topk, int64_t q_offset) {
   if (dtype != DSA_BF16 || topk <= 0) return 0;
-  const int tt = pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset);
+  const int tt = pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset, PackParts::kForward);
   if (tt <= 1) return 0;
-  return pack_plan_bytes(batch, s_q, s_kv, topk, tt, true) +
+  return pack_plan_bytes(batch, s_q, s_kv, topk, tt, PackParts::kMass) +
          mass_chunk_groups(batch, s_q, topk, tt) * batch * tt * pack_cap(topk, tt) * 4;
 }
 }  // namespace dsa
@@ -1006,12 +1007,12 @@ extern "C" int dsa_attn_mass_ws(const void* q, const void* kv, const int32_t* in
     const int64_t max_rows = d_qk == kDqk ? GatherGeomT<kDqk>::kMaxRows : GatherGeomT<kDv>::kMaxRows;
     if (s_kv > max_rows) return set_error(DSA_ERR_UNSUPPORTED, "dsa_attn_mass: S_kv > %lld", (long long)max_rows);
     const int64_t need = workspace ? mass_workspace_bytes(dtype, batch, s_q, s_kv, n_heads, topk, q_offset) : 0;
-    if (need > 0 && workspace_bytes >= need && (uintptr_t)workspace % 16 == 0) {
-      const int tt = pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset);
+    const int tt = pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset, PackParts::kMass);
+    if (tt > 1 && need > 0 && workspace_bytes >= need && (uintptr_t)workspace % 16 == 0) {
       PackView pk;
-      if (int rc = pack_plan_build(indices, batch, s_q, s_kv, n_heads, topk, q_offset, tt, true, workspace, st, &pk))
+      if (int rc = pack_plan_build(indices, batch, s_q, s_kv, n_heads, topk, q_offset, tt, PackParts::kMass, workspace, st, &pk))
         return rc;
-      pk.mass = (float*)((char*)workspace + pack_plan_bytes(batch, s_q, s_kv, topk, tt, true));
+      pk.mass = (float*)((char*)workspace + pack_plan_bytes(batch, s_q, s_kv, topk, tt, PackParts::kMass));
       const int64_t chunk = mass_chunk_groups(batch, s_q, topk, tt);
       for (int64_t g0 = 0; g0 < pk.groups; g0 += chunk) {
         const int64_t n = std::min<int64_t>(chunk, pk.groups - g0);
@@ -1063,8 +1064,8 @@ namespace dsa {
 static int64_t fwd_workspace_bytes(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
                                    int64_t topk, int64_t q_offset) {
   if (dtype != DSA_BF16 || topk <= 0) return 0;
-  const int tt = pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset);
-  if (tt > 1) return pack_plan_bytes(batch, s_q, s_kv, topk, tt, false);
+  const int tt = pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset, PackParts::kForward);
+  if (tt > 1) return pack_plan_bytes(batch, s_q, s_kv, topk, tt, PackParts::kForward);
   const int n_split = fwd_splits(batch, s_q, s_kv, n_heads, topk);
   return n_split > 1 ? batch * s_q * n_heads * n_split * kPartFloats * 4 : 0;
 }
@@ -1094,11 +1095,12 @@ static int sparse_mla_fwd_impl(const void* q, const void* kv, const int32_t* ind
     PackView pk;
     const int64_t need = workspace ? fwd_workspace_bytes(dtype, batch, s_q, s_kv, n_heads, topk, q_offset) : 0;
     const bool use_ws = need > 0 && workspace_bytes >= need && (uintptr_t)workspace % 16 == 0;
-    const bool pack = use_ws && pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset) > 1;
+    const int tt = pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset, PackParts::kForward);
+    const bool pack = use_ws && tt > 1;
     const int n_split = use_ws && !pack ? fwd_splits(batch, s_q, s_kv, n_heads, topk) : 1;
     if (pack) {
-      if (int rc = pack_plan_build(indices, batch, s_q, s_kv, n_heads, topk, q_offset,
-                                   pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset), false, workspace, st, &pk))
+      if (int rc = pack_plan_build(indices, batch, s_q, s_kv, n_heads, topk, q_offset, tt, PackParts::kForward, workspace,
+                                   st, &pk))
         return rc;
     }
     dim3 grid((unsigned)(pack ? pk.groups : s_q), pack ? 1 : n_split > 1 ? n_split : ceil_div(n_heads, kFwdHeads),
@@ -1156,9 +1158,11 @@ extern "C" int dsa_sparse_mla_fwd(const void* q, const void* kv, const int32_t* 
                                   n_heads, d_qk, d_v, topk, scale, q_offset, nullptr, 0, stream);
 }
 
-extern "C" int dsa_attn_packed_tokens(int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
+extern "C" int dsa_attn_packed_tokens(int mass, int dtype, int64_t batch, int64_t s_q, int64_t s_kv, int64_t n_heads,
                                       int64_t topk, int64_t q_offset) {
-  return dtype == DSA_BF16 ? dsa::pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset) : 1;
+  using namespace dsa;
+  if (dtype != DSA_BF16) return 1;
+  return pack_tokens(batch, s_q, s_kv, n_heads, topk, q_offset, mass ? PackParts::kMass : PackParts::kForward);
 }
 
 extern "C" int64_t dsa_sparse_mla_fwd_workspace_size(int dtype, int64_t batch, int64_t s_q, int64_t s_kv,

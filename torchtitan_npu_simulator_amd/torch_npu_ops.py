@@ -754,7 +754,8 @@ def attn_mass(q, kv, indices, smax, ssum, scale, *, q_offset=0):
     indices = indices.reshape(B, S, K).to(torch.int32).contiguous()
     mass = torch.empty(B, S, K, dtype=torch.float32, device=q.device)
     dt = _lib.dtype_code(q.dtype)
-    ws_bytes = int(lib.dsa_attn_mass_workspace_size(dt, B, S, s_kv, H, K, int(q_offset)))
+    ws_bytes = int(lib.dsa_attn_mass_workspace_size(dt, B, S, s_kv, H, K, int(q_offset))) \
+        if lib.dsa_attn_packed_tokens(1, dt, B, S, s_kv, H, K, int(q_offset)) > 1 else 0
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
     check(
         lib.dsa_attn_mass_ws(ptr(q), ptr(kv), ptr(indices), ptr(smax.contiguous()), ptr(ssum.contiguous()), ptr(mass),
@@ -784,7 +785,7 @@ def sparse_mla_fwd_varlen(q, kv, indices, scale, cu_seqlens_q, cu_seqlens_kv, *,
     T, H, D = q.shape
     kv = kv.reshape(kv.shape[0], kv.shape[-1]).contiguous()
     packed = q.dtype == torch.bfloat16 and T > 0 and lib.dsa_attn_packed_tokens(
-        _lib.DSA_BF16, 1, T, kv.shape[0], H, indices.shape[-1], _NO_MASK_OFFSET) > 1
+        0, _lib.DSA_BF16, 1, T, kv.shape[0], H, indices.shape[-1], _NO_MASK_OFFSET) > 1
     g = _varlen_global(indices, cu_seqlens_q, cu_seqlens_kv, T, kv.shape[0], q.device, packed)
     if g is not None:  # device bounds, packed tokens: one launch over the batch
         out, smax, ssum = sparse_mla_fwd(q.unsqueeze(0), kv.unsqueeze(0), g.unsqueeze(0), scale, d_v=d_v,
@@ -856,7 +857,7 @@ def attn_mass_varlen(q, kv, indices, smax, ssum, scale, cu_seqlens_q, cu_seqlens
     T, H, D = q.shape
     kv = kv.reshape(kv.shape[0], kv.shape[-1]).contiguous()
     packed = q.dtype == torch.bfloat16 and T > 0 and lib.dsa_attn_packed_tokens(
-        _lib.DSA_BF16, 1, T, kv.shape[0], H, indices.shape[-1], _NO_MASK_OFFSET) > 1
+        1, _lib.DSA_BF16, 1, T, kv.shape[0], H, indices.shape[-1], _NO_MASK_OFFSET) > 1
     g = _varlen_global(indices, cu_seqlens_q, cu_seqlens_kv, T, kv.shape[0], q.device, packed)
     if g is not None:  # device bounds, packed tokens: one launch over the batch
         return attn_mass(q.unsqueeze(0), kv.unsqueeze(0), g.unsqueeze(0), smax.unsqueeze(0), ssum.unsqueeze(0), scale,
