@@ -24,3 +24,23 @@ def test_v4_indices_kernel(B, S, win_left, win_right, ratio, n_cmp, K):
     ref = ops.v4_attention_indices(B, S, "cpu", cmp_indices=cmp, **kw)
     got = ops.v4_attention_indices(B, S, torch.device("cuda"), cmp_indices=None if cmp is None else cmp.cuda(), **kw)
     assert got.dtype == torch.int32 and torch.equal(got.cpu(), ref)
+
+
+def test_v4_indices_left_to_torch(monkeypatch):
+    """More batch elements than a grid takes, and indices on another GPU (here: another one is made
+    to look current), do not reach the kernel."""
+    from torchtitan_npu_simulator_amd import torch_npu_ops as ops
+
+    cmp = torch.randint(0, 8, (65536, 1, 2), dtype=torch.int32)
+    kw = dict(win_left=0, cmp_ratio=4, n_cmp=4)
+    ref = ops.v4_attention_indices(65536, 1, "cpu", cmp_indices=cmp, **kw)
+    assert torch.equal(ops.v4_attention_indices(65536, 1, "cuda", cmp_indices=cmp.cuda(), **kw).cpu(), ref)
+
+    def no_kernel():
+        raise AssertionError("the kernel was asked for")
+
+    small = cmp[:3].cuda()
+    monkeypatch.setattr(ops, "load_library", no_kernel)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    got = ops.v4_attention_indices(3, 1, "cuda", cmp_indices=small, **kw)
+    assert torch.equal(got.cpu(), ref[:3])

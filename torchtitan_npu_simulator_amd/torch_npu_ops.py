@@ -1096,8 +1096,12 @@ def v4_attention_indices(B, S, device, *, win_left=127, win_right=0, cmp_ratio=1
     """
     W = win_left + win_right + 1
     sel = cmp_ratio > 1 and n_cmp > 0
-    if torch.device(device).type == "cuda" and W > 0 and B > 0 and S > 0 and (not sel or cmp_indices is None or (
-            cmp_indices.is_cuda and cmp_indices.dtype == torch.int32 and cmp_indices.shape[:-1] == (B, S))):
+    dev = torch.device(device)
+    # (one kernel; indices on another GPU, in another type or shape, and more batch elements than a
+    # grid takes go through torch, which takes or refuses them)
+    if dev.type == "cuda" and W > 0 and 0 < B <= 65535 and S > 0 and (not sel or cmp_indices is None or (
+            cmp_indices.dtype == torch.int32 and cmp_indices.shape[:-1] == (B, S) and
+            cmp_indices.get_device() == (torch.cuda.current_device() if dev.index is None else dev.index))):
         n_sel = 0 if not sel else n_cmp if cmp_indices is None else cmp_indices.shape[-1]
         ci = cmp_indices.contiguous() if sel and cmp_indices is not None and n_sel else None
         out = torch.empty(B, S, W + n_sel, dtype=torch.int32, device=device)
