@@ -363,3 +363,23 @@ def test_smallest_workspace():
     part = ops.sparse_mla_bwd(q, kv, idx, out, dout, smax, ssum, scale, workspace_bytes=hi)
     assert torch.equal(full[0], part[0])
     assert rel_err(part[1], full[1]) <= 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,K,part", [(300, 1000, 3), (600, 1800, 4), (40, 70, 2)])  # 128, 256, 32 pairs per segment
+def test_reduction_segment_sizes(S, K, part):
+    """One chunk, whose segments hold as many pairs as its size asks for, against chunks of a
+    capped workspace, whose segments are shorter."""
+    from torchtitan_npu_simulator_amd import _lib
+    from torchtitan_npu_simulator_amd import torch_npu_ops as ops
+
+    H, s_kv = 72, 2000  # (more heads than tokens share workgroups at)
+    q, kv, dout, scale = attn_inputs(S, H, q_offset=s_kv - S, seed=S)
+    idx = rand_indices(S, K, q_offset=s_kv - S, seed=S, holes=0.05).cuda()
+    q, kv, dout = q.cuda(), kv.cuda(), dout.cuda()
+    out, smax, ssum = ops.sparse_mla_fwd(q, kv, idx, scale, q_offset=s_kv - S)
+    most = int(_lib.load_library().dsa_sparse_mla_bwd_workspace_size(1, S, s_kv, H, 576, K))
+    runs = [ops.sparse_mla_bwd(q, kv, idx, out, dout, smax, ssum, scale, q_offset=s_kv - S, workspace_bytes=b)
+            for b in (most, most // part)]
+    assert torch.equal(runs[0][0], runs[1][0])
+    assert rel_err(runs[1][1], runs[0][1]) <= 1e-5

@@ -421,15 +421,17 @@ __global__ void __launch_bounds__(1024) csr_scan_kernel(const int* __restrict__ 
 // chunks): lane l owns chunk l.  128-wide rows
 // (16 chunks): lanes 16s .. 16s+15 own the row of pair 4g + s of each group of 4 (four
 // streams), combined with two lane exchanges at the flush.
-// pairs per wave: 256, fewer where those would not fill the chip (a segment costs two partial
-// rows).  150 rows of top-256: the reduction of 576-wide rows 57 us on 150 segments of 256
-// pairs, 12 us on 1200 of 32; 1500 rows of top-1024, 128-wide: 67 us of 256, 56 us of 64.
+// pairs per wave: 256, fewer where those leave the chip idle (a segment costs two partial rows).
+// Reduction and fix-up of 576-wide and of 128-wide rows, us, with 256 pairs and with the rule's:
+// 38 K pairs 59 and 46, 18 and 13 (32 pairs); 131 K 66 and 45, 34 and 18 (32); 410 K 88 and 52,
+// 90 and 35 (128; with 32 99 and 30); 700 K 97 and 52, 103 and 41 (128; 32: 120 and 42); 1.5 M
+// 214 and 79 (256; 64: 241 and 70).
 // `coarse` keeps 256: a chunk of one row in a workspace that has no room for more partial rows
 // (with room, one row of top-2048 and 128 heads takes 355 us, coarse 585).
 inline int csr_seg_shift(int64_t rows, int64_t K, bool coarse) {
   if (coarse) return 8;
   const int64_t pairs = rows * K;
-  return pairs >= (1 << 22) ? 8 : pairs >= (1 << 21) ? 7 : pairs >= (1 << 20) ? 6 : 5;
+  return pairs >= (1 << 20) ? 8 : pairs >= (1 << 18) ? 7 : 5;
 }
 inline int64_t csr_segments(int64_t rows, int64_t K, bool coarse) {
   const int sh = csr_seg_shift(rows, K, coarse);
@@ -438,7 +440,7 @@ inline int64_t csr_segments(int64_t rows, int64_t K, bool coarse) {
 // the most segments of any chunk of at most `rows` rows
 inline int64_t csr_segments_max(int64_t rows, int64_t K, bool coarse) {
   const int64_t n = csr_segments(rows, K, coarse), few = coarse ? n : (rows * K + 31) / 32;
-  return n > 32768 ? n : few < 32768 ? few : 32768;
+  return n > 8192 ? n : few < 8192 ? few : 8192;
 }
 
 __device__ __forceinline__ void add_bf16x8(float (&acc)[8], const u32x4& v) {
