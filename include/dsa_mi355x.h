@@ -602,8 +602,9 @@ int dsa_lightning_indexer_tnd(const void* q, const float* q_scale, const void* k
  * (0 <= v < len_k_i, v <= s - cu_seqlens_q[i] + max(0, len_k_i - len_q_i)), else -1.  The
  * fixed-length attention, mass and indexer KL entry points then take the whole batch as one
  * [1, t_q] problem with q_offset >= t_k (no causal test): dsa_sparse_mla_fwd(_varlen)
- * results are bit-identical per row (without a forward workspace); dKV and dk_I sum the same
- * contributions in another fp32 grouping.  dsa_tnd_global_indices_varlen: the same from host
+ * results are bit-identical per row without a workspace, and otherwise to rounding where tokens
+ * share a workgroup or a token's keys are split; dKV and dk_I sum the same contributions in
+ * another fp32 grouping.  dsa_tnd_global_indices_varlen: the same from host
  * bounds (host int32 arrays), passed as kernel arguments. */
 int dsa_tnd_global_indices_varlen(const int32_t* indices, int32_t* out, const int32_t* cu_seqlens_q,
                                   const int32_t* cu_seqlens_k, int64_t n_seq, int64_t topk, void* stream);

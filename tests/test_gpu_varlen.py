@@ -2,9 +2,9 @@
 
 A packed batch must give, for every sequence, exactly what the fixed-length entry points
 give on that sequence alone (bit-exact: the same kernels run on the same slices with the
-sequence's own causal offset; the key-gradient sums dKV / dk_idx only to 1e-6, since a
-key whose contributions span several reduction segments adds them with fp32 atomics in
-no fixed order), and the per-sequence oracle at the contract tolerance
+sequence's own causal offset, at sizes where no tokens share a workgroup; the key-gradient
+sums dKV / dk_idx only to 1e-6, since a key whose contributions span several reduction
+segments adds them by segment), and the per-sequence oracle at the contract tolerance
 (bf16 2e-2; top-k bit-exact on identical scores; compressor fp32 1e-5).  Batches mix an
 empty sequence, a single-token one and lengths that are not multiples of any tile.
 """

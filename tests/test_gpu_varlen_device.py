@@ -10,8 +10,9 @@ check by making ``_lib.host_ints`` (the only read-back of the host schedule) rai
 The host schedule (``tests/test_gpu_varlen.py``, itself held to the per-sequence
 fixed-length entry points and the oracle) is the reference here: indices, values, out,
 softmax statistics, dQ, the mass, dq_I, dw and the row losses bit for bit (the same kernels
-compute every row from the same keys in the same order); dKV and dk_I to 1e-6 relative (the
-key-major reductions group the same fp32 contributions by other segments).  Batches mix an
+compute every row from the same keys in the same order: at the sizes here no tokens share a
+workgroup, which ``tests/test_gpu_varlen_packed.py`` covers); dKV and dk_I to 1e-6 relative
+(the key-major reductions group the same fp32 contributions by other segments).  Batches mix an
 empty sequence, a one-token sequence and lengths that are not multiples of any tile; the
 indexer cases include compressed keys with device residuals and rows past 16384 keys (the
 top-k candidate lists).

@@ -246,8 +246,10 @@ extern "C" int dsa_indexer_kl_grad_varlen(const void* q_idx, const void* k_idx, 
 // 0 <= v < (its causal count under the per-sequence rule of the host schedule above:
 // min(len_k, s - cu_q[i] + max(0, len_k - len_q) + 1)), as cu_k[i] + v, and -1 otherwise.
 // Run with the causal test off (q_offset past every key), the fixed-length kernels then
-// compute each row from exactly the rows the per-sequence launch would gather, in the same
-// order; only the key-major reductions (dKV, dk_I) group their fp32 sums differently.
+// compute each row from exactly the rows the per-sequence launch would gather, and in the same
+// order where neither the batch nor the sequences pack tokens or split a token's keys (more
+// than 64 heads, or fewer than 1024 rows in the batch and 512 in each sequence; more than 128
+// rows in each); the key-major reductions (dKV, dk_I) group their fp32 sums differently.
 namespace dsa {
 namespace {
 __global__ void __launch_bounds__(256)

@@ -779,7 +779,9 @@ def sparse_mla_fwd_varlen(q, kv, indices, scale, cu_seqlens_q, cu_seqlens_kv, *,
     indices [T,K] sequence-local; returns (out [T,H,d_v], softmax_max [T,H], softmax_sum [T,H]).
     With GPU-tensor bounds the batch runs as one launch on global key rows
     (tnd_global_indices), with no host read; with host bounds, one launch per sequence, or,
-    with few enough heads for several tokens to share a workgroup, the same one launch."""
+    where several tokens of the batch would share a workgroup (at most 64 heads, 1024 rows or
+    more), the same one launch: rows then agree with per-sequence calls within the tolerance,
+    not bit for bit."""
     lib = load_library()
     require_gpu_tensor(q, "q")
     T, H, D = q.shape
@@ -1720,7 +1722,8 @@ def npu_sparse_lightning_indexer_grad_kl_loss(
     The main-attention target mass at the selected keys is the one the op-level attention
     backward left for exactly these query / key, indices and statistics (take_attn_mass),
     or else recomputed from (query || query_rope, key || key_rope, softmax_max,
-    softmax_sum) - bitwise the same mass either way; ``loss`` is the token SUM
+    softmax_sum): bitwise the same mass unless tokens share a workgroup in one of the two
+    (at most 64 heads and at least 512 tokens), then to fp32 rounding; ``loss`` is the token SUM
     (the caller divides by B*S, reference dsa.py:73).  ``cmp_ratio`` > 1: key / key_index
     are compressed rows (binding.cpp:17) and sparse_indices come from the indexer's
     compressed rule t < (s+1)//r, so the -1 slots carry the validity and no causal test is
